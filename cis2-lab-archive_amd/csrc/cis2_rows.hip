@@ -112,32 +112,30 @@ __device__ __forceinline__ float inv_rms_of(float sumsq, uint32_t K, float eps) 
   return rsqrt_cr(arg);
 }
 
-template <bool DUAL, bool NORM, uint32_t CB>
+template <bool DUAL, bool NORM>
 __global__ __launch_bounds__(256) void k_bgemm(BgemmArgs a) {
   extern __shared__ v4 sm[];
   __shared__ float s_inv[kT];
   uint32_t si = 0;
   if (a.nseg > 1 && blockIdx.x >= a.blk0[1]) si = (a.nseg > 2 && blockIdx.x >= a.blk0[2]) ? 2 : 1;
   const BgemmSeg g = si == 0 ? a.s[0] : (si == 1 ? a.s[1] : a.s[2]);
-  const uint32_t R = g.R, TB = a.TB, KC = a.KC, K = g.K, NB = TB * CB;  // NB batch rows staged
-  const uint32_t blk = blockIdx.x - a.blk0[si], b0 = blockIdx.y * NB, t = threadIdx.x;
-  const uint32_t r = t % R, bb = t / R;  // the thread's rows: b0 + bb + c * TB, c < CB
+  const uint32_t R = g.R, TB = a.TB, KC = a.KC, K = g.K;
+  const uint32_t blk = blockIdx.x - a.blk0[si], b0 = blockIdx.y * TB, t = threadIdx.x;
+  const uint32_t r = t % R, bb = t / R;  // the thread's row: b0 + bb
   const uint32_t wv = __builtin_amdgcn_readfirstlane(t >> 6), lane = t & 63;
   const bool live = t < R * TB;
   const uint32_t qmax = KC / 4, xs4 = qmax + 1;  // padded X rows: no bank aliasing
   v4* Ws = sm;                                   // [q4][R] (DUAL: then W2's at Ws + qmax * R)
   v4* Xs = sm + (size_t)(DUAL ? 2 : 1) * qmax * R;
-  v4* NWs = Xs + (size_t)NB * xs4;               // NORM: the chunk's norm weights
+  v4* NWs = Xs + (size_t)TB * xs4;               // NORM: the chunk's norm weights
   const v4* Wg = reinterpret_cast<const v4*>(g.W + (size_t)blk * R * K);
   const v4* Wg2 = DUAL ? reinterpret_cast<const v4*>(a.W2 + (size_t)blk * R * K) : nullptr;
-  float acc[CB], acc2[CB];
-#pragma unroll
-  for (uint32_t c = 0; c < CB; ++c) acc[c] = acc2[c] = 0.0f;
+  float acc = 0.0f, acc2 = 0.0f;
   // the chunk's X rows (and norm weights), every load in flight at once,
   // straight into LDS; each wave instruction fills 64 consecutive 16-byte
   // slots
   auto stage_x = [&](uint32_t g0, uint32_t q4, bool with_nw) {
-    const uint32_t pieces = (q4 + 63) / 64, nx = NB * pieces;
+    const uint32_t pieces = (q4 + 63) / 64, nx = TB * pieces;
     // workgroups start at different rows: the grid's requests for the
     // shared X rows spread over the cache channels
     const uint32_t rot = (blockIdx.x * 5) % nx;
@@ -164,10 +162,10 @@ __global__ __launch_bounds__(256) void k_bgemm(BgemmArgs a) {
       stage_x(k0 / 4, q4, false);
       wait_vm0();
       __syncthreads();
-      if (t < NB) ssq = sumsq_groups(Xs + t * xs4, q4, ssq, a.tree);
+      if (t < TB) ssq = sumsq_groups(Xs + t * xs4, q4, ssq, a.tree);
       __syncthreads();
     }
-    if (t < NB) s_inv[t] = inv_rms_of(ssq, K, a.eps);
+    if (t < TB) s_inv[t] = inv_rms_of(ssq, K, a.eps);
   }
   for (uint32_t k0 = 0; k0 < K; k0 += KC) {
     const uint32_t q4 = std::min(KC, K - k0) / 4, g0 = k0 / 4;
@@ -183,10 +181,10 @@ __global__ __launch_bounds__(256) void k_bgemm(BgemmArgs a) {
     __syncthreads();
     if (NORM) {
       if (K <= KC) {
-        if (t < NB) s_inv[t] = inv_rms_of(sumsq_groups(Xs + t * xs4, q4, 0.0f, a.tree), K, a.eps);
+        if (t < TB) s_inv[t] = inv_rms_of(sumsq_groups(Xs + t * xs4, q4, 0.0f, a.tree), K, a.eps);
         __syncthreads();
       }
-      for (uint32_t i = t; i < NB * q4; i += kT) {
+      for (uint32_t i = t; i < TB * q4; i += kT) {
         const uint32_t bx = i / q4, q = i - bx * q4;
         const float inv = s_inv[bx];
         const v4 x = Xs[bx * xs4 + q], w = NWs[q];
@@ -203,76 +201,66 @@ __global__ __launch_bounds__(256) void k_bgemm(BgemmArgs a) {
     if (live) {
       const v4* wp = Ws + r;
       const v4* wp2 = Ws + qmax * R + r;
-      const v4* xp[CB];
-#pragma unroll
-      for (uint32_t c = 0; c < CB; ++c) xp[c] = Xs + (bb + c * TB) * xs4;
+      const v4* xp = Xs + bb * xs4;
       if (a.tree) {
         for (uint32_t q = 0; q < q4; q += 8) {
+          float l[32], l2[32];
 #pragma unroll
-          for (uint32_t c = 0; c < CB; ++c) {
-            float l[32], l2[32];
-#pragma unroll
-            for (uint32_t j = 0; j < 8; ++j) {
-              v4 w = v4{0.0f, 0.0f, 0.0f, 0.0f}, x = w, w2 = w;
-              if (q + j < q4) {
-                w = wp[(size_t)(q + j) * R];
-                x = xp[c][q + j];
-                if (DUAL) w2 = wp2[(size_t)(q + j) * R];
-              }
-              l[4 * j] = w.x * x.x;
-              l[4 * j + 1] = w.y * x.y;
-              l[4 * j + 2] = w.z * x.z;
-              l[4 * j + 3] = w.w * x.w;
-              if (DUAL) {
-                l2[4 * j] = w2.x * x.x;
-                l2[4 * j + 1] = w2.y * x.y;
-                l2[4 * j + 2] = w2.z * x.z;
-                l2[4 * j + 3] = w2.w * x.w;
-              }
+          for (uint32_t j = 0; j < 8; ++j) {
+            v4 w = v4{0.0f, 0.0f, 0.0f, 0.0f}, x = w, w2 = w;
+            if (q + j < q4) {
+              w = wp[(size_t)(q + j) * R];
+              x = xp[q + j];
+              if (DUAL) w2 = wp2[(size_t)(q + j) * R];
             }
-            acc[c] = acc[c] + tree32(l);
-            if (DUAL) acc2[c] = acc2[c] + tree32(l2);
+            l[4 * j] = w.x * x.x;
+            l[4 * j + 1] = w.y * x.y;
+            l[4 * j + 2] = w.z * x.z;
+            l[4 * j + 3] = w.w * x.w;
+            if (DUAL) {
+              l2[4 * j] = w2.x * x.x;
+              l2[4 * j + 1] = w2.y * x.y;
+              l2[4 * j + 2] = w2.z * x.z;
+              l2[4 * j + 3] = w2.w * x.w;
+            }
           }
+          acc = acc + tree32(l);
+          if (DUAL) acc2 = acc2 + tree32(l2);
         }
       } else {
         // software pipelined over two register sets: the reads of the next
         // 4 q go out before the current 4 q's products and chain steps
-        // (reads past the end are clamped to the last q and unused); a W
-        // group read serves the CB rows' chains
+        // (reads past the end are clamped to the last q and unused)
         constexpr uint32_t U = 4;
-        v4 aw[U], ax[CB][U], aw2[U], bw[U], bx[CB][U], bw2[U];
-        auto load = [&](v4 (&w)[U], v4 (&x)[CB][U], v4 (&w2)[U], uint32_t q0) {
+        v4 aw[U], ax[U], aw2[U], bw[U], bx[U], bw2[U];
+        auto load = [&](v4 (&w)[U], v4 (&x)[U], v4 (&w2)[U], uint32_t q0) {
 #pragma unroll
           for (uint32_t u = 0; u < U; ++u) {
             const uint32_t qq = std::min(q0 + u, q4 - 1);
             w[u] = wp[(size_t)qq * R];
-#pragma unroll
-            for (uint32_t c = 0; c < CB; ++c) x[c][u] = xp[c][qq];
+            x[u] = xp[qq];
             if (DUAL) w2[u] = wp2[(size_t)qq * R];
           }
         };
-        auto step = [&](const v4 (&w)[U], const v4 (&x)[CB][U], const v4 (&w2)[U]) {
+        auto step = [&](const v4 (&w)[U], const v4 (&x)[U], const v4 (&w2)[U]) {
+          float p[4 * U], p2[4 * U];
 #pragma unroll
-          for (uint32_t c = 0; c < CB; ++c) {
-            float p[4 * U], p2[4 * U];
-#pragma unroll
-            for (uint32_t u = 0; u < U; ++u) {
-              p[4 * u] = w[u].x * x[c][u].x;
-              p[4 * u + 1] = w[u].y * x[c][u].y;
-              p[4 * u + 2] = w[u].z * x[c][u].z;
-              p[4 * u + 3] = w[u].w * x[c][u].w;
-              if (DUAL) {
-                p2[4 * u] = w2[u].x * x[c][u].x;
-                p2[4 * u + 1] = w2[u].y * x[c][u].y;
-                p2[4 * u + 2] = w2[u].z * x[c][u].z;
-                p2[4 * u + 3] = w2[u].w * x[c][u].w;
-              }
+          for (uint32_t u = 0; u < U; ++u) {
+            p[4 * u] = w[u].x * x[u].x;
+            p[4 * u + 1] = w[u].y * x[u].y;
+            p[4 * u + 2] = w[u].z * x[u].z;
+            p[4 * u + 3] = w[u].w * x[u].w;
+            if (DUAL) {
+              p2[4 * u] = w2[u].x * x[u].x;
+              p2[4 * u + 1] = w2[u].y * x[u].y;
+              p2[4 * u + 2] = w2[u].z * x[u].z;
+              p2[4 * u + 3] = w2[u].w * x[u].w;
             }
+          }
 #pragma unroll
-            for (uint32_t i = 0; i < 4 * U; ++i) {
-              acc[c] = acc[c] + p[i];
-              if (DUAL) acc2[c] = acc2[c] + p2[i];
-            }
+          for (uint32_t i = 0; i < 4 * U; ++i) {
+            acc = acc + p[i];
+            if (DUAL) acc2 = acc2 + p2[i];
           }
         };
         uint32_t q = 0;
@@ -290,44 +278,36 @@ __global__ __launch_bounds__(256) void k_bgemm(BgemmArgs a) {
           }
         }
         for (; q < q4; ++q) {
-          const v4 w = wp[(size_t)q * R];
+          const v4 w = wp[(size_t)q * R], x = xp[q];
           const v4 w2 = DUAL ? wp2[(size_t)q * R] : w;
-#pragma unroll
-          for (uint32_t c = 0; c < CB; ++c) {
-            const v4 x = xp[c][q];
-            float pp;
-            pp = w.x * x.x; acc[c] = acc[c] + pp;
-            pp = w.y * x.y; acc[c] = acc[c] + pp;
-            pp = w.z * x.z; acc[c] = acc[c] + pp;
-            pp = w.w * x.w; acc[c] = acc[c] + pp;
-            if (DUAL) {
-              pp = w2.x * x.x; acc2[c] = acc2[c] + pp;
-              pp = w2.y * x.y; acc2[c] = acc2[c] + pp;
-              pp = w2.z * x.z; acc2[c] = acc2[c] + pp;
-              pp = w2.w * x.w; acc2[c] = acc2[c] + pp;
-            }
+          float pp;
+          pp = w.x * x.x; acc = acc + pp;
+          pp = w.y * x.y; acc = acc + pp;
+          pp = w.z * x.z; acc = acc + pp;
+          pp = w.w * x.w; acc = acc + pp;
+          if (DUAL) {
+            pp = w2.x * x.x; acc2 = acc2 + pp;
+            pp = w2.y * x.y; acc2 = acc2 + pp;
+            pp = w2.z * x.z; acc2 = acc2 + pp;
+            pp = w2.w * x.w; acc2 = acc2 + pp;
           }
         }
       }
     }
     __syncthreads();
   }
-  const uint32_t m = blk * R + r;
-#pragma unroll
-  for (uint32_t c = 0; c < CB; ++c) {
-    const uint32_t row = b0 + bb + c * TB;
-    if (live && row < a.n && m < g.M) {
-      float y = acc[c];
-      if (DUAL) {
-        const float sg = silu_pinned(acc[c]);
-        y = sg * acc2[c];
-      } else if (g.epi == kEpiBias) {
-        y = acc[c] + g.add[m];
-      } else if (g.epi == kEpiResidual) {
-        y = g.add[(size_t)row * g.ldadd + m] + acc[c];
-      }
-      g.Y[(size_t)row * g.ldy + m] = y;
+  const uint32_t m = blk * R + r, row = b0 + bb;
+  if (live && row < a.n && m < g.M) {
+    float y = acc;
+    if (DUAL) {
+      const float sg = silu_pinned(acc);
+      y = sg * acc2;
+    } else if (g.epi == kEpiBias) {
+      y = acc + g.add[m];
+    } else if (g.epi == kEpiResidual) {
+      y = g.add[(size_t)row * g.ldadd + m] + acc;
     }
+    g.Y[(size_t)row * g.ldy + m] = y;
   }
 }
 
@@ -598,6 +578,238 @@ __global__ __launch_bounds__(256) void k_bgemm16(BgemmArgs a) {
     }
     g.Y[(size_t)row * g.ldy + m] = y;
   }
+}
+
+// ---------------------------------------------------------------------------
+// Batched GEMM with the products formed by the matrix cores (sequential
+// order, any block height R).  One v_mfma_f32_16x16x1_4b_f32 multiplies four
+// pairs of 16-vectors; given the 16 W rows and 16 X rows of a tile at four
+// consecutive k, and -0 as the addend, each of its 4 x 256 results is one
+// correctly rounded product W[m][k] * X[b][k] (x + (-0) = x for every x, so
+// the sign of a zero product survives; flushing and NaN bits are those of
+// v_mul_f32).  All four blocks leave a given output in the same lane, so the
+// vector units only add: acc = acc + p, k ascending, the strict chain of
+// k_bgemm (code/cis2-fp/src/main.rs:228-243, math.rs:40-48).
+// ---------------------------------------------------------------------------
+typedef float f16v __attribute__((ext_vector_type(16)));
+
+// The four products of a 16 x 16 tile: a holds W[row l % 16][k + l / 16] and
+// b X[row l % 16][k + l / 16] of lane l; element 4u + r of the result is
+// output (W row 4 (l / 16) + r, X row l % 16) at k + u.
+__device__ __forceinline__ f16v products4(float a, float b, const f16v& nz) {
+  return __builtin_amdgcn_mfma_f32_16x16x1f32(a, b, nz, 0, 0, 0);
+}
+// A 16-register operand of -0.
+__device__ __forceinline__ f16v minus_zeros() {
+  float z = __int_as_float((int)0x80000000u);
+  asm volatile("" : "+v"(z));
+  f16v v;
+#pragma unroll
+  for (uint32_t i = 0; i < 16; ++i) v[i] = z;
+  return v;
+}
+
+struct MgemmArgs {
+  BgemmSeg s[kMaxSegs];
+  uint32_t tile0[kMaxSegs + 1];  // first W tile of each segment; tile0[nseg] = W tiles
+  uint32_t nseg, n, tiles;       // tiles: W tiles x X tiles
+  uint32_t vec;                  // 1: outputs (and addends) in 16-byte groups
+  const float* W2;               // DUAL
+};
+
+// What bounds it: the vector and matrix units.  A CU forms a product on
+// either in the same time and they do not overlap (a wave64 product step of
+// 1024 and its 16 adds: 32 + 32 cycles per SIMD with two or more waves), so
+// the least is 64 cycles per 1024 chain steps, 39 T steps/s at 2.4 GHz; 16384
+// rows run at 26 .. 30 T (k_bgemm16: 10 .. 13 T: a DPP broadcast, a multiply
+// and an add per 64 steps, 16 cycles).  Letting the matrix cores form the
+// products saves the operand reads instead: 16 + 16 values feed 256 chains.
+//
+// Four waves, WM x WN of them, each SM x SN tiles of 16 outputs x 16 batch
+// rows.  DUAL: the first half of a wave's SM tiles comes from W, the second
+// half from W2 at the same rows, and silu(gate) * up is stored
+// (main.rs:484-487).
+// LDS, two buffers of one K chunk each: [chunk / 16][4][rows] 16-byte groups;
+// group (g, u, row) holds k = 16 g + u + {0, 4, 8, 12} of the row, so that a
+// wave's 16-byte read gives lane l (row l % 16, u = l / 16) its operands of
+// four products4.  A thread stages whole (row, 16 k) pieces: four 16-byte
+// loads, transposed by register naming.  Past K the pieces hold -0 for W and
+// +0 for X: their products are -0, which no sum notices.  Chunk c + PF is
+// loaded into registers while chunk c is computed.
+template <bool DUAL, uint32_t SM, uint32_t SN, uint32_t WM, uint32_t WN, uint32_t KC>
+struct MgemmCfg {
+  static constexpr uint32_t BM = 16 * SM * WM / (DUAL ? 2 : 1);  // W rows per tile
+  static constexpr uint32_t BN = 16 * SN * WN;                   // X rows per tile
+  static constexpr uint32_t RA = 16 * SM * WM, RB = BN, ROWS = RA + RB;
+  static constexpr uint32_t NG = KC / 16;
+  static constexpr uint32_t items = ROWS * NG, NIT = (items + 255) / 256;
+  static constexpr size_t buf = (size_t)4 * ROWS * NG;  // 16-byte groups of one buffer
+  static_assert(WM * WN == 4 && (!DUAL || SM % 2 == 0), "four waves");
+};
+
+template <bool DUAL, uint32_t SM, uint32_t SN, uint32_t WM, uint32_t WN, uint32_t KC,
+          uint32_t OCC, uint32_t PF>
+__global__ __launch_bounds__(256, OCC) void k_mgemm(MgemmArgs a) {
+  using C = MgemmCfg<DUAL, SM, SN, WM, WN, KC>;
+  constexpr uint32_t ROWS = C::ROWS, RA = C::RA, NG = C::NG, NIT = C::NIT, NT = SM * SN;
+  __shared__ v4 sm[2 * C::buf];
+  // consecutive workgroups go to the eight XCDs in turn: give each XCD a run
+  // of tiles, W tiles first, so that the tiles of one X tile share its L2
+  const uint32_t per = (a.tiles + 7) / 8;
+  const uint32_t tile = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+  if ((blockIdx.x >> 3) >= per || tile >= a.tiles) return;
+  const uint32_t wt = a.tile0[a.nseg], nt = tile / wt, ut = tile - nt * wt;
+  uint32_t si = 0;
+  if (a.nseg > 1 && ut >= a.tile0[1]) si = (a.nseg > 2 && ut >= a.tile0[2]) ? 2 : 1;
+  const BgemmSeg g = si == 0 ? a.s[0] : (si == 1 ? a.s[1] : a.s[2]);
+  const uint32_t m0 = (ut - a.tile0[si]) * C::BM, n0 = nt * C::BN;
+  const uint32_t t = threadIdx.x, wv = __builtin_amdgcn_readfirstlane(t >> 6), lane = t & 63;
+  const uint32_t K4 = g.K / 4, lastblk = (g.M - 1) / g.R;
+  // staging: piece it of this thread
+  const v4* src[NIT];
+  uint32_t step[NIT], q0[NIT], dst[NIT];
+  bool isw[NIT];
+#pragma unroll
+  for (uint32_t j = 0; j < NIT; ++j) {
+    const uint32_t it = min(j * 256 + t, C::items - 1);
+    const uint32_t row = it % ROWS, gi = it / ROWS;
+    isw[j] = row < RA;
+    if (isw[j]) {
+      // rows past M belong to no output: any stored block serves
+      const bool second = DUAL && row >= RA / 2;
+      const uint32_t m = m0 + (second ? row - RA / 2 : row);
+      const uint32_t blk = min(m / g.R, lastblk), r = m % g.R;
+      src[j] = reinterpret_cast<const v4*>((second ? a.W2 : g.W) + (size_t)blk * g.R * g.K) + r;
+      step[j] = g.R;
+    } else {
+      const uint32_t b = min(n0 + row - RA, a.n - 1);
+      src[j] = reinterpret_cast<const v4*>(g.X + (size_t)b * g.ldx);
+      step[j] = 1;
+    }
+    q0[j] = 4 * gi;
+    dst[j] = 4 * gi * ROWS + row;
+  }
+  v4 stage[PF][NIT][4];
+  auto load = [&](uint32_t k0, v4 (&st)[NIT][4]) {
+#pragma unroll
+    for (uint32_t j = 0; j < NIT; ++j)
+#pragma unroll
+      for (uint32_t i = 0; i < 4; ++i) {
+        const uint32_t q = k0 / 4 + q0[j] + i;
+        if (q < K4) {
+          st[j][i] = src[j][(size_t)q * step[j]];
+        } else {
+          const float z = isw[j] ? __int_as_float((int)0x80000000u) : 0.0f;
+          st[j][i] = v4{z, z, z, z};
+        }
+      }
+  };
+  auto store = [&](uint32_t b, const v4 (&st)[NIT][4]) {
+    v4* p = sm + b * C::buf;
+#pragma unroll
+    for (uint32_t j = 0; j < NIT; ++j) {
+      if (C::items % 256 && j * 256 + t >= C::items) break;
+#pragma unroll
+      for (uint32_t u = 0; u < 4; ++u)
+        p[dst[j] + u * ROWS] = v4{st[j][0][u], st[j][1][u], st[j][2][u], st[j][3][u]};
+    }
+  };
+  // wave (wm, wn); tile i of its SM: rows 16 * (i * WM + wm) for one matrix,
+  // of W then of W2 for DUAL
+  const uint32_t wm = wv % WM, wn = wv / WM, u = lane >> 4, c16 = lane & 15;
+  constexpr uint32_t SMH = DUAL ? SM / 2 : SM;
+  auto arow = [&](uint32_t i) {  // first LDS row of A tile i
+    const uint32_t h = i / SMH, ii = i - h * SMH;
+    return h * (RA / 2) * (DUAL ? 1 : 0) + 16 * (wm * SMH + ii);
+  };
+  const f16v nz = minus_zeros();
+  float acc[NT][4];
+#pragma unroll
+  for (uint32_t s = 0; s < NT; ++s)
+#pragma unroll
+    for (uint32_t r = 0; r < 4; ++r) acc[s][r] = 0.0f;
+  f16v d[2];
+#pragma unroll
+  for (uint32_t i = 0; i < 16; ++i) d[1][i] = __int_as_float((int)0x80000000u);
+  auto add = [&](uint32_t s, const f16v& p) {
+#pragma unroll
+    for (uint32_t b = 0; b < 4; ++b)
+#pragma unroll
+      for (uint32_t r = 0; r < 4; ++r) acc[s][r] = acc[s][r] + p[4 * b + r];
+    asm volatile("" : "+v"(acc[s][0]), "+v"(acc[s][1]), "+v"(acc[s][2]), "+v"(acc[s][3]));
+  };
+  const uint32_t nc = (g.K + KC - 1) / KC;
+  load(0, stage[0]);
+  if (PF == 2 && nc > 1) load(KC, stage[1]);
+  store(0, stage[0]);
+  auto chunk = [&](uint32_t ci, v4 (&cur)[NIT][4], v4 (&nxt)[NIT][4]) {
+    __syncthreads();
+    if (ci + PF < nc) load((ci + PF) * KC, cur);
+    const v4* p = sm + (ci & 1) * C::buf + u * ROWS + c16;
+    v4 fa[2][SM], fb[2][SN];
+    auto frags = [&](uint32_t gi, uint32_t f) {
+#pragma unroll
+      for (uint32_t i = 0; i < SM; ++i) fa[f][i] = p[4 * gi * ROWS + arow(i)];
+#pragma unroll
+      for (uint32_t j = 0; j < SN; ++j) fb[f][j] = p[4 * gi * ROWS + RA + 16 * (wn * SN + j)];
+    };
+    frags(0, 0);
+#pragma unroll
+    for (uint32_t gi = 0; gi < NG; ++gi) {
+      if (gi + 1 < NG) frags(gi + 1, (gi + 1) & 1);
+#pragma unroll
+      for (uint32_t m = 0; m < 4; ++m)
+#pragma unroll
+        for (uint32_t s = 0; s < NT; ++s) {
+          // products of tile s while the vector units add the tile before it
+          const uint32_t x = m * NT + s;
+          d[x & 1] = products4(fa[gi & 1][s / SN][m], fb[gi & 1][s % SN][m], nz);
+          asm volatile("" : "+v"(d[x & 1]));
+          add((s + NT - 1) % NT, d[(x + 1) & 1]);
+        }
+    }
+    if (ci + 1 < nc) store((ci + 1) & 1, nxt);
+  };
+  // chunk ci is computed while chunk ci + PF is loaded
+  for (uint32_t ci = 0; ci < nc; ci += PF) {
+    chunk(ci, stage[0], stage[PF - 1]);
+    if (PF == 2 && ci + 1 < nc) chunk(ci + 1, stage[1 % PF], stage[0]);
+  }
+  add(NT - 1, d[1]);
+  // epilogue: lane l holds outputs m .. m+3 of X row n
+#pragma unroll
+  for (uint32_t i = 0; i < SMH; ++i)
+#pragma unroll
+    for (uint32_t j = 0; j < SN; ++j) {
+      const uint32_t m = m0 + 16 * (wm * SMH + i) + 4 * u, row = n0 + 16 * (wn * SN + j) + c16;
+      if (row >= a.n || m >= g.M) continue;
+      float y[4];
+#pragma unroll
+      for (uint32_t r = 0; r < 4; ++r) y[r] = acc[i * SN + j][r];
+      float* yp = g.Y + (size_t)row * g.ldy + m;
+      if (DUAL) {
+#pragma unroll
+        for (uint32_t r = 0; r < 4; ++r) {
+          const float sg = silu_pinned(y[r]);
+          y[r] = sg * acc[(SMH + i) * SN + j][r];
+        }
+      }
+      const float* ad = nullptr;
+      if (!DUAL && g.epi == kEpiBias) ad = g.add + m;
+      if (!DUAL && g.epi == kEpiResidual) ad = g.add + (size_t)row * g.ldadd + m;
+      if (a.vec) {
+        if (ad) {
+          const v4 z = *reinterpret_cast<const v4*>(ad);
+#pragma unroll
+          for (uint32_t r = 0; r < 4; ++r) y[r] = g.epi == kEpiBias ? y[r] + z[r] : z[r] + y[r];
+        }
+        *reinterpret_cast<v4*>(yp) = v4{y[0], y[1], y[2], y[3]};
+      } else {
+#pragma unroll
+        for (uint32_t r = 0; r < 4; ++r)
+          if (m + r < g.M) yp[r] = ad ? (g.epi == kEpiBias ? y[r] + ad[r] : ad[r] + y[r]) : y[r];
+      }
+    }
 }
 
 // (value, index) pick of a strict-> scan from index 0 (first maximum wins;
@@ -1716,9 +1928,9 @@ __global__ __launch_bounds__(1024) void k_argmax_rows(const float* __restrict__ 
 
 }  // namespace
 
-template <bool DUAL, bool NORM, uint32_t CB>
+template <bool DUAL, bool NORM>
 hipError_t launch_bgemm_t(const BgemmArgs& a, dim3 grid, size_t lds, hipStream_t st) {
-  hipLaunchKernelGGL((k_bgemm<DUAL, NORM, CB>), grid, dim3(kT), lds, st, a);
+  hipLaunchKernelGGL((k_bgemm<DUAL, NORM>), grid, dim3(kT), lds, st, a);
   return hipGetLastError();
 }
 
@@ -1727,16 +1939,14 @@ hipError_t launch_bgemm_t(const BgemmArgs& a, dim3 grid, size_t lds, hipStream_t
 // attention), so that no attribute call happens later, e.g. inside a graph
 // capture.
 hipError_t rows_configure() {
-  const void* fns[20] = {reinterpret_cast<const void*>(&k_bgemm<false, false, 1>),
+  const void* fns[18] = {reinterpret_cast<const void*>(&k_bgemm<false, false>),
                          reinterpret_cast<const void*>(&k_bgemm16<false, false>),
                          reinterpret_cast<const void*>(&k_bgemm16<false, true>),
                          reinterpret_cast<const void*>(&k_bgemm16<true, false>),
                          reinterpret_cast<const void*>(&k_bgemm16<true, true>),
-                         reinterpret_cast<const void*>(&k_bgemm<false, true, 1>),
-                         reinterpret_cast<const void*>(&k_bgemm<true, false, 1>),
-                         reinterpret_cast<const void*>(&k_bgemm<true, true, 1>),
-                         reinterpret_cast<const void*>(&k_bgemm<false, false, 2>),
-                         reinterpret_cast<const void*>(&k_bgemm<true, false, 2>),
+                         reinterpret_cast<const void*>(&k_bgemm<false, true>),
+                         reinterpret_cast<const void*>(&k_bgemm<true, false>),
+                         reinterpret_cast<const void*>(&k_bgemm<true, true>),
                          reinterpret_cast<const void*>(&k_attention_kv<1, 64, false>),
                          reinterpret_cast<const void*>(&k_attention_kv<2, 64, false>),
                          reinterpret_cast<const void*>(&k_attention_kv<3, 64, false>),
@@ -1754,18 +1964,8 @@ hipError_t rows_configure() {
   return hipSuccess;
 }
 
-// CIS2_BGEMM_CB=1 keeps one batch row per thread on every grid (for A/B
-// timing of the two-row form; the results are the same bits either way).
-static bool bgemm_cb_allowed() {
-  static const bool allowed = [] {
-    const char* e = std::getenv("CIS2_BGEMM_CB");
-    return !(e && e[0] == '1' && e[1] == 0);
-  }();
-  return allowed;
-}
-
-// CIS2_BGEMM16=0 keeps every batched GEMM on k_bgemm (for A/B timing; the
-// results are the same bits either way).
+// CIS2_BGEMM16=0 keeps every batched GEMM on k_bgemm (for A/B timing and
+// tests; the results are the same bits either way).
 static bool bgemm16_allowed() {
   const char* e = std::getenv("CIS2_BGEMM16");
   return !(e && e[0] == '0' && e[1] == 0);
@@ -1817,6 +2017,67 @@ static hipError_t launch_bgemm16(const BgemmSeg* segs, uint32_t nseg, uint32_t n
   return hipGetLastError();
 }
 
+template <bool DUAL, uint32_t SM, uint32_t SN, uint32_t WM, uint32_t WN, uint32_t KC,
+          uint32_t OCC, uint32_t PF>
+static hipError_t launch_mgemm(const BgemmSeg* segs, uint32_t nseg, uint32_t n,
+                                 const float* W2, hipStream_t st) {
+  using C = MgemmCfg<DUAL, SM, SN, WM, WN, KC>;
+  MgemmArgs a = {};
+  a.nseg = nseg;
+  a.n = n;
+  a.W2 = W2;
+  a.vec = 1;
+  for (uint32_t i = 0; i < kMaxSegs; ++i) {
+    a.s[i] = segs[i < nseg ? i : 0];
+    if (i < nseg) {
+      a.tile0[i + 1] = a.tile0[i] + (segs[i].M + C::BM - 1) / C::BM;
+      if (segs[i].M % 4 || segs[i].ldy % 4 || segs[i].ldadd % 4) a.vec = 0;
+    } else {
+      a.tile0[i + 1] = a.tile0[nseg];
+    }
+  }
+  const uint64_t tiles = (uint64_t)a.tile0[nseg] * ((n + C::BN - 1) / C::BN);
+  if (tiles > 0x7fffffffu - 8) return hipErrorInvalidValue;
+  a.tiles = (uint32_t)tiles;
+  hipLaunchKernelGGL((k_mgemm<DUAL, SM, SN, WM, WN, KC, OCC, PF>), dim3((a.tiles + 7) / 8 * 8),
+                     dim3(256), 0, st, a);
+  return hipGetLastError();
+}
+
+// Which kernel a sequential-order GEMM without a fused norm takes.  Every
+// form costs a time per k that depends on how many workgroups the fullest CU
+// gets; measured on the layer shapes of the three models at n = 7 .. 16384,
+// in ns per k (two figures: one matrix, gate and up):
+//   k_bgemm16 / k_bgemm  256 chains per workgroup     11 | 21 at one per CU,
+//                                                     7.7 | 14.5 each beyond
+//   k_mgemm, 32 x 32     1024 chains (2048 for two)   19 | 39, then 11 | 21 each
+//   k_mgemm, 64 x 64     4096 chains                  57, then 37.5 each
+// A small grid is bound by one wave's latency and wants many short
+// workgroups, a large one by the vector units and wants operands reused: the
+// least of the three estimates is taken.  (o projection of 576 x 576, us:
+// n = 64 8.6 | 12.8 | 35.4, n = 544 23.3 | 16.8 | 35.7, n = 16384 518 | 254 |
+// 188; gate and up of 3072 x 1024 at n = 16384 8254 | 3635 | 3293.)
+enum class MgemmTile { none, small, large };
+static MgemmTile mgemm_tile(const BgemmSeg* segs, uint32_t nseg, uint32_t n, bool dual,
+                            uint32_t ncu) {
+  uint64_t t16 = 0, t32 = 0, t64 = 0;  // W tiles of 16, 32 (16 x 64 rows) and 64 rows
+  const uint32_t sm = n <= 16 && !dual ? 64 : 32, sn = n <= 16 && !dual ? 16 : 32;
+  for (uint32_t i = 0; i < nseg; ++i) {
+    t16 += (segs[i].M + 15) / 16;
+    t32 += (segs[i].M + sm - 1) / sm;
+    t64 += (segs[i].M + (dual ? 31 : 63)) / (dual ? 32 : 64);
+  }
+  auto per_cu = [&](uint64_t wt, uint32_t bn) {
+    return (double)((wt * ((n + bn - 1) / bn) + ncu - 1) / ncu);
+  };
+  const double two = dual ? 2.0 : 1.0;
+  const double t0 = std::max(10.5, 7.5 * per_cu(t16, 16)) * two;
+  const double ts = std::max(19.0, 10.5 * per_cu(t32, sn) + 2.0) * two;
+  const double tl = std::max(57.0, 37.5 * per_cu(t64, 64));
+  if (t0 <= ts && t0 <= tl) return MgemmTile::none;
+  return ts <= tl ? MgemmTile::small : MgemmTile::large;
+}
+
 hipError_t launch_bgemm_multi(const BgemmSeg* segs, uint32_t nseg, uint32_t n,
                               const BgemmOpts& o, hipStream_t st) {
   if (n == 0) return hipSuccess;
@@ -1827,22 +2088,35 @@ hipError_t launch_bgemm_multi(const BgemmSeg* segs, uint32_t nseg, uint32_t n,
   }
   const BgemmSeg& s0 = segs[0];
   if (s0.K % 4 || s0.ldx % 4 || s0.R == 0 || s0.R > kT) return hipErrorInvalidValue;
+  for (uint32_t i = 0; i < nseg; ++i)
+    if (segs[i].M == 0 || segs[i].K != s0.K || segs[i].R != s0.R || segs[i].X != s0.X ||
+        segs[i].ldx != s0.ldx)
+      return hipErrorInvalidValue;
   const int ncu = device_cu_count();
-  {
-    bool tiles = !o.tree && (s0.R == 8 || s0.R == 16) && bgemm16_allowed();
-    for (uint32_t i = 0; i < nseg && tiles; ++i)
-      tiles = segs[i].M % 16 == 0 && segs[i].R == s0.R && segs[i].K == s0.K &&
-              segs[i].X == s0.X && segs[i].ldx == s0.ldx;
+  if (!o.tree && bgemm16_allowed()) {
+    if (!o.norm_w) {
+      switch (mgemm_tile(segs, nseg, n, o.W2 != nullptr, (uint32_t)ncu)) {
+        case MgemmTile::large:
+          return o.W2 ? launch_mgemm<true, 2, 2, 2, 2, 32, 3, 1>(segs, nseg, n, o.W2, st)
+                      : launch_mgemm<false, 2, 2, 2, 2, 32, 3, 1>(segs, nseg, n, o.W2, st);
+        case MgemmTile::small:
+          if (o.W2) return launch_mgemm<true, 2, 1, 2, 2, 32, 2, 2>(segs, nseg, n, o.W2, st);
+          // up to 16 rows: 64 x 16 tiles (the LM head at n = 16: 26 against 41 us)
+          return n <= 16 ? launch_mgemm<false, 1, 1, 4, 1, 64, 2, 1>(segs, nseg, n, o.W2, st)
+                         : launch_mgemm<false, 1, 1, 2, 2, 64, 3, 2>(segs, nseg, n, o.W2, st);
+        default:
+          break;
+      }
+    }
+    bool tiles = s0.R == 8 || s0.R == 16;
+    for (uint32_t i = 0; i < nseg && tiles; ++i) tiles = segs[i].M % 16 == 0;
     if (tiles) return launch_bgemm16(segs, nseg, n, o, ncu, st);
   }
   BgemmArgs a = {};
   a.blk0[0] = 0;
   for (uint32_t i = 0; i < nseg; ++i) {
-    const BgemmSeg& s = segs[i];
-    if (s.M == 0 || s.K != s0.K || s.R != s0.R || s.X != s0.X || s.ldx != s0.ldx)
-      return hipErrorInvalidValue;
-    a.s[i] = s;
-    a.blk0[i + 1] = a.blk0[i] + (s.M + s.R - 1) / s.R;
+    a.s[i] = segs[i];
+    a.blk0[i + 1] = a.blk0[i] + (segs[i].M + segs[i].R - 1) / segs[i].R;
   }
   for (uint32_t i = nseg; i < kMaxSegs; ++i) {
     a.s[i] = s0;
@@ -1857,10 +2131,6 @@ hipError_t launch_bgemm_multi(const BgemmSeg* segs, uint32_t nseg, uint32_t n,
   a.eps = o.eps;
   const uint32_t S = o.W2 ? 2 : 1;
   const uint64_t wgs = (uint64_t)a.blk0[nseg] * ((n + a.TB - 1) / a.TB);
-  // grids of many workgroups per CU (prefill) give each thread two batch
-  // rows, so that one W read from LDS feeds two chains
-  const uint32_t CB = (!o.norm_w && !o.tree && wgs >= 8ull * ncu && bgemm_cb_allowed()) ? 2 : 1;
-  const uint32_t NB = a.TB * CB;
   // a grid of at most one workgroup per CU may take most of a CU's LDS
   // (fewer K chunks, each a full round trip); larger grids keep two
   // workgroups per CU, so that up to two per CU all run at once
@@ -1868,20 +2138,18 @@ hipError_t launch_bgemm_multi(const BgemmSeg* segs, uint32_t nseg, uint32_t n,
   // largest chunk (a multiple of 32 k) whose W slices, X rows and norm
   // weights fit
   const uint32_t NW = o.norm_w ? 1 : 0;
-  const uint32_t q_fit = (budget / 16 - NB) / (S * s0.R + NB + NW);
+  const uint32_t q_fit = (budget / 16 - a.TB) / (S * s0.R + a.TB + NW);
   uint32_t KC = (q_fit * 4) & ~31u;
   if (KC == 0) return hipErrorInvalidValue;
   const uint32_t K32 = (s0.K + 31) & ~31u;
   if (KC > K32) KC = K32;
   a.KC = KC;
-  const size_t lds = ((size_t)(KC / 4) * (s0.R * S + NW) + (size_t)NB * (KC / 4 + 1)) * 16;
-  const dim3 grid(a.blk0[nseg], (n + NB - 1) / NB);
-  if (CB == 2) return o.W2 ? launch_bgemm_t<true, false, 2>(a, grid, lds, st)
-                           : launch_bgemm_t<false, false, 2>(a, grid, lds, st);
-  if (o.W2) return o.norm_w ? launch_bgemm_t<true, true, 1>(a, grid, lds, st)
-                            : launch_bgemm_t<true, false, 1>(a, grid, lds, st);
-  return o.norm_w ? launch_bgemm_t<false, true, 1>(a, grid, lds, st)
-                  : launch_bgemm_t<false, false, 1>(a, grid, lds, st);
+  const size_t lds = ((size_t)(KC / 4) * (s0.R * S + NW) + (size_t)a.TB * (KC / 4 + 1)) * 16;
+  const dim3 grid(a.blk0[nseg], (n + a.TB - 1) / a.TB);
+  if (o.W2) return o.norm_w ? launch_bgemm_t<true, true>(a, grid, lds, st)
+                            : launch_bgemm_t<true, false>(a, grid, lds, st);
+  return o.norm_w ? launch_bgemm_t<false, true>(a, grid, lds, st)
+                  : launch_bgemm_t<false, false>(a, grid, lds, st);
 }
 
 hipError_t launch_bgemm(const BgemmSeg& s, uint32_t n, bool tree, hipStream_t st) {
