@@ -1570,331 +1570,388 @@ __global__ __launch_bounds__(kKvT) void k_attention_kv(const float* __restrict__
 
 // ---------------------------------------------------------------------------
 // Attention of prefill rows in tiles.  A tile is up to kAttQT rows of one
-// sequence at consecutive positions p0 .. p0+nr-1 (built on the host); a
-// workgroup takes one tile and the HPW = nh/nkv query heads of one KV head,
-// P = kAttQT * HPW (row, head) pairs (pair a = row i * HPW + head h), and
-// reads each K and V element of the kv head once for all of them, where the
-// per-row kernel reads them once per row.  Each pair's arithmetic is the
-// per-row kernel's, in the same order (sequential reduction order only):
-//   scores  s_j = dot_seq(q, k_j) * scale, d ascending: K tiles of TK
-//           positions in LDS, a thread carries PB pairs x 4 positions; the
-//           scores go to a global scratch row per pair, the first-wins
-//           maximum (NaN at position 0 wins) is kept on the way;
+// sequence at consecutive positions p0 .. p0+nr-1 (built on the host); a work
+// item is one tile and HPT query heads of one KV head, P = kAttQT * HPT
+// (row, head) pairs (pair a = head h * 16 + row i).  Each pair's arithmetic
+// is the per-row kernel's, in the same order (sequential reduction order
+// only), with the products of both contractions formed by the matrix cores
+// (products4, above) and the chains' adds by the vector units:
+//   scores  s_j = dot_seq(q, k_j) * scale, d ascending: A is 16 pairs of one
+//           head, B 16 positions; a wave takes 64 positions at a time, and a
+//           16-byte load per lane of 4 rows of K is the B operand of four
+//           position tiles, straight from global memory, used by all HPT
+//           heads; the scores go to a scratch row per pair, the maximum (NaN
+//           at position 0 wins) is kept on the way;
 //   softmax the denominator as one strict chain per pair: waves 1..3 copy
 //           stages of TE scores into LDS one stage ahead and turn them into
 //           exp(s - max) in place (written back for the V-mix) while lanes
 //           a < P of wave 0 continue their chains;
-//   V-mix   out_d = fold_j (p_j * v_j[d]), j ascending, p_j = e_j / den:
-//           V tiles and e tiles of TK positions in LDS (the next pair copied
-//           while the current one is used), a thread carries PB3 pairs x 4
-//           dims.
-// LDS (floats): q [P][HD+4], then the phase regions (K tiles 2 x [HD][TK];
-// e stages 2 x [P][TE+4]; V tiles 2 x [HD][TK+4] + e tiles 2 x [P][TK+4]),
-// plus the per-pair maximum and denominator.
+//   V-mix   out_d = fold_j (p_j * v_j[d]), j ascending, p_j = e_j / den: A is
+//           16 pairs, B 16 dims; the p tiles of TP positions are divided one
+//           tile ahead into LDS in operand order, V goes from global memory
+//           to registers (four groups of 16 positions ahead) and is
+//           transposed between lanes there (permlane swaps).  In the groups
+//           that reach past the tile's first row's length every add is
+//           selected by j < the row's length.
+// What bounds it: the vector and matrix units, at the GEMM's 64 cycles per
+// 1024 chain steps, and the exps (about a fifth of a head_dim-64 step).
+// 4096 rows of 16 heads of 128: 1.89 ms per layer (18 T chain steps/s),
+// 4.32 ms with operands read from LDS and multiplied by the vector units;
+// 64 ragged prompts of 16 .. 512 rows, 9 heads of 64: 0.31 ms against 1.37.
+// Workgroups walk the items with a fixed stride, the longest tiles first and
+// every other round in reverse order, each with one scratch slot, so the
+// scratch stays a few hundred MB whatever the row count; the stride is a
+// multiple of 8 and the heads of a tile are neighbours, so the XCD that a
+// workgroup runs on meets one KV head of eight and keeps it in its L2.
+// LDS: q in operand order, then the phase regions (e stages 2 x [P][TE+4]; p
+// tiles 2 x [P][TP]), the wave maxima, the pairs' maximum and denominator.
 // ---------------------------------------------------------------------------
 constexpr uint32_t kAttQT = kAttTileRows;  // rows per attention tile
-constexpr uint32_t kAttTE = 128; // positions per softmax stage
+constexpr uint32_t kAttTE = 64;            // positions per softmax stage
+static_assert(kAttQT == 16, "a tile's rows are one operand's rows");
 
-template <uint32_t HPW, uint32_t HD, uint32_t TK>
+template <uint32_t HPT>
 struct AttTileCfg {
-  static constexpr uint32_t P = kAttQT * HPW;
-  static constexpr uint32_t QS = HD + 4;                 // q row stride
-  static constexpr uint32_t PB = P * TK / 1024;          // pairs per thread, scores
-  static constexpr uint32_t PB3 = P * HD / 1024;         // pairs per thread, V-mix
-  static constexpr uint32_t ES = kAttTE + 4;             // e stage row stride
-  static constexpr uint32_t VS = TK + 4;                 // V / e tile row stride
-  static constexpr size_t region1 = 2 * (size_t)HD * TK;
-  static constexpr size_t region2 = 2 * (size_t)P * ES;
-  static constexpr size_t region3 = 2 * (size_t)HD * VS + 2 * (size_t)P * VS;
-  static constexpr size_t region = region1 > region2 ? (region1 > region3 ? region1 : region3)
-                                                     : (region2 > region3 ? region2 : region3);
-  static constexpr size_t floats = (size_t)P * QS + region + 2 * P;
-  static_assert(P * TK % 1024 == 0 && P * HD % 1024 == 0, "thread blocking");
+  static constexpr uint32_t P = kAttQT * HPT;
+  static constexpr uint32_t ES = kAttTE + 4;                             // e stage row stride
+  static constexpr uint32_t TP = HPT >= 3 ? 64 : (HPT == 2 ? 128 : 256);  // positions per p tile
+  static constexpr size_t region1 = 2 * (size_t)P * ES, region2 = 2 * (size_t)P * TP;
+  static constexpr size_t region = region1 > region2 ? region1 : region2;
+  static constexpr size_t floats(uint32_t hd) { return (size_t)P * hd + region + 6 * P; }
+  static_assert(P * TP / 16 <= 256, "one p piece per thread");
   static_assert(P <= 64, "one denominator lane per pair in wave 0");
 };
 
-// n positions of `rows` rows (row stride `gstride` floats in global memory,
-// starting at src) into LDS rows of stride `lstride` at dst, 16 bytes per
-// lane with global_load_lds_dwordx4, one wave instruction per 256 positions
-// of a row; waves [w0, w0 + nw) issue the rows w0-relative round-robin.
-__device__ __forceinline__ void copy_rows_lds(float* dst, uint32_t lstride, const float* src,
-                                              size_t gstride, uint32_t rows, uint32_t n,
-                                              uint32_t w0, uint32_t nw) {
-  const uint32_t n4 = (n + 3) >> 2, lane = threadIdx.x & 63;
-  const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  if (w < w0 || w >= w0 + nw) return;
-  for (uint32_t r = w - w0; r < rows; r += nw)
-    for (uint32_t q0 = 0; q0 < n4; q0 += 64)
-      if (q0 + lane < n4)
-        lds_load16(reinterpret_cast<const v4*>(src + r * gstride) + q0 + lane,
-                   reinterpret_cast<v4*>(dst + (size_t)r * lstride) + q0);
+// Lane l's four values x = M[l / 16 row][4 (l / 16) + c] become
+// M[row][4 c + l / 16]: a 4 x 4 transpose between the 16-lane groups.
+__device__ __forceinline__ void transpose4(v4& x) {
+  typedef uint32_t u2 __attribute__((ext_vector_type(2)));
+  uint32_t r[4];
+#pragma unroll
+  for (uint32_t i = 0; i < 4; ++i) r[i] = __float_as_uint(x[i]);
+  u2 a = __builtin_amdgcn_permlane16_swap(r[0], r[1], false, false);
+  u2 b = __builtin_amdgcn_permlane16_swap(r[2], r[3], false, false);
+  u2 c = __builtin_amdgcn_permlane32_swap(a[0], b[0], false, false);
+  u2 d = __builtin_amdgcn_permlane32_swap(a[1], b[1], false, false);
+  x = v4{__uint_as_float(c[0]), __uint_as_float(d[0]), __uint_as_float(c[1]),
+         __uint_as_float(d[1])};
 }
 
-template <uint32_t HPW, uint32_t HD, uint32_t TK>
-__global__ __launch_bounds__(256) void k_attention_tiles(
+template <uint32_t HPT, uint32_t HD>
+__global__ __launch_bounds__(256, 2) void k_attention_tiles(
     const float* __restrict__ q, const float* __restrict__ kc, const float* __restrict__ vc,
-    const AttTile* __restrict__ tiles, uint32_t nh, uint32_t max_pos, uint64_t seq_stride,
-    float scale, float* out, float* scratch, uint32_t ls) {
-  using C = AttTileCfg<HPW, HD, TK>;
-  constexpr uint32_t P = C::P, QS = C::QS, PB = C::PB, PB3 = C::PB3, ES = C::ES, VS = C::VS;
+    const AttTile* __restrict__ tiles, uint32_t nitem, uint32_t nh, uint32_t group,
+    uint32_t max_pos, uint64_t seq_stride, float scale, float* out, float* scratch, uint32_t ls) {
+  using C = AttTileCfg<HPT>;
+  constexpr uint32_t P = C::P, ES = C::ES, TP = C::TP, DG = HD / 16, NB = HD / 64;
+  constexpr uint32_t NT1 = 4 * HPT, NT3 = HPT * NB;
   extern __shared__ v4 sh4[];
-  float* sh = reinterpret_cast<float*>(sh4);
-  float* qs = sh;                                  // [P][QS]
-  float* reg = qs + (size_t)P * QS;                // phase region
-  float* smx = reg + C::region;                    // [P] maxima
+  v4* qf = sh4;                                    // [DG][4][P]
+  float* reg = reinterpret_cast<float*>(qf + (size_t)DG * 4 * P);
+  float* wmx = reg + C::region;                    // [4][P] wave maxima
+  float* smx = wmx + 4 * P;                        // [P] maxima
   float* sden = smx + P;                           // [P] denominators
-  const AttTile tl = tiles[blockIdx.x];
-  const uint32_t g = blockIdx.y, qh0 = g * HPW, nkv = nh / HPW, kvh = g;
-  const uint32_t t = threadIdx.x, wv = t >> 6, lane = t & 63;
-  const uint32_t npair = tl.nr * HPW, len_max = tl.p0 + tl.nr;
-  float* S = scratch + ((size_t)blockIdx.x * nkv + g) * P * ls;  // [P][ls] scores, then exps
-  const size_t sb = (size_t)tl.seq * seq_stride + (size_t)kvh * HD * max_pos;
-  const float* kb = kc + sb;
-  const float* vb = vc + sb;
-  auto pair_len = [=](uint32_t a) { return tl.p0 + a / HPW + 1; };
-  // q of every pair (rows past nr: zero, never stored)
-  for (uint32_t i = t; i < P * HD; i += 256) {
-    const uint32_t a = i / HD, d = i - a * HD, ri = a / HPW, h = a - ri * HPW;
-    qs[a * QS + d] = a < npair ? q[(size_t)(tl.row0 + ri) * nh * HD + (size_t)(qh0 + h) * HD + d]
-                               : 0.0f;
-  }
-  // ---- scores ------------------------------------------------------------
-  constexpr uint32_t TPR = TK / 4;  // threads per pair group (4 positions each)
-  const uint32_t pg = t / TPR, jg = t - pg * TPR;
-  Pick best[PB];
-  bool nan0[PB];
+  const uint32_t nhb = nh / HPT, G = gridDim.x;
+  float* S = scratch + (size_t)blockIdx.x * P * ls;  // [P][ls] scores, then exps
+  for (uint32_t round = 0; (uint64_t)round * G < nitem; ++round) {
+    // the thread id through an opaque copy: its many derived values are
+    // formed where they are used, not kept in registers across the items
+    uint32_t t = threadIdx.x;
+    asm volatile("" : "+v"(t));
+    const uint32_t wv = __builtin_amdgcn_readfirstlane(t >> 6);
+    uint32_t lane = t & 63, u = lane >> 4, c16 = lane & 15;
+    const f16v nz = minus_zeros();
+    // odd rounds in reverse, by runs of 8 (a workgroup keeps its head's XCD)
+    const uint32_t b = round & 1 ? G - 8 - (blockIdx.x & ~7u) + (blockIdx.x & 7) : blockIdx.x;
+    const uint64_t w64 = (uint64_t)round * G + b;
+    if (w64 >= nitem) continue;  // the same for the whole workgroup
+    const uint32_t w = (uint32_t)w64, ti = w / nhb, qh0 = (w - ti * nhb) * HPT;
+    const AttTile tl = tiles[ti];
+    const uint32_t kvh = qh0 / group, len_max = tl.p0 + tl.nr, len_min = tl.p0 + 1;
+    const size_t sb = (size_t)tl.seq * seq_stride + (size_t)kvh * HD * max_pos;
+    const float* kb = kc + sb;
+    const float* vb = vc + sb;
+    const float* q0 = q + ((size_t)tl.row0 * nh + qh0) * HD;
+    auto pair_len = [=](uint32_t a) { return tl.p0 + a % kAttQT + 1; };
+    auto live = [=](uint32_t a) { return a % kAttQT < tl.nr; };
+    __syncthreads();  // the item before this one is done with the LDS
+    // q of every pair in operand order (rows past nr: zero, never stored)
+    for (uint32_t i = t; i < P * DG; i += 256) {
+      const uint32_t a = i % P, g = i / P;
+      const v4* src = reinterpret_cast<const v4*>(
+          q0 + (a % kAttQT * nh + a / kAttQT) * HD + 16 * g);
+      v4 x[4];
 #pragma unroll
-  for (uint32_t u = 0; u < PB; ++u) {
-    best[u] = Pick{0.0f, UINT32_MAX};
-    nan0[u] = false;
-  }
-  const uint32_t nkt = (len_max + TK - 1) / TK;
-  float* kt0 = reg;
-  auto kt = [=](uint32_t i) { return kt0 + (size_t)(i & 1) * HD * TK; };
-  auto copy_k = [=](uint32_t i) {
-    const uint32_t j0 = i * TK, n = min(TK, len_max - j0);
-    // rows of TK floats back to back: a wave instruction covers 64 / (TK/4) rows
-    const uint32_t n4 = (n + 3) >> 2, rows_per = 64 / (TK / 4);
-    float* dst = kt(i);
-    for (uint32_t r0 = wv * rows_per; r0 < HD; r0 += 4 * rows_per) {
-      const uint32_t r = r0 + lane / (TK / 4), qq = lane % (TK / 4);
-      if (r < HD && qq < n4)
-        lds_load16(reinterpret_cast<const v4*>(kb + (size_t)r * max_pos + j0) + qq,
-                   reinterpret_cast<v4*>(dst + (size_t)r0 * TK));
+      for (uint32_t m = 0; m < 4; ++m) x[m] = live(a) ? src[m] : v4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (uint32_t e = 0; e < 4; ++e)
+        qf[(4 * g + e) * P + a] = v4{x[0][e], x[1][e], x[2][e], x[3][e]};
     }
-  };
-  copy_k(0);
-  for (uint32_t i = 0; i < nkt; ++i) {
-    wait_vm0();
     __syncthreads();
-    if (i + 1 < nkt) copy_k(i + 1);
-    const float* k = kt(i);
-    float acc[PB][4];
+    // ---- scores ------------------------------------------------------------
+    float best[HPT][4];
 #pragma unroll
-    for (uint32_t u = 0; u < PB; ++u)
+    for (uint32_t h = 0; h < HPT; ++h)
 #pragma unroll
-      for (uint32_t v = 0; v < 4; ++v) acc[u][v] = 0.0f;
-#pragma unroll 2
-    for (uint32_t d4 = 0; d4 < HD; d4 += 4) {
-      v4 qv[PB], kk[4];
+      for (uint32_t r = 0; r < 4; ++r) best[h][r] = -__builtin_inff();
+#pragma unroll 1
+    for (uint32_t j0 = 64 * wv; j0 < len_max; j0 += 256) {
+      // columns past the cache's end are clamped; scores past a row's length
+      // are never used
+      const uint32_t ko = u * max_pos + min(j0 + 4 * c16, max_pos - 4);
+      auto kload = [&](uint32_t d4) {  // rows 4 d4 .. 4 d4 + 3 of K
+        return *reinterpret_cast<const v4*>(kb + (size_t)(4 * d4) * max_pos + ko);
+      };
+      float acc[NT1][4];
 #pragma unroll
-      for (uint32_t u = 0; u < PB; ++u)
-        qv[u] = *reinterpret_cast<const v4*>(qs + (size_t)(pg * PB + u) * QS + d4);
+      for (uint32_t s = 0; s < NT1; ++s)
 #pragma unroll
-      for (uint32_t e = 0; e < 4; ++e)
-        kk[e] = *reinterpret_cast<const v4*>(k + (size_t)(d4 + e) * TK + 4 * jg);
+        for (uint32_t r = 0; r < 4; ++r) acc[s][r] = 0.0f;
+      auto add = [&](uint32_t s, const f16v& p) {
 #pragma unroll
-      for (uint32_t e = 0; e < 4; ++e)
+        for (uint32_t e = 0; e < 4; ++e)
 #pragma unroll
-        for (uint32_t u = 0; u < PB; ++u) {
-          float p;
-          p = qv[u][e] * kk[e].x; acc[u][0] = acc[u][0] + p;
-          p = qv[u][e] * kk[e].y; acc[u][1] = acc[u][1] + p;
-          p = qv[u][e] * kk[e].z; acc[u][2] = acc[u][2] + p;
-          p = qv[u][e] * kk[e].w; acc[u][3] = acc[u][3] + p;
+          for (uint32_t r = 0; r < 4; ++r) acc[s][r] = acc[s][r] + p[4 * e + r];
+        asm volatile("" : "+v"(acc[s][0]), "+v"(acc[s][1]), "+v"(acc[s][2]), "+v"(acc[s][3]));
+      };
+      f16v d[2];
+      d[1] = nz;
+      v4 kf[2][4];
+#pragma unroll
+      for (uint32_t m = 0; m < 4; ++m) kf[0][m] = kload(m);
+      auto dgroup = [&](uint32_t g, const v4 (&cur)[4], v4 (&nxt)[4]) {
+        if (g + 1 < DG) {
+#pragma unroll
+          for (uint32_t m = 0; m < 4; ++m) nxt[m] = kload(4 * (g + 1) + m);
+        }
+        v4 fa[HPT];
+#pragma unroll
+        for (uint32_t h = 0; h < HPT; ++h) fa[h] = qf[(4 * g + u) * P + 16 * h + c16];
+#pragma unroll
+        for (uint32_t m = 0; m < 4; ++m)
+#pragma unroll
+          for (uint32_t s = 0; s < NT1; ++s) {
+            const uint32_t x = m * NT1 + s;
+            d[x & 1] = products4(fa[s / 4][m], cur[m][s % 4], nz);
+            asm volatile("" : "+v"(d[x & 1]));
+            add((s + NT1 - 1) % NT1, d[(x + 1) & 1]);
+          }
+      };
+#pragma unroll 1
+      for (uint32_t g = 0; g < DG; g += 2) {
+        dgroup(g, kf[0], kf[1]);
+        dgroup(g + 1, kf[1], kf[0]);
+      }
+      add(NT1 - 1, d[1]);
+      const uint32_t j = j0 + 4 * c16;
+#pragma unroll
+      for (uint32_t h = 0; h < HPT; ++h)
+#pragma unroll
+        for (uint32_t r = 0; r < 4; ++r) {
+          const uint32_t i = 4 * u + r, len = len_min + i;
+          v4 sv;
+#pragma unroll
+          for (uint32_t c = 0; c < 4; ++c) {
+            sv[c] = acc[4 * h + c][r] * scale;
+            best[h][r] = (j + c < len && sv[c] > best[h][r]) ? sv[c] : best[h][r];
+          }
+          if (i < tl.nr && j < ls)
+            *reinterpret_cast<v4*>(S + (size_t)(16 * h + r) * ls + (4 * u * ls + j)) = sv;
         }
     }
 #pragma unroll
-    for (uint32_t u = 0; u < PB; ++u) {
-      const uint32_t a = pg * PB + u;
-      if (a < npair) {
-        const uint32_t len = pair_len(a);
+    for (uint32_t h = 0; h < HPT; ++h)
 #pragma unroll
-        for (uint32_t v = 0; v < 4; ++v) {
-          const uint32_t j = i * TK + 4 * jg + v;
-          if (j < len) {
-            const float s = acc[u][v] * scale;
-            S[(size_t)a * ls + j] = s;
-            if (s == s) best[u] = pick2(best[u], Pick{s, j});
-            else if (j == 0) nan0[u] = true;
+      for (uint32_t r = 0; r < 4; ++r) {
+        float m = best[h][r];
+#pragma unroll
+        for (uint32_t off = 1; off < 16; off <<= 1) {
+          const float o = __shfl_xor(m, off, 64);
+          m = o > m ? o : m;
+        }
+        if (c16 == 0) wmx[wv * P + 16 * h + 4 * u + r] = m;
+      }
+    // ---- softmax denominators ---------------------------------------------
+    asm volatile("" : "+v"(t));
+    lane = t & 63, u = lane >> 4, c16 = lane & 15;
+    // the scores are stored before they are read back; writer and reader
+    // waves share the CU and its cache, so the workgroup's scope is enough
+    // (an agent-scope fence writes the XCD's L2 back: 5 x the time of a
+    // short tile)
+    __threadfence_block();
+    __syncthreads();
+    // the largest non-NaN score; a NaN at position 0 wins with its own bits
+    if (t < P && live(t)) {
+      float m = wmx[t];
+#pragma unroll
+      for (uint32_t w4 = 1; w4 < 4; ++w4) m = wmx[w4 * P + t] > m ? wmx[w4 * P + t] : m;
+      const float s0 = S[t * ls];
+      smx[t] = s0 != s0 ? s0 : m;
+    }
+    const uint32_t nst = (len_max + kAttTE - 1) / kAttTE;
+    auto es = [=](uint32_t i) { return reg + (i & 1) * P * ES; };
+    // waves 1..3: copy stage i of the pairs' scores and exponentiate it in
+    // place, four pair rows per wave instruction, each wave on the rows it
+    // copied
+    auto stage = [=](uint32_t i) {
+      const uint32_t j0 = i * kAttTE, j = j0 + 4 * c16;
+      float* st = es(i);
+      for (uint32_t a = 4 * (wv - 1) + u; a < P; a += 12) {
+        const uint32_t len = pair_len(a);
+        if (!live(a) || j >= len) continue;
+        v4* sp = reinterpret_cast<v4*>(S + (a * ls + j));
+        const float mx = smx[a];
+        v4 e = *sp;
+#pragma unroll
+        for (uint32_t c = 0; c < 4; ++c) {
+          const float dlt = e[c] - mx;
+          e[c] = exp_pinned(dlt);
+        }
+        *reinterpret_cast<v4*>(st + (a * ES + 4 * c16)) = e;
+        *sp = e;
+      }
+    };
+    __syncthreads();
+    if (wv >= 1) stage(0);
+    __syncthreads();
+    float den = 0.0f;
+    for (uint32_t i = 0; i < nst; ++i) {
+      // lanes a < P of wave 0 chain stage i; waves 1..3 prepare stage i+1 in
+      // the other buffer (its stage i-1 was chained before this barrier)
+      if (wv == 0) {
+        if (lane < P && live(lane)) {
+          const uint32_t j0 = i * kAttTE, len = pair_len(lane);
+          if (j0 < len) den = chain_lds(es(i) + lane * ES, min(kAttTE, len - j0), den);
+        }
+      } else if (i + 1 < nst) {
+        stage(i + 1);
+      }
+      __syncthreads();
+    }
+    if (wv == 0 && lane < P) sden[lane] = den;
+    __threadfence_block();  // the exps are stored before they are read back
+    __syncthreads();
+    // ---- V-mix --------------------------------------------------------------
+    asm volatile("" : "+v"(t));
+    lane = t & 63, u = lane >> 4, c16 = lane & 15;
+    // p tile T of TP positions: this thread's piece is 16 positions of a pair
+    const uint32_t pa = t % P, pg = t / P;
+    const bool mine = t < P * TP / 16;
+    v4* pf0 = reinterpret_cast<v4*>(reg);  // 2 x [TP / 16][4][P]
+    v4 ev[4];
+    auto load_e = [&](uint32_t T) {
+      if (mine) {
+#pragma unroll
+        for (uint32_t m = 0; m < 4; ++m)
+          ev[m] = *reinterpret_cast<const v4*>(S + (pa * ls + min(T * TP + 16 * pg + 4 * m, ls - 4)));
+      }
+    };
+    auto store_p = [&](uint32_t T) {
+      if (mine) {
+        const float dn = sden[pa];
+#pragma unroll
+        for (uint32_t m = 0; m < 4; ++m)
+#pragma unroll
+          for (uint32_t e = 0; e < 4; ++e) ev[m][e] = ev[m][e] / dn;
+        v4* pf = pf0 + (T & 1) * (P * TP / 4);
+#pragma unroll
+        for (uint32_t e = 0; e < 4; ++e)
+          pf[(4 * pg + e) * P + pa] = v4{ev[0][e], ev[1][e], ev[2][e], ev[3][e]};
+      }
+    };
+    float acc[NT3][4];
+#pragma unroll
+    for (uint32_t s = 0; s < NT3; ++s)
+#pragma unroll
+      for (uint32_t r = 0; r < 4; ++r) acc[s][r] = 0.0f;
+    auto add = [&](uint32_t s, const f16v& p) {
+#pragma unroll
+      for (uint32_t e = 0; e < 4; ++e)
+#pragma unroll
+        for (uint32_t r = 0; r < 4; ++r) acc[s][r] = acc[s][r] + p[4 * e + r];
+      asm volatile("" : "+v"(acc[s][0]), "+v"(acc[s][1]), "+v"(acc[s][2]), "+v"(acc[s][3]));
+    };
+    // V of 16-position group gi: lane (dim c16 of a 16-dim tile, u) loads
+    // positions 4u .. 4u+3
+    v4 vr[4][NB];
+    auto load_v = [&](uint32_t gi, v4 (&v)[NB]) {
+      const uint32_t col = min(16 * gi + 4 * u, max_pos - 4);
+#pragma unroll
+      for (uint32_t x = 0; x < NB; ++x)
+        v[x] = *reinterpret_cast<const v4*>(vb + (size_t)(16 * (wv * NB + x)) * max_pos +
+                                            (c16 * max_pos + col));
+    };
+    const uint32_t ngr = (len_max + 15) / 16, ntile = (len_max + TP - 1) / TP;
+#pragma unroll
+    for (uint32_t g = 0; g < 4; ++g)
+      if (g < ngr) load_v(g, vr[g]);
+    f16v d[2];
+    d[1] = nz;
+    load_e(0);
+    store_p(0);
+#pragma unroll 1
+    for (uint32_t T = 0; T < ntile; ++T) {
+      __syncthreads();
+      if (T + 1 < ntile) load_e(T + 1);
+      const v4* pf = pf0 + (T & 1) * (P * TP / 4);
+#pragma unroll 1
+      for (uint32_t g4 = 0; g4 < TP / 16; g4 += 4) {
+#pragma unroll
+        for (uint32_t gg = 0; gg < 4; ++gg) {
+          const uint32_t gl = g4 + gg, gi = T * (TP / 16) + gl;
+          if (gi >= ngr) break;
+          v4 fb[NB], fa[HPT];
+#pragma unroll
+          for (uint32_t x = 0; x < NB; ++x) {
+            fb[x] = vr[gg][x];
+            transpose4(fb[x]);
+          }
+          if (gi + 4 < ngr) load_v(gi + 4, vr[gg]);
+#pragma unroll
+          for (uint32_t h = 0; h < HPT; ++h) fa[h] = pf[(4 * gl + u) * P + 16 * h + c16];
+          if (16 * gi + 16 <= len_min) {
+#pragma unroll
+            for (uint32_t m = 0; m < 4; ++m)
+#pragma unroll
+              for (uint32_t s = 0; s < NT3; ++s) {
+                const uint32_t x = m * NT3 + s;
+                d[x & 1] = products4(fa[s / NB][m], fb[s % NB][m], nz);
+                asm volatile("" : "+v"(d[x & 1]));
+                add((s + NT3 - 1) % NT3, d[(x + 1) & 1]);
+              }
+          } else {
+            // the pending tile's adds, then adds of j < the row's length only
+            add(NT3 - 1, d[1]);
+            d[1] = nz;
+#pragma unroll
+            for (uint32_t m = 0; m < 4; ++m)
+#pragma unroll
+              for (uint32_t s = 0; s < NT3; ++s) {
+                f16v p = products4(fa[s / NB][m], fb[s % NB][m], nz);
+                asm volatile("" : "+v"(p));
+#pragma unroll
+                for (uint32_t e = 0; e < 4; ++e)
+#pragma unroll
+                  for (uint32_t r = 0; r < 4; ++r) {
+                    const float y = acc[s][r] + p[4 * e + r];
+                    acc[s][r] = 16 * gi + 4 * m + e < len_min + 4 * u + r ? y : acc[s][r];
+                  }
+                asm volatile("" : "+v"(acc[s][0]), "+v"(acc[s][1]), "+v"(acc[s][2]), "+v"(acc[s][3]));
+              }
           }
         }
       }
+      if (T + 1 < ntile) store_p(T + 1);
     }
-  }
-  // maxima: the TPR threads of a pair group are consecutive lanes of one wave
+    add(NT3 - 1, d[1]);
+    float* o0 = out + ((size_t)tl.row0 * nh + qh0) * HD;
 #pragma unroll
-  for (uint32_t u = 0; u < PB; ++u) {
-    Pick b = best[u];
-    uint32_t n0 = nan0[u] ? 1u : 0u;
-    for (uint32_t off = TPR / 2; off > 0; off >>= 1) {
-      Pick o;
-      o.v = __shfl_xor(b.v, off, 64);
-      o.i = __shfl_xor(b.i, off, 64);
-      b = pick2(b, o);
-      n0 |= __shfl_xor(n0, off, 64);
-    }
-    const uint32_t a = pg * PB + u;
-    if (jg == 0 && a < P) smx[a] = n0 ? __builtin_nanf("") : b.v;
-  }
-  // ---- softmax denominators ---------------------------------------------
-  // the scores reach global memory, and no stale copy stays in this CU's
-  // cache, before they are read back (agent-scope fence: release + acquire)
-  __threadfence();
-  __syncthreads();
-  // a NaN at position 0 wins with its own bits: re-read the score
-  if (t < npair && smx[t] != smx[t]) smx[t] = S[(size_t)t * ls];
-  const uint32_t nst = (len_max + kAttTE - 1) / kAttTE;
-  float* es0 = reg;
-  auto es = [=](uint32_t i) { return es0 + (size_t)(i & 1) * P * ES; };
-  // waves 1..3: copy stage i of every pair's scores and exponentiate it in
-  // place, each wave on the pair rows it copied
-  auto load_stage = [=](uint32_t i) {
-    const uint32_t j0 = i * kAttTE, n = min(kAttTE, len_max - j0);
-    copy_rows_lds(es(i), ES, S + j0, ls, npair, n, 1, 3);
-  };
-  auto exp_stage = [=](uint32_t i) {
-    const uint32_t j0 = i * kAttTE;
-    float* st = es(i);
-    for (uint32_t a = wv - 1; a < npair; a += 3) {
-      const uint32_t len = pair_len(a);
-      if (j0 >= len) continue;
-      const uint32_t n = min(kAttTE, len - j0);
-      const float mx = smx[a];
-      for (uint32_t j = lane; j < n; j += 64) {
-        const float dlt = st[(size_t)a * ES + j] - mx;
-        const float e = exp_pinned(dlt);
-        st[(size_t)a * ES + j] = e;
-        S[(size_t)a * ls + j0 + j] = e;
+    for (uint32_t s = 0; s < NT3; ++s)
+#pragma unroll
+      for (uint32_t r = 0; r < 4; ++r) {
+        const uint32_t i = 4 * u + r, h = s / NB, dd = 16 * (wv * NB + s % NB) + c16;
+        if (i < tl.nr) o0[(i * nh + h) * HD + dd] = acc[s][r];
       }
-    }
-  };
-  __syncthreads();
-  if (wv >= 1) {
-    load_stage(0);
-    wait_vm0();
-    exp_stage(0);
-  }
-  __syncthreads();
-  float den = 0.0f;
-  for (uint32_t i = 0; i < nst; ++i) {
-    // lanes a < npair of wave 0 chain stage i; waves 1..3 prepare stage i+1
-    // in the other buffer (its stage i-1 was chained before this barrier)
-    if (wv == 0) {
-      if (lane < npair) {
-        const uint32_t j0 = i * kAttTE, len = pair_len(lane);
-        if (j0 < len) den = chain_lds(es(i) + (size_t)lane * ES, min(kAttTE, len - j0), den);
-      }
-    } else if (i + 1 < nst) {
-      load_stage(i + 1);
-      wait_vm0();
-      exp_stage(i + 1);
-    }
-    __syncthreads();
-  }
-  if (wv == 0 && lane < npair) sden[lane] = den;
-  // the exps written by waves 1..3 reach global memory before the V-mix
-  // reads them back through the async copies
-  __threadfence();
-  __syncthreads();
-  // ---- V-mix --------------------------------------------------------------
-  const uint32_t dg = t % (HD / 4), pg3 = t / (HD / 4);
-  float* vt0 = reg;                                // 2 x [HD][VS]
-  float* et0 = reg + 2 * (size_t)HD * VS;          // 2 x [P][VS]
-  auto vt = [=](uint32_t i) { return vt0 + (size_t)(i & 1) * HD * VS; };
-  auto et = [=](uint32_t i) { return et0 + (size_t)(i & 1) * P * VS; };
-  auto copy_ve = [=](uint32_t i) {
-    const uint32_t j0 = i * TK, n = min(TK, len_max - j0);
-    copy_rows_lds(vt(i), VS, vb + j0, max_pos, HD, n, 0, 4);
-    copy_rows_lds(et(i), VS, S + j0, ls, npair, n, 0, 4);
-  };
-  float acc3[PB3][4];
-#pragma unroll
-  for (uint32_t u = 0; u < PB3; ++u)
-#pragma unroll
-    for (uint32_t v = 0; v < 4; ++v) acc3[u][v] = 0.0f;
-  copy_ve(0);
-  for (uint32_t i = 0; i < nkt; ++i) {
-    wait_vm0();
-    __syncthreads();
-    // p_j = e_j / den in place (main.rs softmax: true divide)
-    {
-      const uint32_t j0 = i * TK;
-      float* e = et(i);
-      for (uint32_t x = t; x < npair * TK; x += 256) {
-        const uint32_t a = x / TK, j = x - a * TK;
-        if (j0 + j < pair_len(a)) {
-          const float pj = e[(size_t)a * VS + j] / sden[a];
-          e[(size_t)a * VS + j] = pj;
-        }
-      }
-    }
-    __syncthreads();
-    if (i + 1 < nkt) copy_ve(i + 1);
-    const float* v = vt(i);
-    const float* e = et(i);
-    const uint32_t j0 = i * TK, n = min(TK, len_max - j0);
-    // positions of this tile each of the thread's pairs sees; the common
-    // 4-aligned part reads each V group once for all the pairs
-    uint32_t m[PB3], mall = n;
-#pragma unroll
-    for (uint32_t u = 0; u < PB3; ++u) {
-      const uint32_t a = pg3 * PB3 + u;
-      const uint32_t len = a < npair ? pair_len(a) : 0;
-      m[u] = len > j0 ? min(n, len - j0) : 0;
-      mall = min(mall, m[u]);
-    }
-    const uint32_t m4 = mall & ~3u;
-#pragma unroll 2
-    for (uint32_t j = 0; j < m4; j += 4) {
-      v4 vv[4];
-#pragma unroll
-      for (uint32_t dd = 0; dd < 4; ++dd)
-        vv[dd] = *reinterpret_cast<const v4*>(v + (size_t)(4 * dg + dd) * VS + j);
-#pragma unroll
-      for (uint32_t u = 0; u < PB3; ++u) {
-        const v4 pp = *reinterpret_cast<const v4*>(e + (size_t)(pg3 * PB3 + u) * VS + j);
-#pragma unroll
-        for (uint32_t dd = 0; dd < 4; ++dd) {
-          float p;
-          p = pp.x * vv[dd].x; acc3[u][dd] = acc3[u][dd] + p;
-          p = pp.y * vv[dd].y; acc3[u][dd] = acc3[u][dd] + p;
-          p = pp.z * vv[dd].z; acc3[u][dd] = acc3[u][dd] + p;
-          p = pp.w * vv[dd].w; acc3[u][dd] = acc3[u][dd] + p;
-        }
-      }
-    }
-#pragma unroll
-    for (uint32_t u = 0; u < PB3; ++u) {
-      const float* pr = e + (size_t)(pg3 * PB3 + u) * VS;
-      for (uint32_t j = m4; j < m[u]; ++j) {
-#pragma unroll
-        for (uint32_t dd = 0; dd < 4; ++dd) {
-          const float p = pr[j] * v[(size_t)(4 * dg + dd) * VS + j];
-          acc3[u][dd] = acc3[u][dd] + p;
-        }
-      }
-    }
-  }
-#pragma unroll
-  for (uint32_t u = 0; u < PB3; ++u) {
-    const uint32_t a = pg3 * PB3 + u;
-    if (a < npair) {
-      const uint32_t ri = a / HPW, h = a - ri * HPW;
-      float* o = out + (size_t)(tl.row0 + ri) * nh * HD + (size_t)(qh0 + h) * HD + 4 * dg;
-#pragma unroll
-      for (uint32_t dd = 0; dd < 4; ++dd) o[dd] = acc3[u][dd];
-    }
   }
 }
 
@@ -2348,32 +2405,48 @@ hipError_t launch_argmax_rows(const float* v, uint32_t n, uint32_t width, uint32
 }
 
 
-template <uint32_t HPW, uint32_t HD, uint32_t TK>
+// Workgroups of k_attention_tiles: two per CU (its registers), a multiple of
+// eight, no more than the items need.
+static uint32_t att_tiles_grid(uint64_t nitem) {
+  const uint64_t most = (2 * (uint64_t)device_cu_count() + 7) / 8 * 8;
+  return (uint32_t)std::min<uint64_t>(most, (nitem + 7) / 8 * 8);
+}
+// Query heads per item: those of one KV head share its K and V loads where
+// that leaves enough items for two workgroups per CU, else one.  At head_dim
+// 128 up to three (four spilled registers).
+static uint32_t att_tiles_heads(uint32_t ntiles, uint32_t nh, uint32_t nkv, uint32_t hd) {
+  const uint32_t group = nh / nkv, ncu = (uint32_t)device_cu_count();
+  for (uint32_t h = std::min(group, hd == 64 ? 4u : 3u); h > 1; --h)
+    if (group % h == 0 && (uint64_t)ntiles * (nh / h) >= 2 * (uint64_t)ncu) return h;
+  return 1;
+}
+
+template <uint32_t HPT, uint32_t HD>
 static hipError_t launch_att_tiles_t(const float* q, const float* kc, const float* vc,
                                      const AttTile* tiles, uint32_t ntiles, uint32_t nh,
-                                     uint32_t max_pos, uint64_t seq_stride, float scale, float* out,
-                                     float* scratch, uint32_t ls, hipStream_t st) {
-  using C = AttTileCfg<HPW, HD, TK>;
-  const size_t lds = C::floats * sizeof(float);
-  hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void*>(&k_attention_tiles<HPW, HD, TK>), lds);
+                                     uint32_t group, uint32_t max_pos, uint64_t seq_stride,
+                                     float scale, float* out, float* scratch, uint32_t ls,
+                                     hipStream_t st) {
+  const size_t lds = AttTileCfg<HPT>::floats(HD) * sizeof(float);
+  hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void*>(&k_attention_tiles<HPT, HD>), lds);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL((k_attention_tiles<HPW, HD, TK>), dim3(ntiles, nh / HPW), dim3(256), lds, st,
-                     q, kc, vc, tiles, nh, max_pos, seq_stride, scale, out, scratch, ls);
+  const uint64_t nitem = (uint64_t)ntiles * (nh / HPT);
+  if (nitem > 0x7fffffffu) return hipErrorInvalidValue;
+  hipLaunchKernelGGL((k_attention_tiles<HPT, HD>), dim3(att_tiles_grid(nitem)), dim3(256), lds, st,
+                     q, kc, vc, tiles, (uint32_t)nitem, nh, group, max_pos, seq_stride, scale, out,
+                     scratch, ls);
   return hipGetLastError();
 }
 
 bool attention_tiles_supported(uint32_t nh, uint32_t nkv, uint32_t hd) {
-  if (nkv == 0 || nh % nkv) return false;
-  const uint32_t g = nh / nkv;
-  if (hd == 64) return g >= 1 && g <= 4;
-  if (hd == 128) return g == 2 || g == 4;
-  return false;
+  return nkv != 0 && nh % nkv == 0 && (hd == 64 || hd == 128);
 }
 
-size_t attention_tiles_scratch_floats(uint32_t ntiles, uint32_t nh, uint32_t nkv,
+size_t attention_tiles_scratch_floats(uint32_t ntiles, uint32_t nh, uint32_t nkv, uint32_t hd,
                                       uint32_t max_len) {
   const size_t ls = ((size_t)max_len + 3) / 4 * 4;
-  return (size_t)ntiles * nkv * kAttQT * (nh / nkv) * ls;
+  const uint32_t h = att_tiles_heads(ntiles, nh, nkv, hd);
+  return (size_t)att_tiles_grid((uint64_t)ntiles * (nh / h)) * kAttQT * h * ls;
 }
 
 hipError_t launch_attention_tiles(const float* q, const float* kc, const float* vc,
@@ -2386,16 +2459,20 @@ hipError_t launch_attention_tiles(const float* q, const float* kc, const float* 
       max_pos % 4)
     return hipErrorInvalidValue;
   const uint32_t g = nh / nkv, ls = (max_len + 3) / 4 * 4;
-  if (hd == 64) {
-    switch (g) {
-      case 1: return launch_att_tiles_t<1, 64, 64>(q, kc, vc, tiles, ntiles, nh, max_pos, seq_stride, scale, out, scratch, ls, st);
-      case 2: return launch_att_tiles_t<2, 64, 64>(q, kc, vc, tiles, ntiles, nh, max_pos, seq_stride, scale, out, scratch, ls, st);
-      case 3: return launch_att_tiles_t<3, 64, 64>(q, kc, vc, tiles, ntiles, nh, max_pos, seq_stride, scale, out, scratch, ls, st);
-      default: return launch_att_tiles_t<4, 64, 64>(q, kc, vc, tiles, ntiles, nh, max_pos, seq_stride, scale, out, scratch, ls, st);
-    }
+#define CIS2_ATT_TILES(H, D)                                                                     \
+  return launch_att_tiles_t<H, D>(q, kc, vc, tiles, ntiles, nh, g, max_pos, seq_stride, scale,   \
+                                  out, scratch, ls, st)
+  switch (att_tiles_heads(ntiles, nh, nkv, hd) * 1000 + hd) {
+    case 1064: CIS2_ATT_TILES(1, 64);
+    case 2064: CIS2_ATT_TILES(2, 64);
+    case 3064: CIS2_ATT_TILES(3, 64);
+    case 4064: CIS2_ATT_TILES(4, 64);
+    case 1128: CIS2_ATT_TILES(1, 128);
+    case 2128: CIS2_ATT_TILES(2, 128);
+    case 3128: CIS2_ATT_TILES(3, 128);
+    default: return hipErrorInvalidValue;
   }
-  if (g == 2) return launch_att_tiles_t<2, 128, 32>(q, kc, vc, tiles, ntiles, nh, max_pos, seq_stride, scale, out, scratch, ls, st);
-  return launch_att_tiles_t<4, 128, 32>(q, kc, vc, tiles, ntiles, nh, max_pos, seq_stride, scale, out, scratch, ls, st);
+#undef CIS2_ATT_TILES
 }
 
 }  // namespace cis2

@@ -85,15 +85,17 @@ hipError_t launch_rope_attention_rows(const float* q, const float* k, const floa
 // Prefill attention in tiles: rows row0 .. row0+nr-1 (nr <= 16) are rows of
 // sequence seq at positions p0 .. p0+nr-1; each tile's rows get the same
 // bits as launch_attention_rows gives them (sequential order only), with
-// each K and V element read once per tile and KV head.  Shapes: head_dim
-// 64 with 1..4 query heads per KV head, head_dim 128 with 2 or 4.
-// scratch: attention_tiles_scratch_floats(ntiles, nh, nkv, max_len) floats.
+// each K and V element read once per tile and up to four query heads.
+// Shapes: head_dim 64 or 128.  The longest tiles should come first (the
+// workgroups take them in order).
+// scratch: attention_tiles_scratch_floats(ntiles, nh, nkv, hd, max_len)
+// floats.
 struct AttTile {
   uint32_t row0, nr, seq, p0;
 };
 constexpr uint32_t kAttTileRows = 16;
 bool attention_tiles_supported(uint32_t nh, uint32_t nkv, uint32_t hd);
-size_t attention_tiles_scratch_floats(uint32_t ntiles, uint32_t nh, uint32_t nkv,
+size_t attention_tiles_scratch_floats(uint32_t ntiles, uint32_t nh, uint32_t nkv, uint32_t hd,
                                       uint32_t max_len);
 hipError_t launch_attention_tiles(const float* q, const float* kc, const float* vc,
                                   const AttTile* tiles, uint32_t ntiles, uint32_t max_len,

@@ -655,7 +655,12 @@ int plan_tiles(cis2_ctx* c, uint32_t n, const uint32_t* seq, const uint32_t* pos
   if (off || f.reduction_mode != 0 ||
       !attention_tiles_supported(f.n_heads, f.n_kv_heads, f.head_dim))
     return CIS2_OK;
-  if (!force && (uint64_t)n * f.n_kv_heads < 4 * (uint64_t)c->ncu) return CIS2_OK;
+  // Where the lines lie (us per layer, per-row kernels | tiles): one prompt,
+  // 9 heads of 64: 64 rows 87 | 93, 100 rows 114 | 115, 200 rows 161 | 157,
+  // 544 rows 242 | 204; 16 heads of 128: 64 rows 233 | 235, 100 rows 337 |
+  // 326.  64 runs at position 200: of 4 rows 193 | 200 and 656 | 612, of 6
+  // rows 195 | 186 and 583 | 496.
+  if (!force && (uint64_t)n * f.n_heads < 4 * (uint64_t)c->ncu) return CIS2_OK;
   b.htiles.clear();
   for (uint32_t i = 0; i < n;) {
     uint32_t k = 1;
@@ -664,9 +669,12 @@ int plan_tiles(cis2_ctx* c, uint32_t n, const uint32_t* seq, const uint32_t* pos
     i += k;
   }
   const uint32_t nt = (uint32_t)b.htiles.size();
-  // short runs, or too few tile workgroups to fill the GPU: per-row attention
-  if (!force && ((uint64_t)nt * 8 > n || (uint64_t)nt * f.n_kv_heads < c->ncu)) return CIS2_OK;
-  const size_t scr = attention_tiles_scratch_floats(nt, f.n_heads, f.n_kv_heads, max_len);
+  if (!force && (uint64_t)nt * 5 > n) return CIS2_OK;  // short runs
+  const size_t scr = attention_tiles_scratch_floats(nt, f.n_heads, f.n_kv_heads, f.head_dim, max_len);
+  // the longest first: the workgroups take the tiles in order
+  std::stable_sort(b.htiles.begin(), b.htiles.end(), [](const AttTile& x, const AttTile& y) {
+    return x.p0 + x.nr > y.p0 + y.nr;
+  });
   if (nt > b.tcap || scr > b.acap) {
     HIPCHK(c, hipStreamSynchronize(c->st), "tiles sync");
     for (void* p : b.tmem) (void)hipFree(p);

@@ -1,8 +1,13 @@
-"""The row-batched GEMMs whose products come from the matrix cores
-(k_mgemm): sizes that are no multiple of any tile in rows, outputs or K,
-weights with signed zeros and products that flush to zero.  Every row must
-have the bits of the vector-unit kernel (CIS2_BGEMM16=0) and of the oracle;
-the arithmetic is pinned, so there is no tolerance."""
+"""The row-batched kernels whose products come from the matrix cores.
+
+GEMMs (k_mgemm): sizes that are no multiple of any tile in rows, outputs or
+K, weights with signed zeros and products that flush to zero; against the
+vector-unit kernel (CIS2_BGEMM16=0) and the oracle.  Prefill attention
+(k_attention_tiles): every number of heads per item, runs that end inside a
+tile, lengths around the 16-, 64- and 256-position steps, a cache end inside
+a 16-position group, V rows with infinities and NaN past a row's own
+position; against the per-row kernel (CIS2_ATT_TILES=0) and the oracle.  The
+arithmetic is pinned, so there is no tolerance."""
 import os
 
 import numpy as np
@@ -63,3 +68,73 @@ def test_rows_matrix_core_gemm_bits(spec, n, per_seq):
         for p in range(min(per_seq, n - s * per_seq)):
             want = o.forward(p, int(tok[s * per_seq + p])).view(np.uint32)
             assert np.array_equal(want, lg[s * per_seq + p]), (s, p)
+
+
+def heads_spec(nh, nkv, hd):
+    return artifacts.ModelSpec("h%d-%d-%d" % (nh, nkv, hd), 64, 64, 1, nh, nkv, 67, 1e-6, 10000.0,
+                               True, head_dim=hd, qk_norm=hd == 128, sigma=0.3)
+
+
+def tile_rows(lens):
+    seq = np.repeat(np.arange(len(lens)), lens)
+    return seq, np.concatenate([np.arange(n) for n in lens])
+
+
+@pytest.mark.parametrize("nh,nkv,hd", [(1, 1, 64), (4, 2, 64), (3, 1, 64), (4, 1, 64), (5, 1, 64),
+                                       (2, 2, 128), (2, 1, 128), (3, 1, 128), (4, 1, 128)])
+@pytest.mark.parametrize("copies", [1, 300], ids=["one-head-items", "grouped-items"])
+def test_attention_tiles_bits(nh, nkv, hd, copies):
+    """copies = 300: enough tiles that an item takes the heads of a KV head
+    together and a workgroup walks several items."""
+    spec = heads_spec(nh, nkv, hd)
+    w = artifacts.Weights(spec, 5)
+    lens = [1, 17, 63, 66, 129, 259] if copies == 1 else [19, 34] * (copies // 2)
+    m = Cis2Model(spec, w, max_pos=max(lens), max_seqs=len(lens))
+    seq, pos = tile_rows(lens)
+    tok = np.random.default_rng(3).integers(0, spec.vocab, seq.size).astype(np.uint32)
+    out = {}
+    for v in "01":
+        os.environ["CIS2_ATT_TILES"] = v
+        try:
+            out[v], _ = m.forward_rows(seq, pos, tok)
+        finally:
+            del os.environ["CIS2_ATT_TILES"]
+    assert np.array_equal(out["0"].view(np.uint32), out["1"].view(np.uint32))
+    s = len(lens) - 1
+    o = O.OracleModel(spec, w, max_pos=lens[s], reduction=0)
+    rows = np.flatnonzero(seq == s)
+    for p, r in enumerate(rows):
+        assert np.array_equal(o.forward(p, int(tok[r])).view(np.uint32),
+                              out["1"][r].view(np.uint32)), p
+
+
+def test_attention_tiles_later_rows_do_not_leak():
+    """A row whose V (and K) hold NaN or infinities changes no row before it,
+    also inside one tile, and not a NaN's or a zero's sign there."""
+    spec = heads_spec(2, 1, 64)
+    w = artifacts.Weights(spec, 6)
+    emb = next(a for name, _, a in w.tensors if "embed" in name)
+    emb[7 * spec.hidden] = 0x7F80       # token 7: +inf in one dimension
+    emb[8 * spec.hidden + 1] = 0xFFC1   # token 8: a NaN
+    n = 41
+    tok = np.arange(20, 20 + n).astype(np.uint32)
+    clean = Cis2Model(spec, w, max_pos=n)
+    base, _ = clean.forward_rows(np.zeros(n), np.arange(n), tok)
+    for at, bad in ((5, 7), (18, 8), (40, 7)):
+        t2 = tok.copy()
+        t2[at:at + 1] = bad
+        os.environ["CIS2_ATT_TILES"] = "1"
+        try:
+            got, _ = clean.forward_rows(np.zeros(n), np.arange(n), t2)
+        finally:
+            del os.environ["CIS2_ATT_TILES"]
+        assert np.array_equal(got[:at].view(np.uint32), base[:at].view(np.uint32)), at
+        assert not np.isfinite(got[at]).all()
+        os.environ["CIS2_ATT_TILES"] = "0"
+        try:
+            rows, _ = clean.forward_rows(np.zeros(n), np.arange(n), t2)
+        finally:
+            del os.environ["CIS2_ATT_TILES"]
+        assert np.array_equal(np.isnan(got), np.isnan(rows)), at
+        fin = ~np.isnan(rows)
+        assert np.array_equal(got.view(np.uint32)[fin], rows.view(np.uint32)[fin]), at
