@@ -260,6 +260,28 @@ __global__ __launch_bounds__(256) void k_rmsnorm(const float* x, const float* __
   }
 }
 
+__global__ void k_copy16(const float4* __restrict__ src, float4* __restrict__ dst, uint64_t n) {
+  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
+       i += (uint64_t)gridDim.x * blockDim.x)
+    dst[i] = src[i];
+}
+hipError_t launch_copy16(const float* src, float* dst, uint64_t n16, hipStream_t s) {
+  if (n16 == 0) return hipSuccess;
+  const uint32_t grid = (uint32_t)std::min<uint64_t>((n16 + 255) / 256, 256);
+  hipLaunchKernelGGL(k_copy16, dim3(grid), dim3(256), 0, s, reinterpret_cast<const float4*>(src),
+                     reinterpret_cast<float4*>(dst), n16);
+  return hipGetLastError();
+}
+
+__global__ void k_take_word(uint32_t* word, uint32_t* out) {
+  *out = *word;
+  *word = 0;
+}
+hipError_t launch_take_word(uint32_t* word, uint32_t* out, hipStream_t s) {
+  hipLaunchKernelGGL(k_take_word, dim3(1), dim3(1), 0, s, word, out);
+  return hipGetLastError();
+}
+
 hipError_t launch_rmsnorm(const float* x, const float* w, float eps, uint32_t n,
                           uint32_t nvec, float* out, hipStream_t s, bool tree) {
   if (n == 0 || n > 8192) return hipErrorInvalidValue;  // LDS: squares, partials, scalars

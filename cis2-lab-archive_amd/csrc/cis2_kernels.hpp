@@ -47,6 +47,10 @@ hipError_t launch_gate_up_silu(const float* Wg, const float* Wu, const float* x,
 // Relayout a row-major [M,K] f32 matrix (device) into the blocked layout.
 hipError_t launch_relayout(const float* src, float* dst, uint32_t M, uint32_t K, uint32_t R,
                            hipStream_t s);
+// dst[i] = src[i], i < n 16-byte groups (either side may be mapped host memory).
+hipError_t launch_copy16(const float* src, float* dst, uint64_t n16, hipStream_t s);
+// *out = *word, *word = 0 (out may be mapped host memory).
+hipError_t launch_take_word(uint32_t* word, uint32_t* out, hipStream_t s);
 // Exact BF16 -> F32 widening (bits << 16).
 hipError_t launch_widen(const uint16_t* src, float* dst, uint64_t n, hipStream_t s);
 

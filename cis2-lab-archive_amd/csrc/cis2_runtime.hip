@@ -127,6 +127,11 @@ struct cis2_ctx {
   // decode ring (pinned host)
   float* ring = nullptr;
   uint32_t* ring_tok = nullptr;
+  // cis2_forward of one row through the persistent kernel (mapped pinned
+  // host memory the kernel reads and writes itself): logits [vocab], then
+  // the token, the argmax and the error word
+  float* fwd_logits = nullptr;
+  uint32_t* fwd_words = nullptr;
   hipEvent_t ring_ev[kRing];
   hipEvent_t ring_ready[kRing];  // main stream: step's logits and token final
   Session sess;
@@ -181,6 +186,8 @@ struct cis2_gemv_plan {
   float *W = nullptr, *x = nullptr, *y = nullptr;
   float *xb = nullptr, *yb = nullptr;  // [ncap][K], [ncap][M]: batched launches
   uint32_t ncap = 0;
+  float *hx = nullptr, *hy = nullptr;  // mapped pinned host memory, hcap bytes each
+  size_t hcap = 0;
   hipStream_t st = nullptr;
   hipEvent_t e0 = nullptr, e1 = nullptr;
 };
@@ -906,6 +913,7 @@ void cis2_ctx_destroy(cis2_ctx* c) {
     if (e) (void)hipEventDestroy(e);
   if (c->ring) (void)hipHostFree(c->ring);
   if (c->ring_tok) (void)hipHostFree(c->ring_tok);
+  if (c->fwd_logits) (void)hipHostFree(c->fwd_logits);
   for (int i = 0; i < kRing; ++i) {
     if (c->ring_ev[i]) (void)hipEventDestroy(c->ring_ev[i]);
     if (c->ring_ready[i]) (void)hipEventDestroy(c->ring_ready[i]);
@@ -1014,10 +1022,13 @@ int cis2_ctx_create(const cis2_config* cfg, cis2_ctx** out) {
   if (hipHostMalloc(reinterpret_cast<void**>(&c->ring), (size_t)kRing * V * sizeof(float)) !=
           hipSuccess ||
       hipHostMalloc(reinterpret_cast<void**>(&c->ring_tok), kRing * 2 * sizeof(uint32_t)) !=
+          hipSuccess ||
+      hipHostMalloc(reinterpret_cast<void**>(&c->fwd_logits), ((size_t)V + 4) * sizeof(float)) !=
           hipSuccess) {
     cis2_ctx_destroy(c);
     return CIS2_E_OOM;
   }
+  c->fwd_words = reinterpret_cast<uint32_t*>(c->fwd_logits + V);
   for (int i = 0; i < kRing; ++i)
     if (hipEventCreateWithFlags(&c->ring_ev[i], hipEventDisableTiming) != hipSuccess ||
         hipEventCreateWithFlags(&c->ring_ready[i], hipEventDisableTiming) != hipSuccess) {
@@ -1318,35 +1329,49 @@ int cis2_forward(cis2_ctx* c, uint32_t n, const uint32_t* seq, const uint32_t* p
     return check_err_flag(c);
   }
   const bool held = c->lock_fd >= 0;  // a decode session of this context holds the lock
+  bool flagged = false;  // the device error word has to be looked at again
   for (uint32_t i = 0; i < n; ++i) {
     if (seq[i] >= c->cfg.max_seqs) return fail(c, CIS2_E_ARG, "sequence index out of range");
     if (pos[i] >= c->cfg.max_pos) return fail(c, CIS2_E_RANGE, "position beyond max_pos");
     if (tok[i] >= c->cfg.vocab) return fail(c, CIS2_E_RANGE, "token id >= vocab");
-    HIPCHK(c, hipMemcpyAsync(c->d_tok, &tok[i], 4, hipMemcpyHostToDevice, c->st), "token");
-    bool ops = !use_fast(c);
-    if (!ops) {
+    if (use_fast(c)) {
+      // token, logits, argmax and error word go through mapped host memory:
+      // one launch, one word's launch and one wait, where the copies and
+      // their waits took 130 us more than the kernel's 740 (196 KB of logits)
       decode_lock(c);
-      r = forward_fast(c, seq[i], pos[i], c->d_tok, true);
+      volatile uint32_t* hw = c->fwd_words;
+      hw[0] = tok[i];
+      r = forward_fast(c, seq[i], pos[i], c->fwd_words, true,
+                       logits_host ? c->fwd_logits : nullptr, c->fwd_words + 1);
       if (r) return r;
-      HIPCHK(c, hipMemcpyAsync(c->d_tok + 1, c->d_tok, 4, hipMemcpyDeviceToDevice, c->st),
-             "argmax copy");
+      LAUNCH(launch_take_word(c->d_err, c->fwd_words + 2, c->st), "error word");
+      HIPCHK(c, hipStreamSynchronize(c->st), "forward sync");
+      const uint32_t bits = hw[2];
+      if (!(bits & 2u)) {
+        if (bits) {
+          HIPCHK(c, hipMemcpy(c->d_err, &bits, 4, hipMemcpyHostToDevice), "error flag");
+          flagged = true;
+        }
+        if (logits_host)
+          memcpy(logits_host + (size_t)i * c->cfg.vocab, c->fwd_logits,
+                 (size_t)c->cfg.vocab * sizeof(float));
+        if (argmax_out) argmax_out[i] = hw[1];
+        continue;
+      }
       // a persistent launch that hit the spin cap: this row again on the
       // per-op path (it rewrites the position's K/V rows in every layer)
-      uint32_t bits = 0;
-      r = drain_and_clear_err(c, &bits);
+      uint32_t left = 0;
+      r = drain_and_clear_err(c, &left);
       if (r) return r;
-      if (bits & ~2u) HIPCHK(c, hipMemcpy(c->d_err, &bits, 4, hipMemcpyHostToDevice), "error flag");
-      if (bits & 2u) {
-        c->recoveries++;
-        ops = true;
-        HIPCHK(c, hipMemcpyAsync(c->d_tok, &tok[i], 4, hipMemcpyHostToDevice, c->st), "token");
-      }
+      left = (left | bits) & ~2u;
+      if (left) HIPCHK(c, hipMemcpy(c->d_err, &left, 4, hipMemcpyHostToDevice), "error flag");
+      c->recoveries++;
     }
-    if (ops) {
-      r = forward_one(c, seq[i], pos[i], c->d_tok, true);
-      if (r) return r;
-      if (argmax_out) LAUNCH(launch_argmax(c->logits, c->cfg.vocab, c->d_tok + 1, c->st), "argmax");
-    }
+    flagged = true;
+    HIPCHK(c, hipMemcpyAsync(c->d_tok, &tok[i], 4, hipMemcpyHostToDevice, c->st), "token");
+    r = forward_one(c, seq[i], pos[i], c->d_tok, true);
+    if (r) return r;
+    if (argmax_out) LAUNCH(launch_argmax(c->logits, c->cfg.vocab, c->d_tok + 1, c->st), "argmax");
     HIPCHK(c, hipStreamSynchronize(c->st), "forward sync");
     if (logits_host)
       HIPCHK(c, hipMemcpy(logits_host + (size_t)i * c->cfg.vocab, c->logits,
@@ -1356,7 +1381,7 @@ int cis2_forward(cis2_ctx* c, uint32_t n, const uint32_t* seq, const uint32_t* p
       HIPCHK(c, hipMemcpy(&argmax_out[i], c->d_tok + 1, 4, hipMemcpyDeviceToHost), "argmax copy");
   }
   if (!held) decode_unlock(c);
-  return check_err_flag(c);
+  return flagged ? check_err_flag(c) : CIS2_OK;
 }
 
 // Receipt header of a sampled decode (draft 14.5): "CIS2-SAMPLE-1", seed
@@ -2017,6 +2042,25 @@ int cis2_verify_prefill(cis2_ctx* c, uint32_t seq, const uint32_t* prompt, uint3
 
 // ---- standalone GEMV ------------------------------------------------------
 
+// Host vectors of up to kPlanHost bytes go through the plan's mapped pinned
+// memory, which the GEMV reads and writes itself: 1536 x 576 19.8 us a call,
+// 21.5 with x fetched by a kernel first, 30.5 with copies from and to
+// pageable memory; 49152 x 576 41, 45 and 56 us.  A batch's inputs are
+// fetched first (60 of 200 x 2000: 88 against 120 us).  Larger ones are
+// copied.
+constexpr size_t kPlanHost = 1 << 20;
+static hipError_t plan_host(cis2_gemv_plan* p, size_t bytes) {
+  if (bytes <= p->hcap) return hipSuccess;
+  if (p->hx) (void)hipHostFree(p->hx);
+  if (p->hy) (void)hipHostFree(p->hy);
+  p->hx = p->hy = nullptr;
+  p->hcap = 0;
+  hipError_t e = hipHostMalloc(reinterpret_cast<void**>(&p->hx), bytes);
+  if (e == hipSuccess) e = hipHostMalloc(reinterpret_cast<void**>(&p->hy), bytes);
+  if (e == hipSuccess) p->hcap = bytes;
+  return e;
+}
+
 int cis2_gemv_plan_create(uint32_t M, uint32_t K, uint32_t copies, const float* W,
                           cis2_gemv_plan** out) {
   if (!W || !out || M == 0 || K == 0 || K % 4 || copies == 0) return CIS2_E_ARG;
@@ -2036,6 +2080,8 @@ int cis2_gemv_plan_create(uint32_t M, uint32_t K, uint32_t copies, const float* 
   if (e == hipSuccess) e = hipStreamSynchronize(p->st);
   if (e == hipSuccess) e = hipEventCreate(&p->e0);
   if (e == hipSuccess) e = hipEventCreate(&p->e1);
+  const size_t host = ((size_t)std::max(M, K)) * sizeof(float) + 256;
+  if (e == hipSuccess && host <= kPlanHost) e = plan_host(p, host);
   if (rowmajor) (void)hipFree(rowmajor);
   if (e != hipSuccess) {
     cis2_gemv_plan_destroy(p);
@@ -2057,13 +2103,39 @@ static hipError_t plan_launch(cis2_gemv_plan* p, uint32_t c, const float* x, flo
   return launch_gemv_blk(p->W + per * (c % p->copies), x, y, p->M, p->K, kPlanR, p->st);
 }
 
+// x to the device, the lone GEMV (n = 0) or n GEMVs in one launch, y back.
+static hipError_t plan_through(cis2_gemv_plan* p, uint32_t n, const float* x, float* y) {
+  const size_t nx = (size_t)(n ? n : 1) * p->K, ny = (size_t)(n ? n : 1) * p->M;
+  float *dx = n ? p->xb : p->x, *dy = n ? p->yb : p->y;
+  auto launch = [&](float* yd) {
+    return n ? launch_gemv_many(p->W, blocked_floats(p->M, p->K, kPlanR), p->copies, 0, n, dx, yd,
+                                p->M, p->K, kPlanR, p->st)
+             : plan_launch(p, 0, dx, yd);
+  };
+  const size_t most = std::max(nx, ny) * sizeof(float) + 256;
+  hipError_t e;
+  if (most > kPlanHost || plan_host(p, most) != hipSuccess) {
+    (void)hipGetLastError();  // no pinned memory: copy
+    e = hipMemcpyAsync(dx, x, nx * sizeof(float), hipMemcpyHostToDevice, p->st);
+    if (e == hipSuccess) e = launch(dy);
+    if (e == hipSuccess)
+      e = hipMemcpyAsync(y, dy, ny * sizeof(float), hipMemcpyDeviceToHost, p->st);
+    return e == hipSuccess ? hipStreamSynchronize(p->st) : e;
+  }
+  memcpy(p->hx, x, nx * sizeof(float));
+  if (n)
+    e = launch_copy16(p->hx, dx, nx / 4, p->st);
+  else
+    dx = p->hx, e = hipSuccess;
+  if (e == hipSuccess) e = launch(p->hy);
+  if (e == hipSuccess) e = hipStreamSynchronize(p->st);
+  if (e == hipSuccess) memcpy(y, p->hy, ny * sizeof(float));
+  return e;
+}
+
 int cis2_gemv_plan_run(cis2_gemv_plan* p, const float* x, float* y) {
   if (!p || !x || !y) return CIS2_E_ARG;
-  hipError_t e = hipMemcpyAsync(p->x, x, (size_t)p->K * sizeof(float), hipMemcpyHostToDevice, p->st);
-  if (e == hipSuccess) e = plan_launch(p, 0, p->x, p->y);
-  if (e == hipSuccess) e = hipMemcpyAsync(y, p->y, (size_t)p->M * sizeof(float), hipMemcpyDeviceToHost, p->st);
-  if (e == hipSuccess) e = hipStreamSynchronize(p->st);
-  return e == hipSuccess ? CIS2_OK : CIS2_E_DEVICE;
+  return plan_through(p, 0, x, y) == hipSuccess ? CIS2_OK : CIS2_E_DEVICE;
 }
 
 int cis2_gemv_plan_time(cis2_gemv_plan* p, uint32_t iters, float* ms) {
@@ -2104,14 +2176,7 @@ int cis2_gemv_plan_run_batch(cis2_gemv_plan* p, uint32_t n, const float* x, floa
   if (!p || (n && (!x || !y)) || n > 65535) return CIS2_E_ARG;
   if (n == 0) return CIS2_OK;
   hipError_t e = plan_reserve(p, n);
-  if (e == hipSuccess)
-    e = hipMemcpyAsync(p->xb, x, (size_t)n * p->K * sizeof(float), hipMemcpyHostToDevice, p->st);
-  if (e == hipSuccess)
-    e = launch_gemv_many(p->W, blocked_floats(p->M, p->K, kPlanR), p->copies, 0, n, p->xb, p->yb,
-                         p->M, p->K, kPlanR, p->st);
-  if (e == hipSuccess)
-    e = hipMemcpyAsync(y, p->yb, (size_t)n * p->M * sizeof(float), hipMemcpyDeviceToHost, p->st);
-  if (e == hipSuccess) e = hipStreamSynchronize(p->st);
+  if (e == hipSuccess) e = plan_through(p, n, x, y);
   return e == hipSuccess ? CIS2_OK : (e == hipErrorOutOfMemory ? CIS2_E_OOM : CIS2_E_DEVICE);
 }
 
@@ -2143,6 +2208,8 @@ void cis2_gemv_plan_destroy(cis2_gemv_plan* p) {
   if (p->W) (void)hipFree(p->W);
   if (p->x) (void)hipFree(p->x);
   if (p->y) (void)hipFree(p->y);
+  if (p->hx) (void)hipHostFree(p->hx);
+  if (p->hy) (void)hipHostFree(p->hy);
   if (p->e0) (void)hipEventDestroy(p->e0);
   if (p->e1) (void)hipEventDestroy(p->e1);
   if (p->st) (void)hipStreamDestroy(p->st);
