@@ -3,6 +3,7 @@
 // computed by one lane in the order the single-row kernels use
 // (code/cis2-fp/src/main.rs:355-529), so a row's results do not depend on
 // which other rows share the launch (batch invariance).
+#include "cis2_chain.hpp"
 #include "cis2_device_math.hpp"
 #include "cis2_rows.hpp"
 #include "cis2_kernels.hpp"
@@ -575,6 +576,220 @@ __global__ __launch_bounds__(256) void k_bgemm16(BgemmArgs a) {
       y = acc + g.add[m];
     } else if (g.epi == kEpiResidual) {
       y = g.add[(size_t)row * g.ldadd + m] + acc;
+    }
+    g.Y[(size_t)row * g.ldy + m] = y;
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Batched GEMM for few rows (decode steps; sequential order): a workgroup
+// owns 8 outputs x 8 batch rows, 64 chains, and splits the work of a chain
+// step between its waves.  Eight product waves form p = W[m][k] * X[b][k] for
+// a 16-byte group of every chain (lane l: output l % 8, row l / 8) and store
+// the groups in an LDS ring of four slots of 16 groups; chain wave 0 adds
+// them, k ascending, one chain per lane (k_bgemm's bits).  DUAL: chain wave 1
+// runs the up projection's chains over W2, and silu(gate) * up is stored.
+// NORM: wave 0 chains the rows' squares first, then the rows are scaled in
+// LDS, (x * inv) * w[k].  W (and X without a norm) goes from global memory to
+// the product waves' registers, D slots ahead (all of K = 576).
+// What bounds it: 3.6 us of launch, prologue and end, then the chain, 9.6
+// cycles per k (6.1 with nothing else on the LDS) against 16 when the chain's
+// wave forms its own products (k_bgemm16).  At 8 rows, us, k_bgemm16 then
+// here: 960 x 576 with the norm 12.0 8.6, 576 x 576 8.3 6.1, gate and up of
+// 1536 x 576 with the norm 16.1 10.1, 576 x 1536 16.8 9.8.
+// LDS (16-byte groups): ring [CW][4 slots][16][64] (first the squares), NORM:
+// rows [K/4][8], then inverse RMS [8] and up sums [64].  Past K the products
+// are -0, which no sum notices.
+// ---------------------------------------------------------------------------
+template <bool DUAL, bool NORM>
+struct ChainCfg {
+  static constexpr uint32_t CW = DUAL ? 2 : 1, NP = 8, T = 64 * (CW + NP);
+  static constexpr uint32_t SG = 16, GPW = SG / NP;      // groups per slot, per wave of it
+  static constexpr uint32_t D = DUAL ? (NORM ? 5 : 4) : (NORM ? 9 : 8);  // slots loaded ahead
+  static constexpr uint32_t ring = CW * 4 * SG * 64;     // 16-byte groups
+  static constexpr size_t lds(uint32_t K) {
+    return ((size_t)ring + (NORM ? (size_t)K / 4 * 8 : 0)) * 16 + (8 + 64) * 4;
+  }
+};
+// Largest dynamic LDS of a workgroup.
+constexpr size_t kLdsMost = 160 * 1024 - 256;
+__device__ __forceinline__ void lds_only_barrier() {
+  __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+template <bool DUAL, bool NORM>
+__global__ __launch_bounds__((ChainCfg<DUAL, NORM>::T), 3) void k_chain_gemm(BgemmArgs a) {
+  using C = ChainCfg<DUAL, NORM>;
+  constexpr uint32_t CW = C::CW, NP = C::NP, GPW = C::GPW, SG = C::SG, D = C::D, T = C::T;
+  extern __shared__ v4 sm[];
+  uint32_t si = 0;
+  if (a.nseg > 1 && blockIdx.x >= a.blk0[1]) si = (a.nseg > 2 && blockIdx.x >= a.blk0[2]) ? 2 : 1;
+  const BgemmSeg g = si == 0 ? a.s[0] : (si == 1 ? a.s[1] : a.s[2]);
+  const uint32_t R = g.R, K = g.K, K4 = K / 4, t = threadIdx.x;
+  const uint32_t m0 = (blockIdx.x - a.blk0[si]) * 8, b0 = blockIdx.y * 8;
+  const uint32_t wv = __builtin_amdgcn_readfirstlane(t >> 6), lane = t & 63;
+  const uint32_t r = lane & 7, b = lane >> 3, ns = (K4 + SG - 1) / SG;
+  v4* ring = sm;
+  v4* xs = sm + C::ring;                                    // [K4][8]
+  float* s_inv = reinterpret_cast<float*>(xs + (NORM ? K4 * 8 : 0));  // [8]
+  float* s_up = s_inv + 8;                                  // [64]
+  // X rows as [group][row] (and the squares, into the ring's space): the
+  // loads go out before W's, in the order they are needed
+  const v4* xn = reinterpret_cast<const v4*>(g.X + (size_t)min(b0 + (t & 7), a.n - 1) * g.ldx);
+  constexpr uint32_t XB = 6;  // X loads in flight (K = 1536 in one round)
+  v4 x0[XB];
+#pragma unroll
+  for (uint32_t i = 0; i < XB; ++i)
+    if (NORM && t + T * i < K4 * 8) x0[i] = xn[(t + T * i) >> 3];
+  const bool chain = wv < CW;
+  const size_t woff = (size_t)(m0 / R) * R * K4 + m0 % R + r;
+  const v4* wp = reinterpret_cast<const v4*>(g.W) + woff;
+  const v4* wp2 = DUAL ? reinterpret_cast<const v4*>(a.W2) + woff : nullptr;
+  const v4* xp = reinterpret_cast<const v4*>(g.X + (size_t)min(b0 + b, a.n - 1) * g.ldx);
+  v4 pw[D][GPW], pu[D][GPW], px[D][GPW];
+  // the groups of slot c that this wave forms (past K: the last one again)
+  auto load = [&](uint32_t c, uint32_t s) {
+#pragma unroll
+    for (uint32_t i = 0; i < GPW; ++i) {
+      const uint32_t q = min(c * SG + i * NP + (wv - CW), K4 - 1);
+      pw[s][i] = wp[q * R];
+      if (DUAL) pu[s][i] = wp2[q * R];
+      if (!NORM) px[s][i] = xp[q];
+    }
+  };
+  if (!chain) {
+#pragma unroll
+    for (uint32_t s = 0; s < D; ++s)
+      if (s < ns) load(s, s);
+  }
+  auto square = [](const v4& x) {
+    v4 q;
+    q.x = x.x * x.x;
+    q.y = x.y * x.y;
+    q.z = x.z * x.z;
+    q.w = x.w * x.w;
+    return q;
+  };
+  if (NORM) {
+#pragma unroll
+    for (uint32_t i = 0; i < XB; ++i) {
+      const uint32_t e = t + T * i;
+      if (e < K4 * 8) {
+        xs[e] = x0[i];
+        ring[e] = square(x0[i]);
+      }
+    }
+    for (uint32_t e = t + T * XB; e < K4 * 8; e += T) {
+      const v4 x = xn[e >> 3];
+      xs[e] = x;
+      ring[e] = square(x);
+    }
+    lds_only_barrier();
+    if (wv == 0) {
+      float acc = 0.0f;
+      const v4* sp = ring + r;  // lane l: row l % 8
+      const uint32_t np = K4 / 16;
+      if (np) acc = chain_lds16_low<8>((const AS_LDS void*)sp, np, acc);
+      for (uint32_t q = 16 * np; q < K4; ++q) {
+        const v4 x = sp[q * 8];
+        acc = acc + x.x;
+        acc = acc + x.y;
+        acc = acc + x.z;
+        acc = acc + x.w;
+      }
+      const float inv = inv_rms_of(acc, K, a.eps);
+      if (lane < 8) s_inv[lane] = inv;
+    }
+    lds_only_barrier();
+    const float inv = s_inv[t & 7];
+    for (uint32_t i = t; i < K4 * 8; i += T) {
+      v4 x = xs[i];
+      const v4 w = reinterpret_cast<const v4*>(a.nw)[i >> 3];
+      float sx;
+      sx = x.x * inv; x.x = sx * w.x;
+      sx = x.y * inv; x.y = sx * w.y;
+      sx = x.z * inv; x.z = sx * w.z;
+      sx = x.w * inv; x.w = sx * w.w;
+      xs[i] = x;
+    }
+  }
+  // the addend's load is in flight during the chains
+  const uint32_t m = m0 + r, row = b0 + b;
+  const bool mine = wv == 0 && row < a.n && m < g.M;
+  float addend = 0.0f;
+  if (!DUAL && mine && g.epi != kEpiNone)
+    addend = g.epi == kEpiBias ? g.add[m] : g.add[(size_t)row * g.ldadd + m];
+  lds_only_barrier();
+  float acc = 0.0f;
+  if (chain) {
+    __builtin_amdgcn_s_setprio(3);
+    lds_only_barrier();  // slot 0
+    const uint32_t base = (uint32_t)(uintptr_t)(const AS_LDS void*)(ring + wv * 4 * SG * 64);
+    acc = chain_ring(base + lane * 16, base, ns, acc);
+  } else {
+    v4 x[GPW];
+    auto xload = [&](uint32_t c) {
+#pragma unroll
+      for (uint32_t i = 0; i < GPW; ++i)
+        if (NORM) x[i] = xs[min(c * SG + i * NP + (wv - CW), K4 - 1) * 8 + b];
+    };
+    xload(0);
+    for (uint32_t c0 = 0; c0 < ns; c0 += D) {
+#pragma unroll
+      for (uint32_t s = 0; s < D; ++s) {
+        const uint32_t c = c0 + s;
+        if (c >= ns) break;
+        v4 p[GPW], p2[GPW];
+#pragma unroll
+        for (uint32_t i = 0; i < GPW; ++i) {
+          const v4 w = pw[s][i];
+          if (!NORM) x[i] = px[s][i];
+          p[i].x = w.x * x[i].x;
+          p[i].y = w.y * x[i].y;
+          p[i].z = w.z * x[i].z;
+          p[i].w = w.w * x[i].w;
+          if (DUAL) {
+            const v4 w2 = pu[s][i];
+            p2[i].x = w2.x * x[i].x;
+            p2[i].y = w2.y * x[i].y;
+            p2[i].z = w2.z * x[i].z;
+            p2[i].w = w2.w * x[i].w;
+          }
+        }
+        if ((c + 1) * SG > K4) {  // the last slot's groups past K
+          const float z = __int_as_float((int)0x80000000u);
+#pragma unroll
+          for (uint32_t i = 0; i < GPW; ++i)
+            if (c * SG + i * NP + (wv - CW) >= K4) p[i] = p2[i] = v4{z, z, z, z};
+        }
+        v4* slot = ring + (c & 3) * SG * 64 + lane;
+#pragma unroll
+        for (uint32_t i = 0; i < GPW; ++i) {
+          slot[(i * NP + (wv - CW)) * 64] = p[i];
+          if (DUAL) slot[(4 * SG + i * NP + (wv - CW)) * 64] = p2[i];
+        }
+        xload(c + 1);
+        if (c + D < ns) load(c + D, s);
+        lds_only_barrier();
+      }
+    }
+  }
+  if (DUAL) {
+    if (wv == 1) s_up[lane] = acc;
+    lds_only_barrier();
+  }
+  if (mine) {
+    float y = acc;
+    if (DUAL) {
+      const float sg = silu_pinned(acc);
+      y = sg * s_up[lane];
+    } else if (g.epi == kEpiBias) {
+      y = acc + addend;
+    } else if (g.epi == kEpiResidual) {
+      y = addend + acc;
     }
     g.Y[(size_t)row * g.ldy + m] = y;
   }
@@ -2018,6 +2233,13 @@ hipError_t rows_configure() {
     hipError_t e = ensure_dynamic_lds(f, kBgemmLdsBig);
     if (e != hipSuccess) return e;
   }
+  for (const void* f : {reinterpret_cast<const void*>(&k_chain_gemm<false, false>),
+                        reinterpret_cast<const void*>(&k_chain_gemm<false, true>),
+                        reinterpret_cast<const void*>(&k_chain_gemm<true, false>),
+                        reinterpret_cast<const void*>(&k_chain_gemm<true, true>)}) {
+    hipError_t e = ensure_dynamic_lds(f, kLdsMost);
+    if (e != hipSuccess) return e;
+  }
   return hipSuccess;
 }
 
@@ -2101,6 +2323,44 @@ static hipError_t launch_mgemm(const BgemmSeg* segs, uint32_t nseg, uint32_t n,
   return hipGetLastError();
 }
 
+template <bool DUAL, bool NORM>
+static hipError_t launch_chain_gemm(const BgemmSeg* segs, uint32_t nseg, uint32_t n,
+                                    const BgemmOpts& o, hipStream_t st) {
+  BgemmArgs a = {};
+  for (uint32_t i = 0; i < kMaxSegs; ++i) {
+    a.s[i] = segs[i < nseg ? i : 0];
+    a.blk0[i + 1] = i < nseg ? a.blk0[i] + (segs[i].M + 7) / 8 : a.blk0[nseg];
+  }
+  a.nseg = nseg;
+  a.n = n;
+  a.W2 = o.W2;
+  a.nw = o.norm_w;
+  a.eps = o.eps;
+  hipLaunchKernelGGL((k_chain_gemm<DUAL, NORM>), dim3(a.blk0[nseg], (n + 7) / 8), dim3(ChainCfg<DUAL, NORM>::T),
+                     (ChainCfg<DUAL, NORM>::lds(segs[0].K)), st, a);
+  return hipGetLastError();
+}
+// k_chain_gemm takes segments whose blocks are whole groups of 8 rows, rows
+// that fit the LDS beside the ring (fused norm), and grids that the CUs hold
+// at once, one workgroup per CU: a second round costs more than k_bgemm16's
+// one (n = 8 | 16 | 24, us, k_bgemm16 then k_chain_gemm: 576 x 1536 16.7
+// 9.8 | 16.7 10.0 | 16.8 10.1, 768 x 3072 30.4 16.0 | 30.3 16.4 | 30.5 28.5).
+// Below 256 k its two prologue round trips are not won back (K = 52: 4.6
+// against 5.5).
+static bool chain_gemm_fits(const BgemmSeg* segs, uint32_t nseg, uint32_t n, const BgemmOpts& o,
+                            uint32_t ncu) {
+  const uint32_t K = segs[0].K;
+  if (segs[0].R % 8 || K < 256) return false;
+  if (o.norm_w) {
+    if ((o.W2 ? ChainCfg<true, true>::lds(K) : ChainCfg<false, true>::lds(K)) > kLdsMost ||
+        (size_t)K / 4 * 8 > (o.W2 ? ChainCfg<true, true>::ring : ChainCfg<false, true>::ring))
+      return false;
+  }
+  uint64_t wgs = 0;
+  for (uint32_t i = 0; i < nseg; ++i) wgs += (segs[i].M + 7) / 8;
+  return wgs * ((n + 7) / 8) <= ncu;
+}
+
 // Which kernel a sequential-order GEMM without a fused norm takes.  Every
 // form costs a time per k that depends on how many workgroups the fullest CU
 // gets; measured on the layer shapes of the three models at n = 7 .. 16384,
@@ -2151,6 +2411,12 @@ hipError_t launch_bgemm_multi(const BgemmSeg* segs, uint32_t nseg, uint32_t n,
       return hipErrorInvalidValue;
   const int ncu = device_cu_count();
   if (!o.tree && bgemm16_allowed()) {
+    if (chain_gemm_fits(segs, nseg, n, o, (uint32_t)ncu)) {
+      if (o.W2) return o.norm_w ? launch_chain_gemm<true, true>(segs, nseg, n, o, st)
+                                : launch_chain_gemm<true, false>(segs, nseg, n, o, st);
+      return o.norm_w ? launch_chain_gemm<false, true>(segs, nseg, n, o, st)
+                      : launch_chain_gemm<false, false>(segs, nseg, n, o, st);
+    }
     if (!o.norm_w) {
       switch (mgemm_tile(segs, nseg, n, o.W2 != nullptr, (uint32_t)ncu)) {
         case MgemmTile::large:

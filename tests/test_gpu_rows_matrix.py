@@ -1,6 +1,8 @@
-"""The row-batched kernels whose products come from the matrix cores.
+"""The row-batched kernels that split a chain's products from its adds.
 
-GEMMs (k_mgemm): sizes that are no multiple of any tile in rows, outputs or
+Few rows (k_chain_gemm): row counts around its 8-row tiles, outputs and K
+that are no multiple of its tiles, with and without the fused norm and the
+gate.  GEMMs on the matrix cores (k_mgemm): sizes that are no multiple of any tile in rows, outputs or
 K, weights with signed zeros and products that flush to zero; against the
 vector-unit kernel (CIS2_BGEMM16=0) and the oracle.  Prefill attention
 (k_attention_tiles): every number of heads per item, runs that end inside a
@@ -21,6 +23,14 @@ pytestmark = pytest.mark.gpu
 ODD = artifacts.ModelSpec("odd", 132, 268, 1, 6, 2, 301, 1e-5, 10000.0, True, head_dim=22)
 # K = 20 (one partial group of 16 and one of 4), a vocabulary of many tiles
 WIDE = artifacts.ModelSpec("wide-vocab", 20, 28, 1, 2, 1, 40003, 1e-5, 10000.0, True)
+
+
+# reductions of 260, 264 and 516: a partial 64-k slot; outputs that end inside
+# an 8-row tile
+FEW = artifacts.ModelSpec("few", 260, 516, 2, 4, 1, 301, 1e-5, 10000.0, True, head_dim=66)
+# whole slots, q/k/v biases
+FEW_QWEN2 = artifacts.ModelSpec("few-qwen2", 320, 256, 1, 5, 5, 97, 1e-6, 10000.0, True,
+                                qkv_bias=True)
 
 
 class EdgeWeights(artifacts.Weights):
@@ -48,6 +58,13 @@ def run(m, n, per_seq, tok, mode):
 
 
 @pytest.mark.parametrize("spec,n,per_seq", [
+    (FEW, 1, 1),
+    (FEW, 3, 1),         # one row per sequence (a decode step)
+    (FEW, 8, 4),
+    (FEW, 9, 9),
+    (FEW, 31, 16),
+    (FEW_QWEN2, 7, 7),
+    (FEW_QWEN2, 17, 1),
     (WIDE, 5, 5),        # LM head: 64 x 16 tiles, one partial
     (WIDE, 16, 4),
     (WIDE, 17, 17),      # the first row count of the 32 x 32 tiles
