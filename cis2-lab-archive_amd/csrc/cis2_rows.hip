@@ -613,7 +613,9 @@ struct ChainCfg {
 };
 // Largest dynamic LDS of a workgroup.
 constexpr size_t kLdsMost = 160 * 1024 - 256;
-__device__ __forceinline__ void lds_only_barrier() {
+// s_waitcnt lgkmcnt(0), then s_barrier: LDS written before it is visible
+// after it; global loads in flight stay in flight.
+__device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
   asm volatile("" ::: "memory");
   __builtin_amdgcn_s_barrier();
@@ -687,7 +689,7 @@ __global__ __launch_bounds__((ChainCfg<DUAL, NORM>::T), 3) void k_chain_gemm(Bge
       xs[e] = x;
       ring[e] = square(x);
     }
-    lds_only_barrier();
+    lds_barrier();
     if (wv == 0) {
       float acc = 0.0f;
       const v4* sp = ring + r;  // lane l: row l % 8
@@ -703,7 +705,7 @@ __global__ __launch_bounds__((ChainCfg<DUAL, NORM>::T), 3) void k_chain_gemm(Bge
       const float inv = inv_rms_of(acc, K, a.eps);
       if (lane < 8) s_inv[lane] = inv;
     }
-    lds_only_barrier();
+    lds_barrier();
     const float inv = s_inv[t & 7];
     for (uint32_t i = t; i < K4 * 8; i += T) {
       v4 x = xs[i];
@@ -722,11 +724,11 @@ __global__ __launch_bounds__((ChainCfg<DUAL, NORM>::T), 3) void k_chain_gemm(Bge
   float addend = 0.0f;
   if (!DUAL && mine && g.epi != kEpiNone)
     addend = g.epi == kEpiBias ? g.add[m] : g.add[(size_t)row * g.ldadd + m];
-  lds_only_barrier();
+  lds_barrier();
   float acc = 0.0f;
   if (chain) {
     __builtin_amdgcn_s_setprio(3);
-    lds_only_barrier();  // slot 0
+    lds_barrier();  // slot 0
     const uint32_t base = (uint32_t)(uintptr_t)(const AS_LDS void*)(ring + wv * 4 * SG * 64);
     acc = chain_ring(base + lane * 16, base, ns, acc);
   } else {
@@ -773,13 +775,13 @@ __global__ __launch_bounds__((ChainCfg<DUAL, NORM>::T), 3) void k_chain_gemm(Bge
         }
         xload(c + 1);
         if (c + D < ns) load(c + D, s);
-        lds_only_barrier();
+        lds_barrier();
       }
     }
   }
   if (DUAL) {
     if (wv == 1) s_up[lane] = acc;
-    lds_only_barrier();
+    lds_barrier();
   }
   if (mine) {
     float y = acc;
@@ -1481,12 +1483,6 @@ struct KvFuse {
   uint32_t nkv;
 };
 
-// s_waitcnt lgkmcnt(0), then s_barrier: LDS written before it is visible
-// after it; global loads in flight stay in flight.
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_s_waitcnt(0xC07F);
-  __builtin_amdgcn_s_barrier();
-}
 // acc + P_0 * v[0].x + P_1 * v[0].y + ... + P_15 * v[3].w in order (P_k:
 // lane k of this lane's 16-lane row), each product rounded, then the add.
 template <uint32_t K = 0>
@@ -1781,6 +1777,177 @@ __global__ __launch_bounds__(kKvT) void k_attention_kv(const float* __restrict__
     acc = acc + pr;
   }
   if (wv < CW) out[(size_t)r * nh * HD + (size_t)(qh0 + h) * HD + d] = acc;
+}
+
+// ---------------------------------------------------------------------------
+// Attention of many decode rows (sequential order): one wave per (row, query
+// head), no barrier, with the per-row kernel's arithmetic in the same order.
+// Lane j takes position j of every 64 (the column's 64 K loads in flight, q
+// by LDS broadcast); maximum by shuffles; every lane runs the denominator
+// chain; lane d mixes output dim d from its contiguous V row.  FUSE: RoPE of
+// the row's q head and k head, whose first query head stores k and v at pos,
+// as in k_attention_kv.
+// What bounds it: the cache lines of short K and V rows (and one 4-byte store
+// per row of either); thousands of waves hide each other's chains and load
+// latency, where a workgroup per pair spent its time in barriers with most
+// threads idle.
+// LDS per wave (floats): q [HD], k [HD], v [HD], scores [ls].
+// ---------------------------------------------------------------------------
+// LDS written by other lanes of this wave is readable after it.
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_s_waitcnt(0xC07F);
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_wave_barrier();
+}
+
+template <uint32_t HD, bool FUSE>
+__global__ __launch_bounds__(256) void k_attention_wave(
+    const float* __restrict__ q, float* kc, float* vc, RowsDesc rows, uint32_t nh, uint32_t group,
+    uint32_t max_pos, uint64_t seq_stride, float scale, float* out, uint32_t ls, KvFuse fz) {
+  extern __shared__ v4 sh4[];
+  constexpr uint32_t half = HD / 2;
+  const uint32_t wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const uint32_t item = blockIdx.x * 4 + wv;
+  if (item >= rows.n * nh) return;
+  const uint32_t r = item / nh, h = item - r * nh, kvh = h / group;
+  const uint32_t pos = rows.pos[r], len = pos + 1, lc = FUSE ? pos : len;
+  float* sq = reinterpret_cast<float*>(sh4) + wv * (3 * HD + ls);
+  float *kself = sq + HD, *vself = kself + HD, *ss = vself + HD;
+  const size_t sb = (size_t)rows.seq[r] * seq_stride + (size_t)kvh * HD * max_pos;
+  float* kb = kc + sb;
+  float* vb = vc + sb;
+  const float* qv = q + ((size_t)r * nh + h) * HD;
+  if constexpr (FUSE) {
+    const float* cs = fz.rope_cs + (size_t)pos * half * 2;
+    const float* kin = fz.k + ((size_t)r * fz.nkv + kvh) * HD;
+    const float* vin = fz.v + ((size_t)r * fz.nkv + kvh) * HD;
+    const bool first = h == kvh * group;
+    if (lane < half) {
+      const float cv = cs[2 * lane], sv = cs[2 * lane + 1];
+      auto rotate = [&](const float* src, float& o1, float& o2) {
+        const float x1 = src[lane], x2 = src[lane + half];
+        const float t1 = x1 * cv;
+        const float nx2 = -x2;
+        const float t2 = nx2 * sv;
+        const float t3 = x2 * cv;
+        const float t4 = x1 * sv;
+        o1 = t1 + t2;
+        o2 = t3 + t4;
+      };
+      float o1, o2;
+      rotate(qv, o1, o2);
+      sq[lane] = o1;
+      sq[lane + half] = o2;
+      rotate(kin, o1, o2);
+      kself[lane] = o1;
+      kself[lane + half] = o2;
+      if (first) {
+        kb[(size_t)lane * max_pos + pos] = o1;
+        kb[(size_t)(lane + half) * max_pos + pos] = o2;
+      }
+    }
+#pragma unroll
+    for (uint32_t d = 0; d < HD; d += 64) {
+      const float vv = vin[d + lane];
+      vself[d + lane] = vv;
+      if (first) vb[(size_t)(d + lane) * max_pos + pos] = vv;
+    }
+  } else {
+#pragma unroll
+    for (uint32_t d = 0; d < HD; d += 64) sq[d + lane] = qv[d + lane];
+  }
+  wave_lds_sync();
+  float m = -__builtin_inff();
+  for (uint32_t j0 = 0; j0 < len; j0 += 64) {
+    const uint32_t j = j0 + lane, jl = j < lc ? j : 0;
+    const bool self = FUSE && pos < j0 + 64;  // the round that holds pos
+    float acc = 0.0f;
+#pragma unroll
+    for (uint32_t d0 = 0; d0 < HD; d0 += 64) {
+      float kv[64];
+#pragma unroll
+      for (uint32_t i = 0; i < 64; ++i) kv[i] = kb[(size_t)(d0 + i) * max_pos + jl];
+      if (self) {
+#pragma unroll
+        for (uint32_t i = 0; i < 64; i += 4) {
+          const v4 k4 = *reinterpret_cast<const v4*>(kself + d0 + i);
+#pragma unroll
+          for (uint32_t e = 0; e < 4; ++e) kv[i + e] = j == pos ? k4[e] : kv[i + e];
+        }
+      }
+#pragma unroll
+      for (uint32_t i = 0; i < 64; i += 4) {
+        const v4 q4 = *reinterpret_cast<const v4*>(sq + d0 + i);
+#pragma unroll
+        for (uint32_t e = 0; e < 4; ++e) {
+          const float p = q4[e] * kv[i + e];
+          acc = acc + p;
+        }
+      }
+    }
+    const float sc = acc * scale;
+    if (j < len) {
+      ss[j] = sc;
+      m = sc > m ? sc : m;
+    }
+  }
+#pragma unroll
+  for (uint32_t off = 32; off > 0; off >>= 1) {
+    const float o = __shfl_xor(m, off, 64);
+    m = o > m ? o : m;
+  }
+  wave_lds_sync();
+  // the largest non-NaN score; a NaN at position 0 wins with its own bits
+  const float s0 = ss[0];
+  const float mx = s0 != s0 ? s0 : m;
+  wave_lds_sync();
+  for (uint32_t j = lane; j < len; j += 64) {
+    const float dlt = ss[j] - mx;
+    ss[j] = exp_pinned(dlt);
+  }
+  wave_lds_sync();
+  const float den = chain_lds(ss, len, 0.0f);
+  wave_lds_sync();
+  for (uint32_t j = lane; j < len; j += 64) {
+    const float pj = ss[j] / den;
+    ss[j] = pj;
+  }
+  wave_lds_sync();
+#pragma unroll
+  for (uint32_t x = 0; x < HD / 64; ++x) {
+    const uint32_t d = 64 * x + lane;
+    const float* vr = vb + (size_t)d * max_pos;
+    float acc = 0.0f;
+    uint32_t j = 0;
+    for (; j + 16 <= lc; j += 16) {
+      v4 v[4], p4[4];
+#pragma unroll
+      for (uint32_t e = 0; e < 4; ++e) v[e] = *reinterpret_cast<const v4*>(vr + j + 4 * e);
+#pragma unroll
+      for (uint32_t e = 0; e < 4; ++e) p4[e] = *reinterpret_cast<const v4*>(ss + j + 4 * e);
+#pragma unroll
+      for (uint32_t e = 0; e < 4; ++e)
+#pragma unroll
+        for (uint32_t c = 0; c < 4; ++c) {
+          const float p = p4[e][c] * v[e][c];
+          acc = acc + p;
+        }
+    }
+    for (; j < lc; j += 4) {  // up to 3 positions past lc are read, not added
+      const v4 v = *reinterpret_cast<const v4*>(vr + j);
+#pragma unroll
+      for (uint32_t c = 0; c < 4; ++c)
+        if (j + c < lc) {
+          const float p = ss[j + c] * v[c];
+          acc = acc + p;
+        }
+    }
+    if (FUSE) {
+      const float p = ss[pos] * vself[d];
+      acc = acc + p;
+    }
+    out[((size_t)r * nh + h) * HD + d] = acc;
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -2579,6 +2746,34 @@ static hipError_t launch_kv(const KvPlan& kp, bool fuse, const float* q, float* 
   return hipGetLastError();
 }
 
+// k_attention_wave where the (row, head) pairs give every SIMD two waves or
+// more and no row is long (us per layer with k_attention_rows and k_rope_store
+// | here; 300 rows of 12 heads of 64: 40 positions 299 | 269, 200 349 | 341,
+// 500 477 | 462, 1500 793 | 833; 256 rows of 16 heads of 128: 637 | 582, 683 |
+// 674, 882 | 833, 1236 | 1373); false for another kernel.
+constexpr uint32_t kWaveLen = 512;
+static bool wave_attention(uint32_t n, uint32_t nh, uint32_t nkv, uint32_t hd, uint32_t max_len,
+                           bool tree, size_t* lds) {
+  const size_t ls = ((size_t)max_len + 3) / 4 * 4;
+  *lds = 4 * (3 * (size_t)hd + ls) * sizeof(float);
+  return !tree && (hd == 64 || hd == 128) && nkv != 0 && nh % nkv == 0 &&
+         (uint64_t)n * nh >= 8 * (uint64_t)device_cu_count() &&
+         (uint64_t)n * nh <= 0x7fffffffu && max_len <= kWaveLen && kv_attention_cap() != 0;
+}
+static hipError_t launch_wave(bool fuse, const float* q, float* kc, float* vc, RowsDesc rows,
+                              uint32_t max_len, uint32_t nh, uint32_t nkv, uint32_t hd,
+                              uint32_t max_pos, uint64_t seq_stride, float scale, float* out,
+                              size_t lds, const KvFuse& fz, hipStream_t st) {
+  const uint32_t ls = (max_len + 3) / 4 * 4, g = nh / nkv;
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3((rows.n * nh + 3) / 4), dim3(256), lds, st, q, kc, vc, rows,
+                       nh, g, max_pos, seq_stride, scale, out, ls, fz);
+    return hipGetLastError();
+  };
+  if (hd == 64) return fuse ? go(k_attention_wave<64, true>) : go(k_attention_wave<64, false>);
+  return fuse ? go(k_attention_wave<128, true>) : go(k_attention_wave<128, false>);
+}
+
 hipError_t launch_rope_attention_rows(const float* q, const float* k, const float* v,
                                       const float* rope_cs, RowsDesc rows, uint32_t max_len,
                                       uint32_t nh, uint32_t nkv, uint32_t hd, uint32_t max_pos,
@@ -2589,8 +2784,13 @@ hipError_t launch_rope_attention_rows(const float* q, const float* k, const floa
   KvPlan kp;
   hipError_t e = kv_plan(rows.n, nh, nkv, hd, max_len, &kp);
   if (e != hipSuccess) return e;
-  if (!kp.C) return hipErrorNotSupported;
   const KvFuse fz{k, v, rope_cs, nkv};
+  if (!kp.C) {
+    size_t lds;
+    if (!wave_attention(rows.n, nh, nkv, hd, max_len, tree, &lds)) return hipErrorNotSupported;
+    return launch_wave(true, q, kc, vc, rows, max_len, nh, nkv, hd, max_pos, seq_stride, scale,
+                       out, lds, fz, st);
+  }
   return launch_kv(kp, true, q, kc, vc, rows, nh, hd, max_pos, seq_stride, scale, out, tree, fz,
                    st);
 }
@@ -2614,6 +2814,10 @@ hipError_t launch_attention_rows(const float* q, const float* kc, const float* v
     if (e != hipSuccess) return e;
     if (kp.C) return launch_kv(kp, false, q, const_cast<float*>(kc), const_cast<float*>(vc),
                                rows, nh, hd, max_pos, seq_stride, scale, out, tree, KvFuse{}, st);
+    size_t lds;
+    if (wave_attention(rows.n, nh, nkv, hd, max_len, tree, &lds))
+      return launch_wave(false, q, const_cast<float*>(kc), const_cast<float*>(vc), rows, max_len,
+                         nh, nkv, hd, max_pos, seq_stride, scale, out, lds, KvFuse{}, st);
   }
   // Otherwise, few rows: one head per workgroup, for the most workgroups.
   // Many rows: the most heads of one KV head (a divisor of the group) whose

@@ -8,8 +8,9 @@ vector-unit kernel (CIS2_BGEMM16=0) and the oracle.  Prefill attention
 (k_attention_tiles): every number of heads per item, runs that end inside a
 tile, lengths around the 16-, 64- and 256-position steps, a cache end inside
 a 16-position group, V rows with infinities and NaN past a row's own
-position; against the per-row kernel (CIS2_ATT_TILES=0) and the oracle.  The
-arithmetic is pinned, so there is no tolerance."""
+position; against the per-row kernel (CIS2_ATT_TILES=0) and the oracle.
+Attention of many decode rows (k_attention_wave).  The arithmetic is pinned,
+so there is no tolerance."""
 import os
 
 import numpy as np
@@ -123,6 +124,37 @@ def test_attention_tiles_bits(nh, nkv, hd, copies):
     for p, r in enumerate(rows):
         assert np.array_equal(o.forward(p, int(tok[r])).view(np.uint32),
                               out["1"][r].view(np.uint32)), p
+
+
+@pytest.mark.parametrize("nh,nkv,hd", [(3, 1, 64), (2, 2, 64), (2, 1, 128), (5, 5, 128)])
+@pytest.mark.parametrize("pos", [0, 2, 63, 64, 130])
+def test_attention_wave_bits(nh, nkv, hd, pos):
+    """Decode rows of so many sequences that a wave takes each (row, head),
+    RoPE and cache stores in the same launch: logits equal to the
+    one-workgroup kernel's (CIS2_ATT_KV=0) for this step and the next, which
+    reads what the first one stored, and to the oracle's."""
+    spec = heads_spec(nh, nkv, hd)
+    n = 2100 // nh
+    w = artifacts.Weights(spec, 8)
+    m = Cis2Model(spec, w, max_pos=pos + 2, max_seqs=n)
+    tok = np.random.default_rng(4).integers(0, spec.vocab, (n, pos + 2)).astype(np.uint32)
+    out = {}
+    for v in ("0", "256"):
+        os.environ["CIS2_ATT_KV"] = v
+        try:
+            if pos:
+                m.forward_rows(np.repeat(np.arange(n), pos), np.tile(np.arange(pos), n),
+                               tok[:, :pos].reshape(-1), want_logits=False)
+            out[v] = [m.forward_rows(np.arange(n), np.full(n, p), tok[:, p])[0]
+                      for p in (pos, pos + 1)]
+        finally:
+            del os.environ["CIS2_ATT_KV"]
+    for a, b in zip(out["0"], out["256"]):
+        assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+    o = O.OracleModel(spec, w, max_pos=pos + 2, reduction=0)
+    for p in range(pos + 2):
+        want = o.forward(p, int(tok[n - 1, p]))
+    assert np.array_equal(want.view(np.uint32), out["256"][1][n - 1].view(np.uint32))
 
 
 def test_attention_tiles_later_rows_do_not_leak():
