@@ -260,6 +260,92 @@ __global__ __launch_bounds__(256) void k_rmsnorm(const float* x, const float* __
   }
 }
 
+// The same for n a multiple of 4: a workgroup takes rpw vectors (rpw rows of
+// n + 4 floats of LDS), one chain per lane of wave 0, so that a vector costs a
+// lane and not a workgroup.  Tree order: the blocks' tree32 sums by all threads,
+// then the lanes fold them.
+// What bounds it: memory, once the chains of four or more workgroups per CU
+// overlap (18,000 x 576: 20 us, 58 us with a workgroup per vector), and one
+// chain's latency below that (544 x 576: 7.4 us, 8.0).
+__global__ __launch_bounds__(256) void k_rmsnorm_many(const float* x,  // may be out
+                                                      const float* __restrict__ w, float eps,
+                                                      uint32_t n, uint32_t nvec, uint32_t rpw,
+                                                      float* out, uint32_t tree) {
+  extern __shared__ float4 sm4[];
+  __shared__ float s_inv[64];
+  const uint32_t v0 = blockIdx.x * rpw, nr = min(rpw, nvec - v0), t = threadIdx.x;
+  const uint32_t n4 = n / 4, S4 = n4 + 1;  // row stride in 16-byte groups
+  const float4* xv = reinterpret_cast<const float4*>(x + (size_t)v0 * n);
+  float4* ov = reinterpret_cast<float4*>(out + (size_t)v0 * n);
+  const float4* wv = reinterpret_cast<const float4*>(w);
+  for (uint32_t i = t; i < nr * n4; i += 256) {
+    const float4 v = xv[i];
+    const uint32_t r = i / n4;
+    sm4[r * S4 + i - r * n4] = make_float4(v.x * v.x, v.y * v.y, v.z * v.z, v.w * v.w);
+  }
+  __syncthreads();
+  const uint32_t nb = (n + 31) / 32;
+  float* part = reinterpret_cast<float*>(sm4 + (size_t)rpw * S4);  // tree: [rpw][nb]
+  if (tree) {
+    for (uint32_t i = t; i < nr * nb; i += 256) {
+      const uint32_t r = i / nb, b = i - r * nb;
+      const float* sq = reinterpret_cast<const float*>(sm4 + r * S4) + 32 * b;
+      float l[32];
+#pragma unroll
+      for (uint32_t k = 0; k < 32; ++k) l[k] = 32 * b + k < n ? sq[k] : 0.0f;
+      part[r * nb + b] = tree32(l);
+    }
+    __syncthreads();
+  }
+  if (t < nr) {
+    float acc = 0.0f;
+    if (tree) {
+      for (uint32_t b = 0; b < nb; ++b) acc = acc + part[t * nb + b];
+    } else {
+      // eight groups' reads go out before the current eight are added
+      const float4* p = sm4 + t * S4;
+      float4 a[8], c[8];
+      auto ld = [&](float4 (&d)[8], uint32_t g) {
+#pragma unroll
+        for (uint32_t k = 0; k < 8; ++k) d[k] = p[min(g + k, n4 - 1)];
+      };
+      auto add = [&](const float4 (&d)[8], uint32_t g) {
+#pragma unroll
+        for (uint32_t k = 0; k < 8; ++k)
+          if (g + k < n4) {
+            acc = acc + d[k].x;
+            acc = acc + d[k].y;
+            acc = acc + d[k].z;
+            acc = acc + d[k].w;
+          }
+      };
+      ld(a, 0);
+      for (uint32_t g = 0; g < n4; g += 16) {
+        ld(c, g + 8);
+        add(a, g);
+        ld(a, g + 16);
+        add(c, g + 8);
+      }
+    }
+    const float mean = acc / (float)n;
+    const float arg = mean + eps;
+    s_inv[t] = rsqrt_cr(arg);
+  }
+  __syncthreads();
+  for (uint32_t i = t; i < nr * n4; i += 256) {
+    const uint32_t r = i / n4;
+    const float4 v = xv[i], g = wv[i - r * n4];
+    const float inv = s_inv[r];
+    float sx;
+    float4 y;
+    sx = v.x * inv; y.x = sx * g.x;
+    sx = v.y * inv; y.y = sx * g.y;
+    sx = v.z * inv; y.z = sx * g.z;
+    sx = v.w * inv; y.w = sx * g.w;
+    ov[i] = y;
+  }
+}
+
 __global__ void k_copy16(const float4* __restrict__ src, float4* __restrict__ dst, uint64_t n) {
   for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
        i += (uint64_t)gridDim.x * blockDim.x)
@@ -285,6 +371,17 @@ hipError_t launch_take_word(uint32_t* word, uint32_t* out, hipStream_t s) {
 hipError_t launch_rmsnorm(const float* x, const float* w, float eps, uint32_t n,
                           uint32_t nvec, float* out, hipStream_t s, bool tree) {
   if (n == 0 || n > 8192) return hipErrorInvalidValue;  // LDS: squares, partials, scalars
+  if (n % 4 == 0) {
+    // as many vectors per workgroup as 40 KB of squares and a wave's lanes
+    // hold, fewer where that would leave CUs without a workgroup
+    const size_t per = (n + 4 + (n + 31) / 32) * sizeof(float);
+    const uint32_t ncu = (uint32_t)device_cu_count();
+    uint32_t rpw = 64;
+    while (rpw > 1 && (rpw * per > 40 * 1024 || nvec / rpw < ncu)) rpw /= 2;
+    hipLaunchKernelGGL(k_rmsnorm_many, dim3((nvec + rpw - 1) / rpw), dim3(256), rpw * per, s, x, w,
+                       eps, n, nvec, rpw, out, tree ? 1u : 0u);
+    return hipGetLastError();
+  }
   const size_t shmem = (n + (n + 31) / 32) * sizeof(float);
   hipLaunchKernelGGL(k_rmsnorm, dim3(nvec), dim3(256), shmem, s, x, w, eps, n, out,
                      tree ? 1u : 0u);

@@ -102,6 +102,12 @@ hipError_t launch_attention_tiles(const float* q, const float* kc, const float* 
                                   uint32_t nh, uint32_t nkv, uint32_t hd, uint32_t max_pos,
                                   uint64_t seq_stride, float scale, float* out, float* scratch,
                                   hipStream_t st);
+// launch_rope_store_rows for the rows of the tiles (k is not rotated in
+// place; attention_tiles_supported shapes).
+hipError_t launch_rope_store_tiles(float* q, const float* k, const float* v, const float* rope_cs,
+                                   const AttTile* tiles, uint32_t ntiles, uint32_t nh,
+                                   uint32_t nkv, uint32_t hd, uint32_t max_pos, float* kc,
+                                   float* vc, uint64_t seq_stride, hipStream_t st);
 // dst[i] = src[idx[i]] rows of `width` floats, i < n.
 hipError_t launch_gather_rows(const float* src, const uint32_t* idx, uint32_t n, uint32_t width,
                               float* dst, hipStream_t st);

@@ -600,9 +600,14 @@ int forward_rows(cis2_ctx* c, uint32_t n, const uint32_t* d_tok, uint32_t max_le
     if (fe != hipErrorNotSupported) {
       LAUNCH(fe, "rows rope + attention");
     } else {
-      LAUNCH(launch_rope_store_rows(b.q, b.k, b.v, c->rope_cs, rd, f.n_heads, f.n_kv_heads, hd,
-                                    f.max_pos, kc, vc, seq_stride, s),
-             "rows rope");
+      if (ntiles)
+        LAUNCH(launch_rope_store_tiles(b.q, b.k, b.v, c->rope_cs, b.tiles, ntiles, f.n_heads,
+                                       f.n_kv_heads, hd, f.max_pos, kc, vc, seq_stride, s),
+               "rows rope tiles");
+      else
+        LAUNCH(launch_rope_store_rows(b.q, b.k, b.v, c->rope_cs, rd, f.n_heads, f.n_kv_heads, hd,
+                                      f.max_pos, kc, vc, seq_stride, s),
+               "rows rope");
       if (ntiles)
         LAUNCH(launch_attention_tiles(b.q, kc, vc, b.tiles, ntiles, max_len, f.n_heads,
                                       f.n_kv_heads, hd, f.max_pos, seq_stride, c->scale, b.att,
