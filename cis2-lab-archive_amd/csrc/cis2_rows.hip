@@ -2602,7 +2602,11 @@ static bool chain_gemm_fits(const BgemmSeg* segs, uint32_t nseg, uint32_t n, con
 // n = 64 8.6 | 12.8 | 35.4, n = 544 23.3 | 16.8 | 35.7, n = 16384 518 | 254 |
 // 188; gate and up of 3072 x 1024 at n = 16384 8254 | 3635 | 3293.)
 enum class MgemmTile { none, small, large };
-static MgemmTile mgemm_tile(const BgemmSeg* segs, uint32_t nseg, uint32_t n, bool dual,
+struct MgemmPlan {
+  MgemmTile tile;
+  double none_ns, best_ns;  // per k, without and with the matrix cores
+};
+static MgemmPlan mgemm_plan(const BgemmSeg* segs, uint32_t nseg, uint32_t n, bool dual,
                             uint32_t ncu) {
   uint64_t t16 = 0, t32 = 0, t64 = 0;  // W tiles of 16, 32 (16 x 64 rows) and 64 rows
   const uint32_t sm = n <= 16 && !dual ? 64 : 32, sn = n <= 16 && !dual ? 16 : 32;
@@ -2618,8 +2622,20 @@ static MgemmTile mgemm_tile(const BgemmSeg* segs, uint32_t nseg, uint32_t n, boo
   const double t0 = std::max(10.5, 7.5 * per_cu(t16, 16)) * two;
   const double ts = std::max(19.0, 10.5 * per_cu(t32, sn) + 2.0) * two;
   const double tl = std::max(57.0, 37.5 * per_cu(t64, 64));
-  if (t0 <= ts && t0 <= tl) return MgemmTile::none;
-  return ts <= tl ? MgemmTile::small : MgemmTile::large;
+  if (t0 <= ts && t0 <= tl) return {MgemmTile::none, t0, t0};
+  return {ts <= tl ? MgemmTile::small : MgemmTile::large, t0, std::min(ts, tl)};
+}
+
+bool bgemm_norm_apart(const BgemmSeg* segs, uint32_t nseg, uint32_t n, const BgemmOpts& o) {
+  if (n == 0 || nseg == 0 || nseg > kMaxSegs) return false;
+  const uint32_t ncu = (uint32_t)device_cu_count();
+  if (o.tree || !bgemm16_allowed()) return n > kFuseNormRows;
+  if (chain_gemm_fits(segs, nseg, n, o, ncu)) return false;
+  // the fused norm costs a chain of the row inside the launch (about 6 ns per
+  // k), the separate one a launch of 7 us: 960 x 576, us, fused | apart:
+  // 64 rows 12.2 | 19.8, 130 rows 19 | 20, 256 rows 22 | 20.5
+  const MgemmPlan p = mgemm_plan(segs, nseg, n, o.W2 != nullptr, ncu);
+  return (p.none_ns + 6.0) * segs[0].K > p.best_ns * segs[0].K + 7000.0;
 }
 
 hipError_t launch_bgemm_multi(const BgemmSeg* segs, uint32_t nseg, uint32_t n,
@@ -2645,7 +2661,7 @@ hipError_t launch_bgemm_multi(const BgemmSeg* segs, uint32_t nseg, uint32_t n,
                       : launch_chain_gemm<false, false>(segs, nseg, n, o, st);
     }
     if (!o.norm_w) {
-      switch (mgemm_tile(segs, nseg, n, o.W2 != nullptr, (uint32_t)ncu)) {
+      switch (mgemm_plan(segs, nseg, n, o.W2 != nullptr, (uint32_t)ncu).tile) {
         case MgemmTile::large:
           return o.W2 ? launch_mgemm<true, 2, 2, 2, 2, 32, 3, 1>(segs, nseg, n, o.W2, st)
                       : launch_mgemm<false, 2, 2, 2, 2, 32, 3, 1>(segs, nseg, n, o.W2, st);

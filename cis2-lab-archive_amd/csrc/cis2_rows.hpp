@@ -46,6 +46,11 @@ struct BgemmOpts {
 hipError_t launch_bgemm_multi(const BgemmSeg* segs, uint32_t nseg, uint32_t n,
                               const BgemmOpts& o, hipStream_t st);
 
+// Whether a launch with o.norm_w is better replaced by the norm as a launch of
+// its own and the GEMM over its output.
+constexpr uint32_t kFuseNormRows = 256;  // tree order: fused up to here
+bool bgemm_norm_apart(const BgemmSeg* segs, uint32_t nseg, uint32_t n, const BgemmOpts& o);
+
 // Per-row device descriptors: seq[r], pos[r], tok[r].
 struct RowsDesc {
   const uint32_t* seq;

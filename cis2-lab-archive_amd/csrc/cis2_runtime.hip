@@ -540,10 +540,6 @@ int rows_reserve(cis2_ctx* c, uint32_t n, uint32_t nl) {
 // each other causally.  max_len = 1 + the largest position.  The final
 // norm, LM head and argmax run for the nl rows listed in rows.lrows:
 // logits[i] and arg[i] belong to row lrows[i].
-// Row counts up to which forward_rows applies the layer norms inside the
-// projections that read them.
-constexpr uint32_t kFuseNormRows = 256;
-
 // The logits and argmax go to b.logits / b.arg unless `logits` / `arg` name
 // other buffers of at least nl rows.
 // ntiles > 0: the attention runs over the ntiles tiles in c->rows.tiles
@@ -562,31 +558,27 @@ int forward_rows(cis2_ctx* c, uint32_t n, const uint32_t* d_tok, uint32_t max_le
   const size_t per = (size_t)KV * f.max_pos;           // one layer's K (or V) of one sequence
   const uint64_t seq_stride = (uint64_t)f.n_layers * 2 * per;
   LAUNCH(launch_embed_rows(c->embed, rd, H, f.vocab, b.h, c->d_err, s), "rows embed");
-  // for few rows (decode steps) the RMSNorms run inside the launches that
-  // consume them; each workgroup then repeats the norm chain of its rows,
-  // which is latency hidden by the launch it saves only while the grid is
-  // small
-  const bool fuse_norm = n <= kFuseNormRows;
   for (uint32_t l = 0; l < f.n_layers; ++l) {
     const Layer& Ly = c->L[l];
     float* kc = c->kv + (size_t)l * 2 * per;
     float* vc = kc + per;
-    // q, k and v in one launch over norm1(h): the norm inside the launch
-    // for few rows, as its own pass for many
+    // q, k and v in one launch over norm1(h).  For few rows (decode steps)
+    // the RMSNorms run inside the launches that consume them: each workgroup
+    // then repeats the norm chain of its rows, which is latency hidden by the
+    // launch it saves only while the grid is small.
     BgemmOpts o1;
     o1.tree = tree;
-    const float* xin = b.h;
-    if (fuse_norm) {
-      o1.norm_w = Ly.ln1;
-      o1.eps = f.eps;
-    } else {
+    o1.norm_w = Ly.ln1;
+    o1.eps = f.eps;
+    BgemmSeg qkv[3] = {
+        {Ly.wq, QD, H, c->Rq, b.h, H, b.q, QD, Ly.bq, 0, Ly.bq ? kEpiBias : kEpiNone},
+        {Ly.wk, KV, H, c->Rq, b.h, H, b.k, KV, Ly.bk, 0, Ly.bk ? kEpiBias : kEpiNone},
+        {Ly.wv, KV, H, c->Rq, b.h, H, b.v, KV, Ly.bv, 0, Ly.bv ? kEpiBias : kEpiNone}};
+    if (bgemm_norm_apart(qkv, 3, n, o1)) {
       LAUNCH(launch_rmsnorm(b.h, Ly.ln1, f.eps, H, n, b.x, s, tree), "rows norm1");
-      xin = b.x;
+      for (BgemmSeg& g : qkv) g.X = b.x;
+      o1.norm_w = nullptr;
     }
-    const BgemmSeg qkv[3] = {
-        {Ly.wq, QD, H, c->Rq, xin, H, b.q, QD, Ly.bq, 0, Ly.bq ? kEpiBias : kEpiNone},
-        {Ly.wk, KV, H, c->Rq, xin, H, b.k, KV, Ly.bk, 0, Ly.bk ? kEpiBias : kEpiNone},
-        {Ly.wv, KV, H, c->Rq, xin, H, b.v, KV, Ly.bv, 0, Ly.bv ? kEpiBias : kEpiNone}};
     LAUNCH(launch_bgemm_multi(qkv, 3, n, o1, s), "rows qkv");
     if (Ly.qn) LAUNCH(launch_rmsnorm(b.q, Ly.qn, f.eps, hd, n * f.n_heads, b.q, s, tree), "rows q_norm");
     if (Ly.kn) LAUNCH(launch_rmsnorm(b.k, Ly.kn, f.eps, hd, n * f.n_kv_heads, b.k, s, tree), "rows k_norm");
@@ -621,19 +613,18 @@ int forward_rows(cis2_ctx* c, uint32_t n, const uint32_t* d_tok, uint32_t max_le
     const BgemmSeg so{Ly.wo, H, QD, c->Ro, b.att, QD, b.h2, H, b.h, H, kEpiResidual};
     LAUNCH(launch_bgemm(so, n, tree, s), "rows o_proj");
     std::swap(b.h, b.h2);
-    // gate and up as two chains per thread, silu(gate) * up stored
+    // gate and up in one launch, silu(gate) * up stored
     BgemmOpts o2;
     o2.tree = tree;
     o2.W2 = Ly.wu;
-    const float* x2 = b.h;
-    if (fuse_norm) {
-      o2.norm_w = Ly.ln2;
-      o2.eps = f.eps;
-    } else {
+    o2.norm_w = Ly.ln2;
+    o2.eps = f.eps;
+    BgemmSeg sg{Ly.wg, I, H, c->Rg, b.h, H, b.hid, I, nullptr, 0, kEpiNone};
+    if (bgemm_norm_apart(&sg, 1, n, o2)) {
       LAUNCH(launch_rmsnorm(b.h, Ly.ln2, f.eps, H, n, b.x, s, tree), "rows norm2");
-      x2 = b.x;
+      sg.X = b.x;
+      o2.norm_w = nullptr;
     }
-    const BgemmSeg sg{Ly.wg, I, H, c->Rg, x2, H, b.hid, I, nullptr, 0, kEpiNone};
     LAUNCH(launch_bgemm_multi(&sg, 1, n, o2, s), "rows gate_up");
     const BgemmSeg sd{Ly.wd, H, I, c->Rd, b.hid, I, b.h2, H, b.h, H, kEpiResidual};
     LAUNCH(launch_bgemm(sd, n, tree, s), "rows down");
