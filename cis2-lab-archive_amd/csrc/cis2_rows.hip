@@ -798,15 +798,16 @@ __global__ __launch_bounds__((ChainCfg<DUAL, NORM>::T), 3) void k_chain_gemm(Bge
 }
 
 // ---------------------------------------------------------------------------
-// Batched GEMM with the products formed by the matrix cores (sequential
-// order, any block height R).  One v_mfma_f32_16x16x1_4b_f32 multiplies four
+// Batched GEMM with the products formed by the matrix cores (either order,
+// any block height R).  One v_mfma_f32_16x16x1_4b_f32 multiplies four
 // pairs of 16-vectors; given the 16 W rows and 16 X rows of a tile at four
 // consecutive k, and -0 as the addend, each of its 4 x 256 results is one
 // correctly rounded product W[m][k] * X[b][k] (x + (-0) = x for every x, so
 // the sign of a zero product survives; flushing and NaN bits are those of
 // v_mul_f32).  All four blocks leave a given output in the same lane, so the
 // vector units only add: acc = acc + p, k ascending, the strict chain of
-// k_bgemm (code/cis2-fp/src/main.rs:228-243, math.rs:40-48).
+// k_bgemm (code/cis2-fp/src/main.rs:228-243, math.rs:40-48).  In tree order
+// they add pairs of a lane's products instead, the same number of adds.
 // ---------------------------------------------------------------------------
 typedef float f16v __attribute__((ext_vector_type(16)));
 
@@ -825,6 +826,55 @@ __device__ __forceinline__ f16v minus_zeros() {
   for (uint32_t i = 0; i < 16; ++i) v[i] = z;
   return v;
 }
+
+// Step x of 16 k over NT tiles: its tile and its four k.  Tree order takes a
+// tile's four steps in turn, so that only one tile's partial sums are open.
+template <uint32_t NT, bool TREE>
+constexpr __host__ __device__ uint32_t mtile_s(uint32_t x) { return TREE ? x / 4 : x % NT; }
+template <uint32_t NT, bool TREE>
+constexpr __host__ __device__ uint32_t mtile_k(uint32_t x) { return TREE ? x % 4 : x / NT; }
+
+// The adds of NT tiles.  add(): products4's p, for k = 4q .. 4q + 3 of every
+// 32, into tile s: k ascending, or in tree order (math.rs:60-125) the pairs'
+// sums of the 32, whose total acc takes (zeros before the first step: acc is
+// +0 and stays so).
+template <uint32_t NT, bool TREE>
+struct ChainSums {
+  float t4[4] = {}, t8[4] = {}, t16[TREE ? NT : 1][4] = {};
+  __device__ __forceinline__ void add(float (&acc)[NT][4], uint32_t s, uint32_t q, const f16v& p) {
+    if constexpr (TREE) {
+#pragma unroll
+      for (uint32_t r = 0; r < 4; ++r) {
+        const float lo = p[r] + p[4 + r], hi = p[8 + r] + p[12 + r];
+        const float v4k = lo + hi;
+        if (q % 2 == 0) {
+          t4[r] = v4k;
+          continue;
+        }
+        const float v8k = t4[r] + v4k;
+        if (q % 4 == 1) {
+          t8[r] = v8k;
+          continue;
+        }
+        const float v16k = t8[r] + v8k;
+        if (q == 3) {
+          t16[s][r] = v16k;
+          continue;
+        }
+        const float v32k = t16[s][r] + v16k;
+        acc[s][r] = acc[s][r] + v32k;
+      }
+      float* o = q == 7 ? acc[s] : (q == 3 ? t16[s] : (q % 2 ? t8 : t4));
+      asm volatile("" : "+v"(o[0]), "+v"(o[1]), "+v"(o[2]), "+v"(o[3]));
+    } else {
+#pragma unroll
+      for (uint32_t b = 0; b < 4; ++b)
+#pragma unroll
+        for (uint32_t r = 0; r < 4; ++r) acc[s][r] = acc[s][r] + p[4 * b + r];
+      asm volatile("" : "+v"(acc[s][0]), "+v"(acc[s][1]), "+v"(acc[s][2]), "+v"(acc[s][3]));
+    }
+  }
+};
 
 struct MgemmArgs {
   BgemmSeg s[kMaxSegs];
@@ -851,8 +901,44 @@ struct MgemmArgs {
 // wave's 16-byte read gives lane l (row l % 16, u = l / 16) its operands of
 // four products4.  A thread stages whole (row, 16 k) pieces: four 16-byte
 // loads, transposed by register naming.  Past K the pieces hold -0 for W and
-// +0 for X: their products are -0, which no sum notices.  Chunk c + PF is
+// +0 for X: their products are -0, which no sum notices (tree order: zeros, as
+// its last block of 32 has them).  Chunk c + PF is
 // loaded into registers while chunk c is computed.
+// Stores a lane's outputs m .. m + 3 of X row `row`: sums y, with y2 those of
+// the second matrix (DUAL).
+template <bool DUAL>
+__device__ __forceinline__ void mgemm_store(const MgemmArgs& a, const BgemmSeg& g, uint32_t m,
+                                            uint32_t row, const float (&acc)[4],
+                                            const float (&acc2)[4]) {
+  if (row >= a.n || m >= g.M) return;
+  float y[4];
+#pragma unroll
+  for (uint32_t r = 0; r < 4; ++r) y[r] = acc[r];
+  float* yp = g.Y + (size_t)row * g.ldy + m;
+  if (DUAL) {
+#pragma unroll
+    for (uint32_t r = 0; r < 4; ++r) {
+      const float sg = silu_pinned(y[r]);
+      y[r] = sg * acc2[r];
+    }
+  }
+  const float* ad = nullptr;
+  if (!DUAL && g.epi == kEpiBias) ad = g.add + m;
+  if (!DUAL && g.epi == kEpiResidual) ad = g.add + (size_t)row * g.ldadd + m;
+  if (a.vec) {
+    if (ad) {
+      const v4 z = *reinterpret_cast<const v4*>(ad);
+#pragma unroll
+      for (uint32_t r = 0; r < 4; ++r) y[r] = g.epi == kEpiBias ? y[r] + z[r] : z[r] + y[r];
+    }
+    *reinterpret_cast<v4*>(yp) = v4{y[0], y[1], y[2], y[3]};
+  } else {
+#pragma unroll
+    for (uint32_t r = 0; r < 4; ++r)
+      if (m + r < g.M) yp[r] = ad ? (g.epi == kEpiBias ? y[r] + ad[r] : ad[r] + y[r]) : y[r];
+  }
+}
+
 template <bool DUAL, uint32_t SM, uint32_t SN, uint32_t WM, uint32_t WN, uint32_t KC>
 struct MgemmCfg {
   static constexpr uint32_t BM = 16 * SM * WM / (DUAL ? 2 : 1);  // W rows per tile
@@ -864,7 +950,7 @@ struct MgemmCfg {
   static_assert(WM * WN == 4 && (!DUAL || SM % 2 == 0), "four waves");
 };
 
-template <bool DUAL, uint32_t SM, uint32_t SN, uint32_t WM, uint32_t WN, uint32_t KC,
+template <bool DUAL, bool TREE, uint32_t SM, uint32_t SN, uint32_t WM, uint32_t WN, uint32_t KC,
           uint32_t OCC, uint32_t PF>
 __global__ __launch_bounds__(256, OCC) void k_mgemm(MgemmArgs a) {
   using C = MgemmCfg<DUAL, SM, SN, WM, WN, KC>;
@@ -916,7 +1002,7 @@ __global__ __launch_bounds__(256, OCC) void k_mgemm(MgemmArgs a) {
         if (q < K4) {
           st[j][i] = src[j][(size_t)q * step[j]];
         } else {
-          const float z = isw[j] ? __int_as_float((int)0x80000000u) : 0.0f;
+          const float z = isw[j] && !TREE ? __int_as_float((int)0x80000000u) : 0.0f;
           st[j][i] = v4{z, z, z, z};
         }
       }
@@ -948,13 +1034,7 @@ __global__ __launch_bounds__(256, OCC) void k_mgemm(MgemmArgs a) {
   f16v d[2];
 #pragma unroll
   for (uint32_t i = 0; i < 16; ++i) d[1][i] = __int_as_float((int)0x80000000u);
-  auto add = [&](uint32_t s, const f16v& p) {
-#pragma unroll
-    for (uint32_t b = 0; b < 4; ++b)
-#pragma unroll
-      for (uint32_t r = 0; r < 4; ++r) acc[s][r] = acc[s][r] + p[4 * b + r];
-    asm volatile("" : "+v"(acc[s][0]), "+v"(acc[s][1]), "+v"(acc[s][2]), "+v"(acc[s][3]));
-  };
+  ChainSums<NT, TREE> sums;
   const uint32_t nc = (g.K + KC - 1) / KC;
   load(0, stage[0]);
   if (PF == 2 && nc > 1) load(KC, stage[1]);
@@ -975,15 +1055,15 @@ __global__ __launch_bounds__(256, OCC) void k_mgemm(MgemmArgs a) {
     for (uint32_t gi = 0; gi < NG; ++gi) {
       if (gi + 1 < NG) frags(gi + 1, (gi + 1) & 1);
 #pragma unroll
-      for (uint32_t m = 0; m < 4; ++m)
-#pragma unroll
-        for (uint32_t s = 0; s < NT; ++s) {
-          // products of tile s while the vector units add the tile before it
-          const uint32_t x = m * NT + s;
-          d[x & 1] = products4(fa[gi & 1][s / SN][m], fb[gi & 1][s % SN][m], nz);
-          asm volatile("" : "+v"(d[x & 1]));
-          add((s + NT - 1) % NT, d[(x + 1) & 1]);
-        }
+      for (uint32_t x = 0; x < 4 * NT; ++x) {
+        // these products while the vector units add the ones before them
+        const uint32_t m = mtile_k<NT, TREE>(x), s = mtile_s<NT, TREE>(x);
+        d[x & 1] = products4(fa[gi & 1][s / SN][m], fb[gi & 1][s % SN][m], nz);
+        asm volatile("" : "+v"(d[x & 1]));
+        const uint32_t y = (x + 4 * NT - 1) % (4 * NT);
+        sums.add(acc, mtile_s<NT, TREE>(y), 4 * ((x ? gi : gi + 1) & 1) + mtile_k<NT, TREE>(y),
+                 d[(x + 1) & 1]);
+      }
     }
     if (ci + 1 < nc) store((ci + 1) & 1, nxt);
   };
@@ -992,41 +1072,14 @@ __global__ __launch_bounds__(256, OCC) void k_mgemm(MgemmArgs a) {
     chunk(ci, stage[0], stage[PF - 1]);
     if (PF == 2 && ci + 1 < nc) chunk(ci + 1, stage[1 % PF], stage[0]);
   }
-  add(NT - 1, d[1]);
+  sums.add(acc, NT - 1, 7, d[1]);
   // epilogue: lane l holds outputs m .. m+3 of X row n
 #pragma unroll
   for (uint32_t i = 0; i < SMH; ++i)
 #pragma unroll
-    for (uint32_t j = 0; j < SN; ++j) {
-      const uint32_t m = m0 + 16 * (wm * SMH + i) + 4 * u, row = n0 + 16 * (wn * SN + j) + c16;
-      if (row >= a.n || m >= g.M) continue;
-      float y[4];
-#pragma unroll
-      for (uint32_t r = 0; r < 4; ++r) y[r] = acc[i * SN + j][r];
-      float* yp = g.Y + (size_t)row * g.ldy + m;
-      if (DUAL) {
-#pragma unroll
-        for (uint32_t r = 0; r < 4; ++r) {
-          const float sg = silu_pinned(y[r]);
-          y[r] = sg * acc[(SMH + i) * SN + j][r];
-        }
-      }
-      const float* ad = nullptr;
-      if (!DUAL && g.epi == kEpiBias) ad = g.add + m;
-      if (!DUAL && g.epi == kEpiResidual) ad = g.add + (size_t)row * g.ldadd + m;
-      if (a.vec) {
-        if (ad) {
-          const v4 z = *reinterpret_cast<const v4*>(ad);
-#pragma unroll
-          for (uint32_t r = 0; r < 4; ++r) y[r] = g.epi == kEpiBias ? y[r] + z[r] : z[r] + y[r];
-        }
-        *reinterpret_cast<v4*>(yp) = v4{y[0], y[1], y[2], y[3]};
-      } else {
-#pragma unroll
-        for (uint32_t r = 0; r < 4; ++r)
-          if (m + r < g.M) yp[r] = ad ? (g.epi == kEpiBias ? y[r] + ad[r] : ad[r] + y[r]) : y[r];
-      }
-    }
+    for (uint32_t j = 0; j < SN; ++j)
+      mgemm_store<DUAL>(a, g, m0 + 16 * (wm * SMH + i) + 4 * u, n0 + 16 * (wn * SN + j) + c16,
+                        acc[i * SN + j], acc[((DUAL ? SMH : 0) + i) * SN + j]);
 }
 
 // (value, index) pick of a strict-> scan from index 0 (first maximum wins;
@@ -2015,9 +2068,9 @@ __global__ __launch_bounds__(256) void k_attention_wave(
 // sequence at consecutive positions p0 .. p0+nr-1 (built on the host); a work
 // item is one tile and HPT query heads of one KV head, P = kAttQT * HPT
 // (row, head) pairs (pair a = head h * 16 + row i).  Each pair's arithmetic
-// is the per-row kernel's, in the same order (sequential reduction order
-// only), with the products of both contractions formed by the matrix cores
-// (products4, above) and the chains' adds by the vector units:
+// is the per-row kernel's, in the same order, with the products of both
+// contractions formed by the matrix cores (products4, above) and the chains'
+// adds by the vector units:
 //   scores  s_j = dot_seq(q, k_j) * scale, d ascending: A is 16 pairs of one
 //           head, B 16 positions; a wave takes 64 positions at a time, and a
 //           16-byte load per lane of 4 rows of K is the B operand of four
@@ -2035,11 +2088,16 @@ __global__ __launch_bounds__(256) void k_attention_wave(
 //           transposed between lanes there (permlane swaps).  In the groups
 //           that reach past the tile's first row's length every add is
 //           selected by j < the row's length.
+// TREE: the scores' products are added in blocks of 32 d and the denominators
+// in blocks of 32 positions (tree32); the V-mix is the same fold.
 // What bounds it: the vector and matrix units, at the GEMM's 64 cycles per
 // 1024 chain steps, and the exps (about a fifth of a head_dim-64 step).
 // 4096 rows of 16 heads of 128: 1.89 ms per layer (18 T chain steps/s),
 // 4.32 ms with operands read from LDS and multiplied by the vector units;
 // 64 ragged prompts of 16 .. 512 rows, 9 heads of 64: 0.31 ms against 1.37.
+// Tree order, us per layer with k_attention_rows | with this: one prompt of 544
+// rows 290 | 213 (9 heads of 64), 948 | 662 (16 of 128); 200 rows 143 | 135,
+// 404 | 331.
 // Workgroups walk the items with a fixed stride, the longest tiles first and
 // every other round in reverse order, each with one scratch slot, so the
 // scratch stays a few hundred MB whatever the row count; the stride is a
@@ -2079,7 +2137,7 @@ __device__ __forceinline__ void transpose4(v4& x) {
          __uint_as_float(d[1])};
 }
 
-template <uint32_t HPT, uint32_t HD>
+template <uint32_t HPT, uint32_t HD, bool TREE>
 __global__ __launch_bounds__(256, 2) void k_attention_tiles(
     const float* __restrict__ q, const float* __restrict__ kc, const float* __restrict__ vc,
     const AttTile* __restrict__ tiles, uint32_t nitem, uint32_t nh, uint32_t group,
@@ -2149,19 +2207,13 @@ __global__ __launch_bounds__(256, 2) void k_attention_tiles(
       for (uint32_t s = 0; s < NT1; ++s)
 #pragma unroll
         for (uint32_t r = 0; r < 4; ++r) acc[s][r] = 0.0f;
-      auto add = [&](uint32_t s, const f16v& p) {
-#pragma unroll
-        for (uint32_t e = 0; e < 4; ++e)
-#pragma unroll
-          for (uint32_t r = 0; r < 4; ++r) acc[s][r] = acc[s][r] + p[4 * e + r];
-        asm volatile("" : "+v"(acc[s][0]), "+v"(acc[s][1]), "+v"(acc[s][2]), "+v"(acc[s][3]));
-      };
+      ChainSums<NT1, TREE> sums;
       f16v d[2];
       d[1] = nz;
       v4 kf[2][4];
 #pragma unroll
       for (uint32_t m = 0; m < 4; ++m) kf[0][m] = kload(m);
-      auto dgroup = [&](uint32_t g, const v4 (&cur)[4], v4 (&nxt)[4]) {
+      auto dgroup = [&](uint32_t g, uint32_t odd, const v4 (&cur)[4], v4 (&nxt)[4]) {
         if (g + 1 < DG) {
 #pragma unroll
           for (uint32_t m = 0; m < 4; ++m) nxt[m] = kload(4 * (g + 1) + m);
@@ -2170,21 +2222,21 @@ __global__ __launch_bounds__(256, 2) void k_attention_tiles(
 #pragma unroll
         for (uint32_t h = 0; h < HPT; ++h) fa[h] = qf[(4 * g + u) * P + 16 * h + c16];
 #pragma unroll
-        for (uint32_t m = 0; m < 4; ++m)
-#pragma unroll
-          for (uint32_t s = 0; s < NT1; ++s) {
-            const uint32_t x = m * NT1 + s;
-            d[x & 1] = products4(fa[s / 4][m], cur[m][s % 4], nz);
-            asm volatile("" : "+v"(d[x & 1]));
-            add((s + NT1 - 1) % NT1, d[(x + 1) & 1]);
-          }
+        for (uint32_t x = 0; x < 4 * NT1; ++x) {
+          const uint32_t m = mtile_k<NT1, TREE>(x), s = mtile_s<NT1, TREE>(x);
+          d[x & 1] = products4(fa[s / 4][m], cur[m][s % 4], nz);
+          asm volatile("" : "+v"(d[x & 1]));
+          const uint32_t y = (x + 4 * NT1 - 1) % (4 * NT1);  // the products before these
+          sums.add(acc, mtile_s<NT1, TREE>(y), 4 * ((x ? odd : odd + 1) & 1) + mtile_k<NT1, TREE>(y),
+                   d[(x + 1) & 1]);
+        }
       };
 #pragma unroll 1
       for (uint32_t g = 0; g < DG; g += 2) {
-        dgroup(g, kf[0], kf[1]);
-        dgroup(g + 1, kf[1], kf[0]);
+        dgroup(g, 0, kf[0], kf[1]);
+        dgroup(g + 1, 1, kf[1], kf[0]);
       }
-      add(NT1 - 1, d[1]);
+      sums.add(acc, NT1 - 1, 7, d[1]);
       const uint32_t j = j0 + 4 * c16;
 #pragma unroll
       for (uint32_t h = 0; h < HPT; ++h)
@@ -2263,7 +2315,19 @@ __global__ __launch_bounds__(256, 2) void k_attention_tiles(
       if (wv == 0) {
         if (lane < P && live(lane)) {
           const uint32_t j0 = i * kAttTE, len = pair_len(lane);
-          if (j0 < len) den = chain_lds(es(i) + lane * ES, min(kAttTE, len - j0), den);
+          const float* ep = es(i) + lane * ES;
+          if constexpr (TREE) {
+#pragma unroll
+            for (uint32_t b = 0; b < kAttTE; b += 32)
+              if (j0 + b < len) {
+                float l[32];
+#pragma unroll
+                for (uint32_t k = 0; k < 32; ++k) l[k] = j0 + b + k < len ? ep[b + k] : 0.0f;
+                den = den + tree32(l);
+              }
+          } else if (j0 < len) {
+            den = chain_lds(ep, min(kAttTE, len - j0), den);
+          }
         }
       } else if (i + 1 < nst) {
         stage(i + 1);
@@ -2523,11 +2587,9 @@ static hipError_t launch_bgemm16(const BgemmSeg* segs, uint32_t nseg, uint32_t n
   return hipGetLastError();
 }
 
-template <bool DUAL, uint32_t SM, uint32_t SN, uint32_t WM, uint32_t WN, uint32_t KC,
-          uint32_t OCC, uint32_t PF>
-static hipError_t launch_mgemm(const BgemmSeg* segs, uint32_t nseg, uint32_t n,
-                                 const float* W2, hipStream_t st) {
-  using C = MgemmCfg<DUAL, SM, SN, WM, WN, KC>;
+// Arguments of a grid of bm x bn tiles.
+static bool mgemm_args(const BgemmSeg* segs, uint32_t nseg, uint32_t n, const float* W2,
+                       uint32_t bm, uint32_t bn, MgemmArgs* out) {
   MgemmArgs a = {};
   a.nseg = nseg;
   a.n = n;
@@ -2536,16 +2598,27 @@ static hipError_t launch_mgemm(const BgemmSeg* segs, uint32_t nseg, uint32_t n,
   for (uint32_t i = 0; i < kMaxSegs; ++i) {
     a.s[i] = segs[i < nseg ? i : 0];
     if (i < nseg) {
-      a.tile0[i + 1] = a.tile0[i] + (segs[i].M + C::BM - 1) / C::BM;
+      a.tile0[i + 1] = a.tile0[i] + (segs[i].M + bm - 1) / bm;
       if (segs[i].M % 4 || segs[i].ldy % 4 || segs[i].ldadd % 4) a.vec = 0;
     } else {
       a.tile0[i + 1] = a.tile0[nseg];
     }
   }
-  const uint64_t tiles = (uint64_t)a.tile0[nseg] * ((n + C::BN - 1) / C::BN);
-  if (tiles > 0x7fffffffu - 8) return hipErrorInvalidValue;
+  const uint64_t tiles = (uint64_t)a.tile0[nseg] * ((n + bn - 1) / bn);
+  if (tiles > 0x7fffffffu - 8) return false;
   a.tiles = (uint32_t)tiles;
-  hipLaunchKernelGGL((k_mgemm<DUAL, SM, SN, WM, WN, KC, OCC, PF>), dim3((a.tiles + 7) / 8 * 8),
+  *out = a;
+  return true;
+}
+
+template <bool DUAL, bool TREE, uint32_t SM, uint32_t SN, uint32_t WM, uint32_t WN, uint32_t KC,
+          uint32_t OCC, uint32_t PF>
+static hipError_t launch_mgemm(const BgemmSeg* segs, uint32_t nseg, uint32_t n,
+                                 const float* W2, hipStream_t st) {
+  using C = MgemmCfg<DUAL, SM, SN, WM, WN, KC>;
+  MgemmArgs a;
+  if (!mgemm_args(segs, nseg, n, W2, C::BM, C::BN, &a)) return hipErrorInvalidValue;
+  hipLaunchKernelGGL((k_mgemm<DUAL, TREE, SM, SN, WM, WN, KC, OCC, PF>), dim3((a.tiles + 7) / 8 * 8),
                      dim3(256), 0, st, a);
   return hipGetLastError();
 }
@@ -2588,26 +2661,31 @@ static bool chain_gemm_fits(const BgemmSeg* segs, uint32_t nseg, uint32_t n, con
   return wgs * ((n + 7) / 8) <= ncu;
 }
 
-// Which kernel a sequential-order GEMM without a fused norm takes.  Every
+// Which kernel a GEMM without a fused norm takes.  Every
 // form costs a time per k that depends on how many workgroups the fullest CU
 // gets; measured on the layer shapes of the three models at n = 7 .. 16384,
 // in ns per k (two figures: one matrix, gate and up):
 //   k_bgemm16 / k_bgemm  256 chains per workgroup     11 | 21 at one per CU,
 //                                                     7.7 | 14.5 each beyond
+//   k_bgemm, tree order                               18 | 36, 10.8 | 21.6
 //   k_mgemm, 32 x 32     1024 chains (2048 for two)   19 | 39, then 11 | 21 each
 //   k_mgemm, 64 x 64     4096 chains                  57, then 37.5 each
 // A small grid is bound by one wave's latency and wants many short
 // workgroups, a large one by the vector units and wants operands reused: the
 // least of the three estimates is taken.  (o projection of 576 x 576, us:
 // n = 64 8.6 | 12.8 | 35.4, n = 544 23.3 | 16.8 | 35.7, n = 16384 518 | 254 |
-// 188; gate and up of 3072 x 1024 at n = 16384 8254 | 3635 | 3293.)
+// 188; gate and up of 3072 x 1024 at n = 16384 8254 | 3635 | 3293.  Tree order,
+// us per layer, k_bgemm | 32 x 32 | 64 x 64: 30-layer shape of 576, 64 rows
+// 104 | 105 | 234, 124 rows 141 | 114 | 244, 2000 rows 1298 | 476 | 520; that
+// of 1024, 16 rows 195 | 219 | 498, 2000 rows 5908 | 2281 | 2096.)
 enum class MgemmTile { none, small, large };
 struct MgemmPlan {
   MgemmTile tile;
   double none_ns, best_ns;  // per k, without and with the matrix cores
 };
-static MgemmPlan mgemm_plan(const BgemmSeg* segs, uint32_t nseg, uint32_t n, bool dual,
+static MgemmPlan mgemm_plan(const BgemmSeg* segs, uint32_t nseg, uint32_t n, const BgemmOpts& o,
                             uint32_t ncu) {
+  const bool dual = o.W2 != nullptr;
   uint64_t t16 = 0, t32 = 0, t64 = 0;  // W tiles of 16, 32 (16 x 64 rows) and 64 rows
   const uint32_t sm = n <= 16 && !dual ? 64 : 32, sn = n <= 16 && !dual ? 16 : 32;
   for (uint32_t i = 0; i < nseg; ++i) {
@@ -2619,23 +2697,37 @@ static MgemmPlan mgemm_plan(const BgemmSeg* segs, uint32_t nseg, uint32_t n, boo
     return (double)((wt * ((n + bn - 1) / bn) + ncu - 1) / ncu);
   };
   const double two = dual ? 2.0 : 1.0;
-  const double t0 = std::max(10.5, 7.5 * per_cu(t16, 16)) * two;
+  const double t0 = (o.tree ? std::max(18.0, 10.8 * per_cu(t16, 16))
+                            : std::max(10.5, 7.5 * per_cu(t16, 16))) * two;
   const double ts = std::max(19.0, 10.5 * per_cu(t32, sn) + 2.0) * two;
   const double tl = std::max(57.0, 37.5 * per_cu(t64, 64));
   if (t0 <= ts && t0 <= tl) return {MgemmTile::none, t0, t0};
   return {ts <= tl ? MgemmTile::small : MgemmTile::large, t0, std::min(ts, tl)};
 }
 
+template <bool TREE>
+static hipError_t launch_mgemm_tile(MgemmTile tile, const BgemmSeg* segs, uint32_t nseg,
+                                    uint32_t n, const float* W2, hipStream_t st) {
+  if (tile == MgemmTile::large)
+    return W2 ? launch_mgemm<true, TREE, 2, 2, 2, 2, 32, 3, 1>(segs, nseg, n, W2, st)
+              : launch_mgemm<false, TREE, 2, 2, 2, 2, 32, 3, 1>(segs, nseg, n, W2, st);
+  if (W2) return launch_mgemm<true, TREE, 2, 1, 2, 2, 32, 2, 2>(segs, nseg, n, W2, st);
+  // up to 16 rows: 64 x 16 tiles (the LM head at n = 16: 26 against 41 us)
+  return n <= 16 ? launch_mgemm<false, TREE, 1, 1, 4, 1, 64, 2, 1>(segs, nseg, n, W2, st)
+                 : launch_mgemm<false, TREE, 1, 1, 2, 2, 64, 3, 2>(segs, nseg, n, W2, st);
+}
+
 bool bgemm_norm_apart(const BgemmSeg* segs, uint32_t nseg, uint32_t n, const BgemmOpts& o) {
   if (n == 0 || nseg == 0 || nseg > kMaxSegs) return false;
   const uint32_t ncu = (uint32_t)device_cu_count();
-  if (o.tree || !bgemm16_allowed()) return n > kFuseNormRows;
-  if (chain_gemm_fits(segs, nseg, n, o, ncu)) return false;
+  if (!bgemm16_allowed()) return n > kFuseNormRows;
+  if (!o.tree && chain_gemm_fits(segs, nseg, n, o, ncu)) return false;
   // the fused norm costs a chain of the row inside the launch (about 6 ns per
   // k), the separate one a launch of 7 us: 960 x 576, us, fused | apart:
-  // 64 rows 12.2 | 19.8, 130 rows 19 | 20, 256 rows 22 | 20.5
-  const MgemmPlan p = mgemm_plan(segs, nseg, n, o.W2 != nullptr, ncu);
-  return (p.none_ns + 6.0) * segs[0].K > p.best_ns * segs[0].K + 7000.0;
+  // 64 rows 12.2 | 19.8, 130 rows 19 | 20, 256 rows 22 | 20.5; in tree order
+  // 20 ns per k (us per layer, 2 rows: 105 | 96, 146 | 134, 199 | 180)
+  const MgemmPlan p = mgemm_plan(segs, nseg, n, o, ncu);
+  return (p.none_ns + (o.tree ? 20.0 : 6.0)) * segs[0].K > p.best_ns * segs[0].K + 7000.0;
 }
 
 hipError_t launch_bgemm_multi(const BgemmSeg* segs, uint32_t nseg, uint32_t n,
@@ -2653,6 +2745,10 @@ hipError_t launch_bgemm_multi(const BgemmSeg* segs, uint32_t nseg, uint32_t n,
         segs[i].ldx != s0.ldx)
       return hipErrorInvalidValue;
   const int ncu = device_cu_count();
+  if (o.tree && !o.norm_w && bgemm16_allowed()) {
+    const MgemmTile tile = mgemm_plan(segs, nseg, n, o, (uint32_t)ncu).tile;
+    if (tile != MgemmTile::none) return launch_mgemm_tile<true>(tile, segs, nseg, n, o.W2, st);
+  }
   if (!o.tree && bgemm16_allowed()) {
     if (chain_gemm_fits(segs, nseg, n, o, (uint32_t)ncu)) {
       if (o.W2) return o.norm_w ? launch_chain_gemm<true, true>(segs, nseg, n, o, st)
@@ -2661,18 +2757,8 @@ hipError_t launch_bgemm_multi(const BgemmSeg* segs, uint32_t nseg, uint32_t n,
                       : launch_chain_gemm<false, false>(segs, nseg, n, o, st);
     }
     if (!o.norm_w) {
-      switch (mgemm_plan(segs, nseg, n, o.W2 != nullptr, (uint32_t)ncu).tile) {
-        case MgemmTile::large:
-          return o.W2 ? launch_mgemm<true, 2, 2, 2, 2, 32, 3, 1>(segs, nseg, n, o.W2, st)
-                      : launch_mgemm<false, 2, 2, 2, 2, 32, 3, 1>(segs, nseg, n, o.W2, st);
-        case MgemmTile::small:
-          if (o.W2) return launch_mgemm<true, 2, 1, 2, 2, 32, 2, 2>(segs, nseg, n, o.W2, st);
-          // up to 16 rows: 64 x 16 tiles (the LM head at n = 16: 26 against 41 us)
-          return n <= 16 ? launch_mgemm<false, 1, 1, 4, 1, 64, 2, 1>(segs, nseg, n, o.W2, st)
-                         : launch_mgemm<false, 1, 1, 2, 2, 64, 3, 2>(segs, nseg, n, o.W2, st);
-        default:
-          break;
-      }
+      const MgemmTile tile = mgemm_plan(segs, nseg, n, o, (uint32_t)ncu).tile;
+      if (tile != MgemmTile::none) return launch_mgemm_tile<false>(tile, segs, nseg, n, o.W2, st);
     }
     bool tiles = s0.R == 8 || s0.R == 16;
     for (uint32_t i = 0; i < nseg && tiles; ++i) tiles = segs[i].M % 16 == 0;
@@ -2970,26 +3056,27 @@ static uint32_t att_tiles_grid(uint64_t nitem) {
 }
 // Query heads per item: those of one KV head share its K and V loads where
 // that leaves enough items for two workgroups per CU, else one.  At head_dim
-// 128 up to three (four spilled registers).
-static uint32_t att_tiles_heads(uint32_t ntiles, uint32_t nh, uint32_t nkv, uint32_t hd) {
+// 128 up to three (four spilled registers), in tree order up to two (three).
+static uint32_t att_tiles_heads(uint32_t ntiles, uint32_t nh, uint32_t nkv, uint32_t hd,
+                                bool tree) {
   const uint32_t group = nh / nkv, ncu = (uint32_t)device_cu_count();
-  for (uint32_t h = std::min(group, hd == 64 ? 4u : 3u); h > 1; --h)
+  for (uint32_t h = std::min(group, tree ? 2u : (hd == 64 ? 4u : 3u)); h > 1; --h)
     if (group % h == 0 && (uint64_t)ntiles * (nh / h) >= 2 * (uint64_t)ncu) return h;
   return 1;
 }
 
-template <uint32_t HPT, uint32_t HD>
+template <uint32_t HPT, uint32_t HD, bool TREE>
 static hipError_t launch_att_tiles_t(const float* q, const float* kc, const float* vc,
                                      const AttTile* tiles, uint32_t ntiles, uint32_t nh,
                                      uint32_t group, uint32_t max_pos, uint64_t seq_stride,
                                      float scale, float* out, float* scratch, uint32_t ls,
                                      hipStream_t st) {
   const size_t lds = AttTileCfg<HPT>::floats(HD) * sizeof(float);
-  hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void*>(&k_attention_tiles<HPT, HD>), lds);
+  hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void*>(&k_attention_tiles<HPT, HD, TREE>), lds);
   if (e != hipSuccess) return e;
   const uint64_t nitem = (uint64_t)ntiles * (nh / HPT);
   if (nitem > 0x7fffffffu) return hipErrorInvalidValue;
-  hipLaunchKernelGGL((k_attention_tiles<HPT, HD>), dim3(att_tiles_grid(nitem)), dim3(256), lds, st,
+  hipLaunchKernelGGL((k_attention_tiles<HPT, HD, TREE>), dim3(att_tiles_grid(nitem)), dim3(256), lds, st,
                      q, kc, vc, tiles, (uint32_t)nitem, nh, group, max_pos, seq_stride, scale, out,
                      scratch, ls);
   return hipGetLastError();
@@ -3000,9 +3087,9 @@ bool attention_tiles_supported(uint32_t nh, uint32_t nkv, uint32_t hd) {
 }
 
 size_t attention_tiles_scratch_floats(uint32_t ntiles, uint32_t nh, uint32_t nkv, uint32_t hd,
-                                      uint32_t max_len) {
+                                      uint32_t max_len, bool tree) {
   const size_t ls = ((size_t)max_len + 3) / 4 * 4;
-  const uint32_t h = att_tiles_heads(ntiles, nh, nkv, hd);
+  const uint32_t h = att_tiles_heads(ntiles, nh, nkv, hd, tree);
   return (size_t)att_tiles_grid((uint64_t)ntiles * (nh / h)) * kAttQT * h * ls;
 }
 
@@ -3010,23 +3097,27 @@ hipError_t launch_attention_tiles(const float* q, const float* kc, const float* 
                                   const AttTile* tiles, uint32_t ntiles, uint32_t max_len,
                                   uint32_t nh, uint32_t nkv, uint32_t hd, uint32_t max_pos,
                                   uint64_t seq_stride, float scale, float* out, float* scratch,
-                                  hipStream_t st) {
+                                  hipStream_t st, bool tree) {
   if (ntiles == 0) return hipSuccess;
   if (!attention_tiles_supported(nh, nkv, hd) || max_len == 0 || max_len > max_pos ||
       max_pos % 4)
     return hipErrorInvalidValue;
   const uint32_t g = nh / nkv, ls = (max_len + 3) / 4 * 4;
-#define CIS2_ATT_TILES(H, D)                                                                     \
-  return launch_att_tiles_t<H, D>(q, kc, vc, tiles, ntiles, nh, g, max_pos, seq_stride, scale,   \
-                                  out, scratch, ls, st)
-  switch (att_tiles_heads(ntiles, nh, nkv, hd) * 1000 + hd) {
-    case 1064: CIS2_ATT_TILES(1, 64);
-    case 2064: CIS2_ATT_TILES(2, 64);
-    case 3064: CIS2_ATT_TILES(3, 64);
-    case 4064: CIS2_ATT_TILES(4, 64);
-    case 1128: CIS2_ATT_TILES(1, 128);
-    case 2128: CIS2_ATT_TILES(2, 128);
-    case 3128: CIS2_ATT_TILES(3, 128);
+#define CIS2_ATT_TILES(H, D, TREE)                                                               \
+  return launch_att_tiles_t<H, D, TREE>(q, kc, vc, tiles, ntiles, nh, g, max_pos, seq_stride,    \
+                                        scale, out, scratch, ls, st)
+  switch ((tree ? 10000 : 0) + att_tiles_heads(ntiles, nh, nkv, hd, tree) * 1000 + hd) {
+    case 1064: CIS2_ATT_TILES(1, 64, false);
+    case 2064: CIS2_ATT_TILES(2, 64, false);
+    case 3064: CIS2_ATT_TILES(3, 64, false);
+    case 4064: CIS2_ATT_TILES(4, 64, false);
+    case 1128: CIS2_ATT_TILES(1, 128, false);
+    case 2128: CIS2_ATT_TILES(2, 128, false);
+    case 3128: CIS2_ATT_TILES(3, 128, false);
+    case 11064: CIS2_ATT_TILES(1, 64, true);
+    case 12064: CIS2_ATT_TILES(2, 64, true);
+    case 11128: CIS2_ATT_TILES(1, 128, true);
+    case 12128: CIS2_ATT_TILES(2, 128, true);
     default: return hipErrorInvalidValue;
   }
 #undef CIS2_ATT_TILES

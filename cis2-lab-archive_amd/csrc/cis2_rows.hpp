@@ -46,9 +46,9 @@ struct BgemmOpts {
 hipError_t launch_bgemm_multi(const BgemmSeg* segs, uint32_t nseg, uint32_t n,
                               const BgemmOpts& o, hipStream_t st);
 
+constexpr uint32_t kFuseNormRows = 256;  // k_bgemm alone: norm fused up to here
 // Whether a launch with o.norm_w is better replaced by the norm as a launch of
 // its own and the GEMM over its output.
-constexpr uint32_t kFuseNormRows = 256;  // tree order: fused up to here
 bool bgemm_norm_apart(const BgemmSeg* segs, uint32_t nseg, uint32_t n, const BgemmOpts& o);
 
 // Per-row device descriptors: seq[r], pos[r], tok[r].
@@ -89,24 +89,23 @@ hipError_t launch_rope_attention_rows(const float* q, const float* k, const floa
                                       float* out, bool tree, hipStream_t st);
 // Prefill attention in tiles: rows row0 .. row0+nr-1 (nr <= 16) are rows of
 // sequence seq at positions p0 .. p0+nr-1; each tile's rows get the same
-// bits as launch_attention_rows gives them (sequential order only), with
-// each K and V element read once per tile and up to four query heads.
-// Shapes: head_dim 64 or 128.  The longest tiles should come first (the
-// workgroups take them in order).
-// scratch: attention_tiles_scratch_floats(ntiles, nh, nkv, hd, max_len)
-// floats.
+// bits as launch_attention_rows gives them, with each K and V element read
+// once per tile and up to four query heads.  Shapes: head_dim 64 or 128.  The
+// longest tiles should come first (the workgroups take them in order).
+// scratch: attention_tiles_scratch_floats(ntiles, nh, nkv, hd, max_len,
+// tree) floats.
 struct AttTile {
   uint32_t row0, nr, seq, p0;
 };
 constexpr uint32_t kAttTileRows = 16;
 bool attention_tiles_supported(uint32_t nh, uint32_t nkv, uint32_t hd);
 size_t attention_tiles_scratch_floats(uint32_t ntiles, uint32_t nh, uint32_t nkv, uint32_t hd,
-                                      uint32_t max_len);
+                                      uint32_t max_len, bool tree);
 hipError_t launch_attention_tiles(const float* q, const float* kc, const float* vc,
                                   const AttTile* tiles, uint32_t ntiles, uint32_t max_len,
                                   uint32_t nh, uint32_t nkv, uint32_t hd, uint32_t max_pos,
                                   uint64_t seq_stride, float scale, float* out, float* scratch,
-                                  hipStream_t st);
+                                  hipStream_t st, bool tree);
 // launch_rope_store_rows for the rows of the tiles (k is not rotated in
 // place; attention_tiles_supported shapes).
 hipError_t launch_rope_store_tiles(float* q, const float* k, const float* v, const float* rope_cs,

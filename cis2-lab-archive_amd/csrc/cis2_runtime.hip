@@ -603,7 +603,7 @@ int forward_rows(cis2_ctx* c, uint32_t n, const uint32_t* d_tok, uint32_t max_le
       if (ntiles)
         LAUNCH(launch_attention_tiles(b.q, kc, vc, b.tiles, ntiles, max_len, f.n_heads,
                                       f.n_kv_heads, hd, f.max_pos, seq_stride, c->scale, b.att,
-                                      b.ascr, s),
+                                      b.ascr, s, tree),
                "rows attention tiles");
       else
         LAUNCH(launch_attention_rows(b.q, kc, vc, rd, max_len, f.n_heads, f.n_kv_heads, hd,
@@ -645,8 +645,8 @@ int forward_rows(cis2_ctx* c, uint32_t n, const uint32_t* d_tok, uint32_t max_le
 
 // Uploads row descriptors (and the logit-row list) and runs forward_rows.
 // Rows that attend in tiles: the prefill of many rows (runs of one sequence
-// at consecutive positions, up to kAttTileRows per tile) in the sequential
-// order, for the shapes the tiled kernel has; *ntiles = 0 otherwise.
+// at consecutive positions, up to kAttTileRows per tile) for the shapes the
+// tiled kernel has; *ntiles = 0 otherwise.
 // CIS2_ATT_TILES=1 / 0 forces the tiles on / off (the bits are the same).
 int plan_tiles(cis2_ctx* c, uint32_t n, const uint32_t* seq, const uint32_t* pos,
                uint32_t max_len, uint32_t* ntiles) {
@@ -655,9 +655,7 @@ int plan_tiles(cis2_ctx* c, uint32_t n, const uint32_t* seq, const uint32_t* pos
   *ntiles = 0;
   const char* pe = getenv("CIS2_ATT_TILES");
   const bool force = pe && pe[0] == '1', off = pe && pe[0] == '0';
-  if (off || f.reduction_mode != 0 ||
-      !attention_tiles_supported(f.n_heads, f.n_kv_heads, f.head_dim))
-    return CIS2_OK;
+  if (off || !attention_tiles_supported(f.n_heads, f.n_kv_heads, f.head_dim)) return CIS2_OK;
   // Where the lines lie (us per layer, per-row kernels | tiles): one prompt,
   // 9 heads of 64: 64 rows 87 | 93, 100 rows 114 | 115, 200 rows 161 | 157,
   // 544 rows 242 | 204; 16 heads of 128: 64 rows 233 | 235, 100 rows 337 |
@@ -672,8 +670,11 @@ int plan_tiles(cis2_ctx* c, uint32_t n, const uint32_t* seq, const uint32_t* pos
     i += k;
   }
   const uint32_t nt = (uint32_t)b.htiles.size();
-  if (!force && (uint64_t)nt * 5 > n) return CIS2_OK;  // short runs
-  const size_t scr = attention_tiles_scratch_floats(nt, f.n_heads, f.n_kv_heads, f.head_dim, max_len);
+  // short runs; tree order (its per-row kernel is the slower one): of 4 rows
+  // 154 | 160 and 440 | 358, 256 of them at position 8 332 | 289 and 1222 | 994
+  if (!force && (uint64_t)nt * (f.reduction_mode == 1 ? 4 : 5) > n) return CIS2_OK;
+  const size_t scr = attention_tiles_scratch_floats(nt, f.n_heads, f.n_kv_heads, f.head_dim, max_len,
+                                                    f.reduction_mode == 1);
   // the longest first: the workgroups take the tiles in order
   std::stable_sort(b.htiles.begin(), b.htiles.end(), [](const AttTile& x, const AttTile& y) {
     return x.p0 + x.nr > y.p0 + y.nr;

@@ -9,7 +9,9 @@ vector-unit kernel (CIS2_BGEMM16=0) and the oracle.  Prefill attention
 tile, lengths around the 16-, 64- and 256-position steps, a cache end inside
 a 16-position group, V rows with infinities and NaN past a row's own
 position; against the per-row kernel (CIS2_ATT_TILES=0) and the oracle.
-Attention of many decode rows (k_attention_wave).  The arithmetic is pinned,
+Attention of many decode rows (k_attention_wave).  The tree order of both:
+reductions that end inside a block of 32 and inside a staged chunk, K long
+enough that a partial block's zeros meet signed zeros.  The arithmetic is pinned,
 so there is no tolerance."""
 import os
 
@@ -187,3 +189,56 @@ def test_attention_tiles_later_rows_do_not_leak():
         assert np.array_equal(np.isnan(got), np.isnan(rows)), at
         fin = ~np.isnan(rows)
         assert np.array_equal(got.view(np.uint32)[fin], rows.view(np.uint32)[fin]), at
+
+
+def tree_model(spec, w, per_seq, nseq):
+    return Cis2Model(spec, w, max_pos=per_seq, max_seqs=nseq, reduction_mode=1)
+
+
+@pytest.mark.parametrize("spec,n,per_seq", [
+    (WIDE, 5, 5),        # LM head: 64 x 16 tiles, one partial, K = 20 of 32
+    (WIDE, 17, 17),      # 32 x 32 tiles
+    (ODD, 931, 19),      # K = 132 and 268: a block of 4 and one of 12
+    (FEW, 300, 30),      # 260 and 516
+    (FEW_QWEN2, 700, 50),
+    (ODD, 16001, 40),    # 64 x 64 tiles, the last with one row
+], ids=lambda v: getattr(v, "name", str(v)))
+def test_tree_rows_matrix_core_gemm_bits(spec, n, per_seq):
+    w = EdgeWeights(spec, 12)
+    nseq = (n + per_seq - 1) // per_seq
+    m = tree_model(spec, w, per_seq, nseq)
+    tok = np.random.default_rng(n).integers(0, spec.vocab, n).astype(np.uint32)
+    lg, am = run(m, n, per_seq, tok, "1")
+    lv, av = run(m, n, per_seq, tok, "0")
+    assert np.array_equal(lg, lv)
+    assert np.array_equal(am, av)
+    o = O.OracleModel(spec, w, max_pos=per_seq, reduction=1)
+    first = (nseq - 1) * per_seq
+    for p in range(n - first):
+        want = o.forward(p, int(tok[first + p])).view(np.uint32)
+        assert np.array_equal(want, lg[first + p]), p
+
+
+@pytest.mark.parametrize("nh,nkv,hd", [(1, 1, 64), (4, 2, 64), (3, 1, 64), (2, 1, 128),
+                                       (3, 1, 128)])
+@pytest.mark.parametrize("copies", [1, 300], ids=["one-head-items", "grouped-items"])
+def test_tree_attention_tiles_bits(nh, nkv, hd, copies):
+    spec = heads_spec(nh, nkv, hd)
+    w = artifacts.Weights(spec, 5)
+    lens = [1, 17, 31, 33, 66, 129, 259] if copies == 1 else [19, 34] * (copies // 2)
+    m = tree_model(spec, w, max(lens), len(lens))
+    seq, pos = tile_rows(lens)
+    tok = np.random.default_rng(3).integers(0, spec.vocab, seq.size).astype(np.uint32)
+    out = {}
+    for v in "01":
+        os.environ["CIS2_ATT_TILES"] = v
+        try:
+            out[v], _ = m.forward_rows(seq, pos, tok)
+        finally:
+            del os.environ["CIS2_ATT_TILES"]
+    assert np.array_equal(out["0"].view(np.uint32), out["1"].view(np.uint32))
+    s = len(lens) - 1
+    o = O.OracleModel(spec, w, max_pos=lens[s], reduction=1)
+    for p, r in enumerate(np.flatnonzero(seq == s)):
+        assert np.array_equal(o.forward(p, int(tok[r])).view(np.uint32),
+                              out["1"][r].view(np.uint32)), p
