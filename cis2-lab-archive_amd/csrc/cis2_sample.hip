@@ -23,6 +23,7 @@
 
 #include <mutex>
 
+#include "cis2_chain.hpp"
 #include "cis2_device_math.hpp"
 
 namespace cis2 {
@@ -151,17 +152,24 @@ __global__ __launch_bounds__(256) void k_gather_top(const uint64_t* __restrict__
 // cut; with top_p < 1, m = s of rank 0, e_r = exp(s_r - m), denom =
 // sum_seq(e) in rank order, p_r = e_r / denom, c_r = c_{r-1} + p_r from 0,
 // and the kept ranks end at the first r > 0 with !(c_{r-1} < top_p).
-// The ranks pass through LDS in tiles of kKeepTile: lane 0 runs the strict
-// chain over one tile (16 LDS reads in flight) while waves 1.. form the
-// next tile's terms in the other buffer.  c never decreases (p_r >= 0), so a group of four needs a
-// per-rank test only when its third sum fails.
+// The ranks pass through LDS in tiles of kKeepTile: wave 0 runs the strict
+// chain over one tile in the assembly loop of chain_lds16 while waves 1.. form
+// the next tile's terms in the other buffer (512 threads: the loop's registers
+// allow two waves per SIMD).  c never decreases (p_r >= 0), so the running
+// sum is tested once per 512 ranks, in the block that fails once per 64, and
+// rank by rank in the last of those; a NaN fails the tests and ends there too.
+// What bounds it: the two chains over the ranks.  49,152 ranks, top-p 0.95: a
+// sampled token 1967 -> 1237 us (27 -> 9 cycles per rank and chain; the running
+// sum had been tested after every four of them), top-p 0.5 1401 -> 1155.
 constexpr uint32_t kKeepTile = 8192;
+constexpr uint32_t kKeepT = 512;
 
-__global__ __launch_bounds__(1024) void k_keep(const uint64_t* __restrict__ key,
+__global__ __launch_bounds__(kKeepT) void k_keep(const uint64_t* __restrict__ key,
                                                const float* __restrict__ l, float T, uint32_t K,
                                                float top_p, float* e, uint32_t* nkeep) {
   // two tile buffers: wave 0 chains one while waves 1.. form the next
-  __shared__ __attribute__((aligned(16))) float t[2][kKeepTile];
+  // (32 floats past a tile are readable: the chain loop reads ahead)
+  __shared__ __attribute__((aligned(16))) float t[2][kKeepTile + 32];
   __shared__ float s_den;
   __shared__ uint32_t s_keep;
   if (!(top_p < 1.0f)) {
@@ -183,30 +191,20 @@ __global__ __launch_bounds__(1024) void k_keep(const uint64_t* __restrict__ key,
       e[base + j] = ev;
     }
   };
+  auto chain = [](const float* p, uint32_t np, float acc) {  // 64 np terms
+    return chain_lds16<1>((const __attribute__((address_space(3))) void*)p, np, acc);
+  };
   // the denominator
   float den = 0.0f;
   form_e(0, t[0], threadIdx.x, blockDim.x);
   __syncthreads();
   for (uint32_t tile = 0; tile < nt; ++tile) {
     if (wv == 0) {
-      if (threadIdx.x == 0) {
-        const float4* t4 = reinterpret_cast<const float4*>(t[tile & 1]);
-        const uint32_t n = len(tile), n4 = n / 4;
-        uint32_t g = 0;
-        for (; g + 16 <= n4; g += 16) {
-          float4 v[16];
-#pragma unroll
-          for (uint32_t u = 0; u < 16; ++u) v[u] = t4[g + u];
-#pragma unroll
-          for (uint32_t u = 0; u < 16; ++u) {
-            den = den + v[u].x;
-            den = den + v[u].y;
-            den = den + v[u].z;
-            den = den + v[u].w;
-          }
-        }
-        for (uint32_t r = 4 * g; r < n; ++r) den = den + t[tile & 1][r];
-      }
+      const float* tb = t[tile & 1];
+      const uint32_t n = len(tile), np = n / 64;
+      if (np) den = chain(tb, np, den);
+#pragma unroll 16
+      for (uint32_t r = 64 * np; r < n; ++r) den = den + tb[r];
     } else if (tile + 1 < nt) {
       form_e(tile + 1, t[(tile + 1) & 1], fid, fn);
     }
@@ -232,41 +230,28 @@ __global__ __launch_bounds__(1024) void k_keep(const uint64_t* __restrict__ key,
   __syncthreads();
   for (uint32_t tile = 0; tile < nt; ++tile) {
     if (wv == 0) {
-      if (threadIdx.x == 0) {
-        const float* tb = t[tile & 1];
-        const float4* t4 = reinterpret_cast<const float4*>(tb);
-        const uint32_t base = tile * kKeepTile, n = len(tile), n4 = n / 4;
-        uint32_t keep = 0xFFFFFFFFu, g = 0;
-        for (; g < n4 && keep == 0xFFFFFFFFu; g += 16) {
-          float4 v[16];
+      const float* tb = t[tile & 1];
+      const uint32_t base = tile * kKeepTile, n = len(tile);
+      uint32_t keep = 0xFFFFFFFFu, j = 0;
+      for (uint32_t step = 512; step >= 64; step /= 8)
+        for (; j + step <= n; j += step) {
+          const float end = __int_as_float(
+              __builtin_amdgcn_readfirstlane(__float_as_int(chain(tb + j, step / 64, c))));
+          if (!(end < top_p)) break;
+          c = end;
+        }
+      for (; j < n && keep == 0xFFFFFFFFu; j += 16) {
+        float v[16];
 #pragma unroll
-          for (uint32_t u = 0; u < 16; ++u)
-            if (g + u < n4) v[u] = t4[g + u];
+        for (uint32_t u = 0; u < 16; ++u) v[u] = tb[min(j + u, n - 1)];
 #pragma unroll
-          for (uint32_t u = 0; u < 16; ++u) {
-            if (g + u < n4 && keep == 0xFFFFFFFFu) {
-              const uint32_t r = base + 4 * (g + u);
-              const float c0 = c + v[u].x;
-              const float c1 = c0 + v[u].y;
-              const float c2 = c1 + v[u].z;
-              const float c3 = c2 + v[u].w;
-              if (!(c2 < top_p)) {  // the prefix ends inside ranks r..r+3
-                if (r > 0 && !(c < top_p)) keep = r;
-                else if (!(c0 < top_p)) keep = r + 1;
-                else if (!(c1 < top_p)) keep = r + 2;
-                else keep = r + 3;
-              }
-              c = c3;
-            }
+        for (uint32_t u = 0; u < 16; ++u)
+          if (j + u < n && keep == 0xFFFFFFFFu) {
+            if (base + j + u > 0 && !(c < top_p)) keep = base + j + u;
+            else c = c + v[u];
           }
-        }
-        for (uint32_t j = 4 * n4; j < n && keep == 0xFFFFFFFFu; ++j) {
-          const uint32_t r = base + j;
-          if (r > 0 && !(c < top_p)) keep = r;
-          else c = c + tb[j];
-        }
-        s_keep = keep;
       }
+      if (threadIdx.x == 0) s_keep = keep;
     } else if (tile + 1 < nt) {
       form_p(tile + 1, t[(tile + 1) & 1], fid, fn);
     }
@@ -390,7 +375,7 @@ hipError_t launch_sample(const float* logits, uint32_t V, const SampleParams& p,
     } else {
       sort(b.key, Vp);
     }
-    hipLaunchKernelGGL(k_keep, dim3(1), dim3(1024), 0, s, order, logits, p.temperature, K,
+    hipLaunchKernelGGL(k_keep, dim3(1), dim3(kKeepT), 0, s, order, logits, p.temperature, K,
                        p.top_p, b.e, b.nkeep);
   }
   hipLaunchKernelGGL(k_draw, dim3(kSampleBlocks), dim3(256), 0, s, order, logits,

@@ -80,6 +80,21 @@ def test_draws_match_oracle(V, ctx_by_vocab):
     m.set_sampling(None)
 
 
+@pytest.mark.parametrize("K", [1, 63, 64, 65, 511, 512, 513, 577, 8191, 8192, 8193, 8257, 9000])
+def test_top_p_ends_at_block_edges(K, ctx_by_vocab):
+    """Equal logits: the kept prefix of K ranks ends inside, at and after the
+    blocks of 64, 512 and 8192 ranks that the running sum is tested by."""
+    m = ctx_by_vocab(49152)
+    lg = np.full(49152, np.float32(-0.5))
+    for r in sorted({1, 2, 63, 64, 65, 128, 512, 513, 1024, 8192, 8193, K - 1, K} & set(range(1, K + 1))):
+        p = np.float32((r - 0.5) / K)
+        m.set_sampling(3, 1.0, K, p)
+        ids, nk = m.sample_logits(lg[None], [r])
+        want, _, kept = O.sample(lg, 3, r, 1.0, K, p)
+        assert (int(ids[0]), int(nk[0])) == (want, kept), (K, r)
+    m.set_sampling(None)
+
+
 def test_top_k_at_and_beyond_vocab_is_disabled(ctx_by_vocab):
     V = 512
     m = ctx_by_vocab(V)
