@@ -242,3 +242,101 @@ def test_tree_attention_tiles_bits(nh, nkv, hd, copies):
     for p, r in enumerate(np.flatnonzero(seq == s)):
         assert np.array_equal(o.forward(p, int(tok[r])).view(np.uint32),
                               out["1"][r].view(np.uint32)), p
+
+
+def logits_spec(k, vocab=40003):
+    return artifacts.ModelSpec("lm%d" % k, k, 72, 1, 2, 1, vocab, 1e-5, 10000.0, False)
+
+
+class TinySums(artifacts.Weights):
+    """The seeded weights, final norm weights of 2; an LM head row is +-0 but
+    for one entry of 2^-126 .. 2^-122 in its first block of 32 and one at its
+    end, so that among many rows some sums cancel to a negative value that is
+    flushed, to -0."""
+
+    def __init__(self, spec, seed):
+        super().__init__(spec, seed)
+        rng = np.random.default_rng(seed)
+        h, v = spec.hidden, spec.vocab
+        w = (rng.integers(0, 2, (v, h)) << 15).astype(np.uint16)
+        for lo, hi in ((0, 32), (h - 1, h)):
+            at = (np.arange(v), rng.integers(lo, hi, v))
+            w[at] |= rng.integers(1 << 7, 5 << 7, v).astype(np.uint16)
+        for name, _, arr in self.tensors:
+            if name == "lm_head.weight":
+                arr[:] = w.reshape(-1)
+            elif name == "model.norm.weight":
+                arr[:] = 0x4000
+
+
+@pytest.mark.parametrize("tree", [True, False], ids=["tree", "seq"])
+@pytest.mark.parametrize("k", [68, 96, 100, 132, 160])
+@pytest.mark.parametrize("n", [5, 17])  # 64 x 16 and 32 x 32 tiles
+def test_rows_matrix_core_gemm_negative_zero_sums(k, n, tree):
+    """A sum of -0 stays -0 whatever lies between K and the end of the staged
+    chunk (64 k: at K = 68, 96, 132 and 160 a whole block of 32 lies past K)."""
+    spec = logits_spec(k)
+    w = TinySums(spec, 13)
+    m = Cis2Model(spec, w, max_pos=n, max_seqs=1, reduction_mode=1 if tree else 0)
+    tok = np.random.default_rng(n).integers(0, spec.vocab, n).astype(np.uint32)
+    lg, am = run(m, n, n, tok, "1")
+    o = O.OracleModel(spec, w, max_pos=n, reduction=1 if tree else 0)
+    want = np.stack([o.forward(p, int(tok[p])) for p in range(n)]).view(np.uint32)
+    assert (want == 0x80000000).sum() > 1000
+    assert np.array_equal(want, lg)
+    lv, av = run(m, n, n, tok, "0")
+    assert np.array_equal(want, lv)
+    assert np.array_equal(am, av)
+
+
+class Extremes(artifacts.Weights):
+    """The seeded weights, final norm weights of 2^8; of every four LM head
+    rows one holds subnormals only (times activations that would lift them
+    far above 2^-126 if they were not flushed), one a NaN of any
+    sign and payload among its values, one two infinities, one +-0 and entries
+    whose products lie around 2^-126."""
+
+    def __init__(self, spec, seed):
+        super().__init__(spec, seed)
+        rng = np.random.default_rng(seed)
+        h, v = spec.hidden, spec.vocab
+        for name, _, arr in self.tensors:
+            if name == "model.norm.weight":
+                arr[:] = 0x4380
+            elif name == "lm_head.weight":
+                w = arr.reshape(v, h)
+                sign = (rng.integers(0, 2, (v, h)) << 15).astype(np.uint16)
+                w[0::4] = (sign | rng.integers(1, 0x80, (v, h)).astype(np.uint16))[0::4]
+                r = np.arange(1, v, 4)
+                w[r, rng.integers(0, h, r.size)] = (0x7F81 + rng.integers(0, 0x7F, r.size) |
+                                                   rng.integers(0, 2, r.size) << 15)
+                r = np.arange(2, v, 4)
+                for _ in range(2):
+                    w[r, rng.integers(0, h, r.size)] = 0x7F80 | rng.integers(0, 2, r.size) << 15
+                k = rng.integers(0, 5 << 7, (v, h)).astype(np.uint16)
+                w[3::4] = (sign | np.where(rng.random((v, h)) < 0.5, k, 0).astype(np.uint16))[3::4]
+
+
+@pytest.mark.parametrize("tree", [True, False], ids=["tree", "seq"])
+@pytest.mark.parametrize("k", [20, 68])
+@pytest.mark.parametrize("n", [5, 17])
+def test_rows_matrix_core_gemm_subnormals_and_nans(k, n, tree):
+    """The matrix cores' products flush subnormal operands and results and
+    carry NaNs as the vector unit's multiply does: the bits of every logit,
+    NaNs' sign and payload too, are the vector-unit kernel's, and those of
+    every other logit the oracle's (NaNs made by x86 have another sign)."""
+    spec = logits_spec(k)
+    w = Extremes(spec, 14)
+    m = Cis2Model(spec, w, max_pos=n, max_seqs=1, reduction_mode=1 if tree else 0)
+    tok = np.random.default_rng(n).integers(0, spec.vocab, n).astype(np.uint32)
+    lg, am = run(m, n, n, tok, "1")
+    lv, av = run(m, n, n, tok, "0")
+    assert np.array_equal(lg, lv)
+    assert np.array_equal(am, av)
+    o = O.OracleModel(spec, w, max_pos=n, reduction=1 if tree else 0)
+    want = np.stack([o.forward(p, int(tok[p])) for p in range(n)])
+    got = lg.view(np.float32)
+    assert not want[:, 0::4].any()  # subnormal weights are zeros
+    nan = np.isnan(want)
+    assert nan[:, 1::4].all() and np.array_equal(nan, np.isnan(got))
+    assert np.array_equal(want.view(np.uint32)[~nan], lg[~nan])
