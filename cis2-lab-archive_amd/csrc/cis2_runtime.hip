@@ -181,13 +181,16 @@ constexpr uint32_t kPlanR = 16;
 // streaming batch kernel.
 constexpr uint32_t kPlanStreamBlocks = 512;
 
+// Largest vectors of a GEMV plan that go through its pinned memory.
+constexpr size_t kPlanHost = 1 << 20;
+
 struct cis2_gemv_plan {
   uint32_t M, K, copies;
   float *W = nullptr, *x = nullptr, *y = nullptr;
   float *xb = nullptr, *yb = nullptr;  // [ncap][K], [ncap][M]: batched launches
   uint32_t ncap = 0;
   float *hx = nullptr, *hy = nullptr;  // mapped pinned host memory, hcap bytes each
-  size_t hcap = 0;
+  size_t hcap = 0, hmost = kPlanHost;  // hmost: the most that is asked for
   hipStream_t st = nullptr;
   hipEvent_t e0 = nullptr, e1 = nullptr;
 };
@@ -2042,20 +2045,32 @@ int cis2_verify_prefill(cis2_ctx* c, uint32_t seq, const uint32_t* prompt, uint3
 // Host vectors of up to kPlanHost bytes go through the plan's mapped pinned
 // memory, which the GEMV reads and writes itself: 1536 x 576 19.8 us a call,
 // 21.5 with x fetched by a kernel first, 30.5 with copies from and to
-// pageable memory; 49152 x 576 41, 45 and 56 us.  A batch's inputs are
-// fetched first (60 of 200 x 2000: 88 against 120 us).  Larger ones are
-// copied.
-constexpr size_t kPlanHost = 1 << 20;
-static hipError_t plan_host(cis2_gemv_plan* p, size_t bytes) {
-  if (bytes <= p->hcap) return hipSuccess;
+// pageable memory; 49152 x 576 41, 45 and 56 us.  A workgroup's block of W
+// has to fit its LDS, so x is at most 2,300 floats or so; copies against
+// mapped memory over the rest of that range: 16 x 64 33 | 20, 151936 x 64
+// 113 | 93, 16 x 2048 37 | 27, 16384 x 2048 129 | 83 us.  A batch's inputs are
+// fetched first (60 of 200 x 2000: 88 against 120 us; 60 of 4096 x 64, copied
+// | mapped, 165 | 156).  Larger ones are copied, and all of them where no
+// pinned memory is to be had.
+// Pinned memory of `bytes` for each of the plan's vectors; false where it is
+// refused, and from then on for that size and above without asking again.
+static bool plan_host(cis2_gemv_plan* p, size_t bytes) {
+  if (bytes <= p->hcap) return true;
+  if (bytes > p->hmost) return false;
   if (p->hx) (void)hipHostFree(p->hx);
   if (p->hy) (void)hipHostFree(p->hy);
   p->hx = p->hy = nullptr;
   p->hcap = 0;
-  hipError_t e = hipHostMalloc(reinterpret_cast<void**>(&p->hx), bytes);
-  if (e == hipSuccess) e = hipHostMalloc(reinterpret_cast<void**>(&p->hy), bytes);
-  if (e == hipSuccess) p->hcap = bytes;
-  return e;
+  if (hipHostMalloc(reinterpret_cast<void**>(&p->hx), bytes) != hipSuccess ||
+      hipHostMalloc(reinterpret_cast<void**>(&p->hy), bytes) != hipSuccess) {
+    (void)hipGetLastError();
+    if (p->hx) (void)hipHostFree(p->hx);
+    p->hx = nullptr;
+    p->hmost = bytes - 1;
+    return false;
+  }
+  p->hcap = bytes;
+  return true;
 }
 
 int cis2_gemv_plan_create(uint32_t M, uint32_t K, uint32_t copies, const float* W,
@@ -2078,7 +2093,7 @@ int cis2_gemv_plan_create(uint32_t M, uint32_t K, uint32_t copies, const float* 
   if (e == hipSuccess) e = hipEventCreate(&p->e0);
   if (e == hipSuccess) e = hipEventCreate(&p->e1);
   const size_t host = ((size_t)std::max(M, K)) * sizeof(float) + 256;
-  if (e == hipSuccess && host <= kPlanHost) e = plan_host(p, host);
+  if (e == hipSuccess) (void)plan_host(p, host);
   if (rowmajor) (void)hipFree(rowmajor);
   if (e != hipSuccess) {
     cis2_gemv_plan_destroy(p);
@@ -2111,8 +2126,7 @@ static hipError_t plan_through(cis2_gemv_plan* p, uint32_t n, const float* x, fl
   };
   const size_t most = std::max(nx, ny) * sizeof(float) + 256;
   hipError_t e;
-  if (most > kPlanHost || plan_host(p, most) != hipSuccess) {
-    (void)hipGetLastError();  // no pinned memory: copy
+  if (!plan_host(p, most)) {
     e = hipMemcpyAsync(dx, x, nx * sizeof(float), hipMemcpyHostToDevice, p->st);
     if (e == hipSuccess) e = launch(dy);
     if (e == hipSuccess)

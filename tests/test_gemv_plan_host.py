@@ -1,0 +1,62 @@
+"""The host side of the standalone GEMV plan over a HIP runtime of stubs
+(hip_stub.cpp), without a GPU: where its pinned memory is refused, the plan
+copies instead."""
+import os
+import shutil
+import subprocess
+import sys
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+PKG = os.path.join(ROOT, "cis2-lab-archive_amd")
+ROCM = "/opt/rocm"
+
+SETUP = """
+import ctypes, sys
+import numpy as np
+sys.path.insert(0, %r)
+stub = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+from cis2amd import GemvPlan
+def check(M, x, y):
+    assert np.array_equal(y, x[..., :1] + np.arange(M, dtype=np.float32)), y
+M, K = 40, 8
+x = np.arange(1, 9, dtype=np.float32)
+X = np.arange(8, 8 + 5 * K, dtype=np.float32).reshape(5, K)
+""" % PKG
+
+
+@pytest.fixture(scope="module")
+def stub(tmp_path_factory):
+    gxx = shutil.which("g++")
+    if not gxx or not os.path.isdir(os.path.join(ROCM, "include", "hip")):
+        pytest.skip("no g++ or no HIP headers")
+    so = tmp_path_factory.mktemp("stub") / "libhipstub.so"
+    b = subprocess.run([gxx, "-std=c++17", "-O1", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__",
+                        "-I" + os.path.join(ROCM, "include"), "-o", str(so),
+                        os.path.join(ROOT, "tests", "hip_stub.cpp")],
+                       capture_output=True, text=True, timeout=300)
+    assert b.returncode == 0, b.stderr[-2000:]
+    return str(so)
+
+
+def run(stub, body):
+    r = subprocess.run([sys.executable, "-c", SETUP + body, stub], capture_output=True, text=True,
+                       timeout=120)
+    assert r.returncode == 0, r.stderr[-2000:]
+
+
+@pytest.mark.parametrize("pinned", [0, 1, 2, 100])
+def test_plan_without_pinned_memory(stub, pinned):
+    """`pinned` allocations of pinned memory succeed: the plan is made, lone
+    and batched products go through it, and everything is given back."""
+    run(stub, """
+stub.stub_allow_pinned(%d)
+p = GemvPlan(np.ones((M, K), np.float32))
+check(M, x, p(x))
+check(M, X, p.run_batch(X))
+check(M, x, p(x))
+assert stub.stub_launches() == 3 and stub.stub_undefined_inputs() == 0
+p.close()
+assert stub.stub_live() == 0
+""" % pinned)
