@@ -2084,6 +2084,8 @@ int cis2_gemv_plan_create(uint32_t M, uint32_t K, uint32_t copies, const float* 
   hipError_t e = hipStreamCreateWithFlags(&p->st, hipStreamNonBlocking);
   if (e == hipSuccess) e = hipMalloc(&p->W, per * copies * sizeof(float));
   if (e == hipSuccess) e = hipMalloc(&p->x, (size_t)K * sizeof(float));
+  // defined inputs for the timing runs
+  if (e == hipSuccess) e = hipMemsetAsync(p->x, 0, (size_t)K * sizeof(float), p->st);
   if (e == hipSuccess) e = hipMalloc(&p->y, ((size_t)M + 64) * sizeof(float));
   if (e == hipSuccess) e = hipMalloc(&rowmajor, (size_t)M * K * sizeof(float));
   if (e == hipSuccess) e = hipMemcpy(rowmajor, W, (size_t)M * K * sizeof(float), hipMemcpyHostToDevice);

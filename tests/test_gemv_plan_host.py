@@ -1,6 +1,6 @@
 """The host side of the standalone GEMV plan over a HIP runtime of stubs
 (hip_stub.cpp), without a GPU: where its pinned memory is refused, the plan
-copies instead."""
+copies instead; its timing runs read defined memory."""
 import os
 import shutil
 import subprocess
@@ -60,3 +60,20 @@ assert stub.stub_launches() == 3 and stub.stub_undefined_inputs() == 0
 p.close()
 assert stub.stub_live() == 0
 """ % pinned)
+
+
+@pytest.mark.parametrize("rows", [40, 16 * 513], ids=["lone-kernel", "streaming-kernel"])
+def test_timing_runs_have_defined_inputs(stub, rows):
+    """plan_time and plan_time_batch multiply memory that was written, before
+    and after a run."""
+    run(stub, """
+M = %d
+p = GemvPlan(np.ones((M, K), np.float32), copies=2)
+p.time(3)
+check(M, x, p(x))
+p.time(3)
+p.time_batch(4, 3)
+assert stub.stub_launches() == 2 * (2 + 3) + 1 + 4 and stub.stub_undefined_inputs() == 0
+p.close()
+assert stub.stub_live() == 0
+""" % rows)
