@@ -626,6 +626,7 @@ template <bool DUAL, bool NORM>
 __global__ __launch_bounds__((ChainCfg<DUAL, NORM>::T), 3) void k_chain_gemm(BgemmArgs a) {
   using C = ChainCfg<DUAL, NORM>;
   constexpr uint32_t CW = C::CW, NP = C::NP, GPW = C::GPW, SG = C::SG, D = C::D, T = C::T;
+  // at LDS address 0, as chain_ring needs: no static __shared__ in this kernel
   extern __shared__ v4 sm[];
   uint32_t si = 0;
   if (a.nseg > 1 && blockIdx.x >= a.blk0[1]) si = (a.nseg > 2 && blockIdx.x >= a.blk0[2]) ? 2 : 1;

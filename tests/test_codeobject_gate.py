@@ -17,6 +17,11 @@ each kernel is checked:
     integer split with a -2^32 literal), which carry no float data;
   - the pure reduction kernels (the standalone GEMVs, the per-op GEMV, the
     row GEMMs without norm or gate) contain no FMA and no divide at all;
+  - the matrix cores only form products: v_mfma_f32_16x16x1_4b_f32 (one
+    product per result) in the two kernels that use them, and its addend is
+    always -0, never a sum;
+  - the few-row GEMM has no static LDS: its ring is addressed as (address &
+    0xffff) | ring, which needs the dynamic LDS to start at 0;
   - no scalar-cache writes of any kind (stores, atomics, write-back).
 
 The per-kernel FMA accounting is printed (pytest -s)."""
@@ -43,7 +48,10 @@ FMA64 = re.compile(r"^v_fma(c)?_f64$")
 # integer sequences: +-2^32 as an f32 literal, or as the high word of an f64
 INT_LIT32 = re.compile(r"0x[4c]f800000\b")
 INT_LIT64 = re.compile(r"0x[4c]1f00000\b")
-STRICT_ZERO = re.compile(r"(k_gemv_blk|k_gemv_pipe|k_gemv_many|4cis26k_gemvE|k_bgemmILb0ELb0E|k_bgemm16ILb0ELb0E)")
+STRICT_ZERO = re.compile(r"(k_gemv_blk|k_gemv_pipe|k_gemv_many|4cis26k_gemvE|k_bgemmILb0ELb0E|"
+                         r"k_bgemm16ILb0ELb0E|k_mgemmILb0E|k_chain_gemmILb0ELb0E)")
+MFMA = "v_mfma_f32_16x16x1_4b_f32"
+MFMA_KERNELS = re.compile(r"(k_mgemmI|k_attention_tilesI)")
 
 
 def tools():
@@ -100,6 +108,41 @@ def account(ins):
     }
 
 
+def regs(text):
+    """The vector registers that an operand text names."""
+    out = set()
+    for c, a, b in re.findall(r"\b([va])\[(\d+):(\d+)\]", text):
+        out.update(c + str(i) for i in range(int(a), int(b) + 1))
+    out.update(c + n for c, n in re.findall(r"\b([va])(\d+)\b", text))
+    return out
+
+
+def mfma_faults(ins):
+    """What breaks the rule on matrix-core instructions, in program order:
+    another one than MFMA, or an addend register that does not hold -0
+    (v_bfrev_b32 of 1, through moves)."""
+    zero, bad = set(), []
+    for op, a in ins:
+        args = [x.strip() for x in a.split(",")]
+        if op.startswith(("v_mfma", "v_smfmac")):
+            if op != MFMA:
+                bad.append((op, a))
+            elif not regs(args[3]) or not regs(args[3]) <= zero or regs(args[0]) & regs(args[3]):
+                bad.append((op, a))
+        if op.startswith("s_") or "store" in op or op.startswith("ds_write"):
+            continue
+        dst = regs(args[0])
+        if op.startswith(("v_swap", "v_permlane")):
+            dst |= regs(args[1])
+        if op == "v_bfrev_b32" and args[1] == "1":
+            zero |= dst
+        elif op.startswith("v_mov_b") and regs(args[1]) and regs(args[1]) <= zero:
+            zero |= dst
+        else:
+            zero -= dst
+    return bad
+
+
 @pytest.fixture(scope="module")
 def code(tmp_path_factory):
     tools()
@@ -138,6 +181,37 @@ def test_fma_only_in_divide_and_sqrt_expansions(code):
                 bad.append((f, a))
     print("\n".join(lines))
     assert not bad, bad
+
+
+def test_matrix_cores_only_form_products(code):
+    used = set()
+    for obj in code.values():
+        for f, ins in obj.items():
+            if any(op.startswith(("v_mfma", "v_smfmac")) for op, _ in ins):
+                assert MFMA_KERNELS.search(f), f
+                used.add(f)
+                assert not mfma_faults(ins), (f, mfma_faults(ins)[:3])
+    assert len(used) >= 10
+
+
+def test_few_row_gemm_has_no_static_lds(tmp_path):
+    tools()
+    disassemble("cis2_rows", str(tmp_path))
+    r = subprocess.run([os.path.join(LLVM, "llvm-readelf"), "--notes",
+                        os.path.join(str(tmp_path), "cis2_rows.co")], check=True,
+                       capture_output=True, text=True)
+    # .group_segment_fixed_size comes before its kernel's .name
+    sizes, size = {}, None
+    for line in r.stdout.splitlines():
+        m = re.match(r"\s*\.group_segment_fixed_size:\s+(\d+)", line)
+        if m:
+            size = int(m.group(1))
+        m = re.match(r"\s*\.name:\s+(_Z\S+)", line)
+        if m:
+            sizes[m.group(1)] = size
+    few = {k: v for k, v in sizes.items() if "k_chain_gemm" in k}
+    assert len(few) == 4 and not any(few.values()), few
+    assert any(v for k, v in sizes.items() if "k_mgemm" in k)  # the field is read
 
 
 def test_no_kernel_spills_vector_registers(tmp_path):
@@ -206,7 +280,7 @@ def test_pure_reduction_kernels_have_no_fma(code):
                 seen += 1
                 a = account(ins)
                 assert a["fma32"] == a["fma64"] == 0 and a["div32"] == a["div64"] == 0, (f, a)
-    assert seen >= 6
+    assert seen >= 17
 
 
 PROBE = r"""
@@ -219,16 +293,14 @@ __global__ void probe_dot(const float* w, const float* x, float* y, int n) {
 """
 
 
-@pytest.mark.parametrize("contract,flagged", [("off", False), ("fast", True)])
-def test_gate_catches_contraction(contract, flagged, tmp_path):
-    """A strict dot product compiled with -ffp-contract=fast (a plausible
-    build mistake) has FMAs the gate rejects; with =off it passes."""
+def build_probe(text, contract, tmp_path):
+    """{kernel: instructions} of a source compiled here."""
     tools()
     hipcc = "/opt/rocm/bin/hipcc"
     if not os.path.exists(hipcc):
         pytest.skip("no hipcc")
     src = tmp_path / "probe.hip"
-    src.write_text(PROBE)
+    src.write_text(text)
     obj = tmp_path / "probe.o"
     r = subprocess.run([hipcc, "--offload-arch=gfx950", "-O3", "-ffp-contract=" + contract,
                         "-c", "-o", str(obj), str(src)], capture_output=True, text=True, timeout=300)
@@ -241,8 +313,46 @@ def test_gate_catches_contraction(contract, flagged, tmp_path):
                     "--output=" + co], check=True, capture_output=True)
     asm = subprocess.run([os.path.join(LLVM, "llvm-objdump"), "-d", "--mcpu=gfx950", co],
                          check=True, capture_output=True, text=True).stdout
-    k = kernels(asm)
+    return kernels(asm)
+
+
+@pytest.mark.parametrize("contract,flagged", [("off", False), ("fast", True)])
+def test_gate_catches_contraction(contract, flagged, tmp_path):
+    """A strict dot product compiled with -ffp-contract=fast (a plausible
+    build mistake) has FMAs the gate rejects; with =off it passes."""
+    k = build_probe(PROBE, contract, tmp_path)
     f = [n for n in k if "probe_dot" in n][0]
     a = account(k[f])
     extra = a["fma32"] - (5 * a["div32"] + 5 * a["sqrt32"] + a["int_fma32"])
     assert (extra > 0) == flagged, a
+
+
+PROBE_MFMA = r"""
+#include <hip/hip_runtime.h>
+typedef float f16v __attribute__((ext_vector_type(16)));
+__global__ void probe_mfma(const float* w, const float* x, f16v* y, int n) {
+  float z = __int_as_float((int)%s);
+  asm volatile("" : "+v"(z));
+  f16v nz, acc;
+  for (int i = 0; i < 16; ++i) nz[i] = acc[i] = z;
+  for (int k = 0; k < n; ++k) {
+    f16v d = __builtin_amdgcn_%s(w[k * 64 + threadIdx.x], x[k * 64 + threadIdx.x], %s, 0, 0, 0);
+    asm volatile("" : "+v"(d));
+    for (int i = 0; i < 16; ++i) acc[i] = acc[i] + d[i];
+  }
+  y[threadIdx.x] = acc;
+}
+"""
+
+
+@pytest.mark.parametrize("zero,builtin,addend,flagged", [
+    ("0x80000000u", "mfma_f32_16x16x1f32", "nz", False),
+    ("0x80000000u", "mfma_f32_16x16x1f32", "acc", True),   # sums in the matrix cores
+    ("0u", "mfma_f32_16x16x1f32", "nz", True),             # +0 loses a product's sign
+    ("0x80000000u", "mfma_f32_32x32x2f32", "nz", True),    # two products per result
+], ids=["products", "accumulates", "plus-zero", "another-shape"])
+def test_gate_catches_matrix_core_sums(zero, builtin, addend, flagged, tmp_path):
+    k = build_probe(PROBE_MFMA % (zero, builtin, addend), "off", tmp_path)
+    f = [n for n in k if "probe_mfma" in n][0]
+    assert any(op.startswith("v_mfma") for op, _ in k[f])
+    assert bool(mfma_faults(k[f])) == flagged, mfma_faults(k[f])
