@@ -76,3 +76,20 @@ def test_batched_gemvs_equal_single_and_oracle(M, K, n):
         assert np.array_equal(Y[i].view(np.uint32), plan(X[i]).view(np.uint32)), i
         assert np.array_equal(Y[i].view(np.uint32), O.gemv(W, X[i]).view(np.uint32)), i
     plan.close()
+
+
+@pytest.mark.parametrize("M,K,n", [(4096, 64, 80),     # outputs of more than 1 MB
+                                   (16, 2048, 140)])   # inputs of more than 1 MB
+def test_copied_and_mapped_vectors_in_turn(M, K, n):
+    """A plan's vectors go through pinned memory up to 1 MB and are copied
+    above: a batch of either side, lone products between them."""
+    rng = np.random.default_rng(M + K)
+    W = rng.standard_normal((M, K)).astype(np.float32)
+    X = rng.standard_normal((n, K)).astype(np.float32)
+    want = np.stack([O.gemv(W, x) for x in X]).view(np.uint32)
+    plan = GemvPlan(W, copies=2)
+    for k in (1, n, 3, n - 1, 0):
+        assert np.array_equal(plan(X[k % n]).view(np.uint32), want[k % n])
+        if k:
+            assert np.array_equal(plan.run_batch(X[:k]).view(np.uint32), want[:k]), k
+    plan.close()

@@ -2,9 +2,10 @@
 
 Few rows (k_chain_gemm): row counts around its 8-row tiles, outputs and K
 that are no multiple of its tiles, with and without the fused norm and the
-gate.  GEMMs on the matrix cores (k_mgemm): sizes that are no multiple of any tile in rows, outputs or
-K, weights with signed zeros and products that flush to zero; against the
-vector-unit kernel (CIS2_BGEMM16=0) and the oracle.  Prefill attention
+gate.  GEMMs on the matrix cores (k_mgemm): sizes that are no multiple of any
+tile in rows, outputs or K, weights with signed zeros, sums that are flushed
+to -0, subnormal weights, NaNs and infinities; against the vector-unit kernel
+(CIS2_BGEMM16=0) and the oracle.  Prefill attention
 (k_attention_tiles): every number of heads per item, runs that end inside a
 tile, lengths around the 16-, 64- and 256-position steps, a cache end inside
 a 16-position group, V rows with infinities and NaN past a row's own
@@ -38,7 +39,8 @@ FEW_QWEN2 = artifacts.ModelSpec("few-qwen2", 320, 256, 1, 5, 5, 97, 1e-6, 10000.
 
 class EdgeWeights(artifacts.Weights):
     """The seeded weights with one entry in 16 replaced by +-0 and one in 16
-    by +-2^-125 (times an activation below 1/2: a product that is flushed)."""
+    by +-2^-125 (in sums of ordinary size; Extremes has the sums that a
+    product not flushed would change)."""
 
     def __init__(self, spec, seed):
         super().__init__(spec, seed)
@@ -161,7 +163,8 @@ def test_attention_wave_bits(nh, nkv, hd, pos):
 
 def test_attention_tiles_later_rows_do_not_leak():
     """A row whose V (and K) hold NaN or infinities changes no row before it,
-    also inside one tile, and not a NaN's or a zero's sign there."""
+    also inside one tile; it and the rows after it get the per-row kernel's
+    bits, those of the NaNs among them."""
     spec = heads_spec(2, 1, 64)
     w = artifacts.Weights(spec, 6)
     emb = next(a for name, _, a in w.tensors if "embed" in name)
@@ -186,9 +189,8 @@ def test_attention_tiles_later_rows_do_not_leak():
             rows, _ = clean.forward_rows(np.zeros(n), np.arange(n), t2)
         finally:
             del os.environ["CIS2_ATT_TILES"]
-        assert np.array_equal(np.isnan(got), np.isnan(rows)), at
-        fin = ~np.isnan(rows)
-        assert np.array_equal(got.view(np.uint32)[fin], rows.view(np.uint32)[fin]), at
+        assert np.isnan(rows[at:]).any()
+        assert np.array_equal(got.view(np.uint32), rows.view(np.uint32)), at  # NaNs' bits too
 
 
 def tree_model(spec, w, per_seq, nseq):
@@ -340,3 +342,24 @@ def test_rows_matrix_core_gemm_subnormals_and_nans(k, n, tree):
     nan = np.isnan(want)
     assert nan[:, 1::4].all() and np.array_equal(nan, np.isnan(got))
     assert np.array_equal(want.view(np.uint32)[~nan], lg[~nan])
+
+
+@pytest.mark.parametrize("tree", [True, False], ids=["tree", "seq"])
+@pytest.mark.parametrize("hd", [6, 22, 34])
+def test_qk_norm_of_head_dims_that_are_no_multiple_of_four(hd, tree):
+    """The vectors of such a QK-norm take the norm kernel that has a workgroup
+    per vector; many and few rows, and one position at a time."""
+    spec = artifacts.ModelSpec("qk%d" % hd, 64, 96, 2, 4, 2, 131, 1e-6, 10000.0, True,
+                               head_dim=hd, qk_norm=True, sigma=0.3)
+    w = artifacts.Weights(spec, 15)
+    n = 70
+    tok = np.random.default_rng(hd).integers(0, spec.vocab, n).astype(np.uint32)
+    o = O.OracleModel(spec, w, max_pos=n, reduction=1 if tree else 0)
+    want = np.stack([o.forward(p, int(tok[p])) for p in range(n)]).view(np.uint32)
+    m = Cis2Model(spec, w, max_pos=n, max_seqs=1, reduction_mode=1 if tree else 0)
+    lg, _ = m.forward_rows(np.zeros(n), np.arange(n), tok)
+    assert np.array_equal(want, lg.view(np.uint32))
+    m.reset(0)
+    for at, k in ((0, 1), (1, 3), (4, 1)):
+        lg, _ = m.forward_rows(np.zeros(k), np.arange(at, at + k), tok[at:at + k])
+        assert np.array_equal(want[at:at + k], lg.view(np.uint32)), at
