@@ -902,12 +902,11 @@ struct MgemmArgs {
 // wave's 16-byte read gives lane l (row l % 16, u = l / 16) its operands of
 // four products4.  A thread stages whole (row, 16 k) pieces: four 16-byte
 // loads, transposed by register naming.  Past K the pieces hold -0 for W and
-// +0 for X: their products are -0, which no sum notices, a sum of -0 (values
-// that cancel to a flushed subnormal) included.  In tree order the block of 32
-// that K ends in holds +0 for both, as tree32's last block does, and the blocks
-// past it in the chunk -0 for W again: -0 is their sum, and +0 would turn a
-// sum of -0 into +0.  Chunk c + PF is loaded into registers while chunk c is
-// computed.
+// +0 for X: their products are -0, which no sum notices.  In tree order the
+// block of 32 that K ends in is filled with zeros, as tree32's last block is,
+// and the last chunk ends with it: a block past K would add +0, which turns a
+// sum of -0 (values that cancel to a flushed subnormal) into +0.  Chunk c + PF
+// is loaded into registers while chunk c is computed.
 // Stores a lane's outputs m .. m + 3 of X row `row`: sums y, with y2 those of
 // the second matrix (DUAL).
 template <bool DUAL>
@@ -972,7 +971,6 @@ __global__ __launch_bounds__(256, OCC) void k_mgemm(MgemmArgs a) {
   const uint32_t m0 = (ut - a.tile0[si]) * C::BM, n0 = nt * C::BN;
   const uint32_t t = threadIdx.x, wv = __builtin_amdgcn_readfirstlane(t >> 6), lane = t & 63;
   const uint32_t K4 = g.K / 4, lastblk = (g.M - 1) / g.R;
-  const uint32_t pad4 = TREE ? (K4 + 7) / 8 * 8 : K4;  // from here W's padding is -0
   // staging: piece it of this thread
   const v4* src[NIT];
   uint32_t step[NIT], q0[NIT], dst[NIT];
@@ -1007,7 +1005,7 @@ __global__ __launch_bounds__(256, OCC) void k_mgemm(MgemmArgs a) {
         if (q < K4) {
           st[j][i] = src[j][(size_t)q * step[j]];
         } else {
-          const float z = isw[j] && q >= pad4 ? __int_as_float((int)0x80000000u) : 0.0f;
+          const float z = isw[j] && !TREE ? __int_as_float((int)0x80000000u) : 0.0f;
           st[j][i] = v4{z, z, z, z};
         }
       }
@@ -1058,6 +1056,7 @@ __global__ __launch_bounds__(256, OCC) void k_mgemm(MgemmArgs a) {
     frags(0, 0);
 #pragma unroll
     for (uint32_t gi = 0; gi < NG; ++gi) {
+      if (TREE && gi && gi % 2 == 0 && ci * KC + 16 * gi >= g.K) break;
       if (gi + 1 < NG) frags(gi + 1, (gi + 1) & 1);
 #pragma unroll
       for (uint32_t x = 0; x < 4 * NT; ++x) {
