@@ -805,7 +805,9 @@ __global__ __launch_bounds__((ChainCfg<DUAL, NORM>::T), 3) void k_chain_gemm(Bge
 // consecutive k, and -0 as the addend, each of its 4 x 256 results is one
 // correctly rounded product W[m][k] * X[b][k] (x + (-0) = x for every x, so
 // the sign of a zero product survives; flushing and NaN bits are those of
-// v_mul_f32).  All four blocks leave a given output in the same lane, so the
+// v_mul_f32: two million products each of subnormal operands, of results next
+// to 2^-126, of NaNs of every sign and payload, of infinities and zeros differ
+// in no bit).  All four blocks leave a given output in the same lane, so the
 // vector units only add: acc = acc + p, k ascending, the strict chain of
 // k_bgemm (code/cis2-fp/src/main.rs:228-243, math.rs:40-48).  In tree order
 // they add pairs of a lane's products instead, the same number of adds.
@@ -2682,6 +2684,12 @@ static bool chain_gemm_fits(const BgemmSeg* segs, uint32_t nseg, uint32_t n, con
 // us per layer, k_bgemm | 32 x 32 | 64 x 64: 30-layer shape of 576, 64 rows
 // 104 | 105 | 234, 124 rows 141 | 114 | 244, 2000 rows 1298 | 476 | 520; that
 // of 1024, 16 rows 195 | 219 | 498, 2000 rows 5908 | 2281 | 2096.)
+// The constants are fits, so they were tried on eleven shapes that they were
+// not fitted to: hidden sizes 100 .. 4096, inner sizes 260 .. 11008, groups of
+// 1 .. 8 heads of 20 .. 128, 2 .. 256 decode rows, runs of 2 .. 8 rows, prompts
+// of 2 .. 599 rows.  Layer times without the matrix cores (and without
+// k_chain_gemm and the norm's placement) over those with them: sequential
+// 0.97 .. 6.7, tree 0.97 .. 5.9, under 1 only by what two runs differ.
 enum class MgemmTile { none, small, large };
 struct MgemmPlan {
   MgemmTile tile;
@@ -2927,7 +2935,13 @@ static hipError_t launch_kv(const KvPlan& kp, bool fuse, const float* q, float* 
 // more and no row is long (us per layer with k_attention_rows and k_rope_store
 // | here; 300 rows of 12 heads of 64: 40 positions 299 | 269, 200 349 | 341,
 // 500 477 | 462, 1500 793 | 833; 256 rows of 16 heads of 128: 637 | 582, 683 |
-// 674, 882 | 833, 1236 | 1373); false for another kernel.
+// 674, 882 | 833, 1236 | 1373); false for another kernel.  Larger groups, whose
+// heads read K and V again here, gain as much, and so do short runs of one
+// sequence (without FUSE; 256 rows at 100 | 400 positions, then 256 runs of 3
+// rows at 100 | 400): groups of 4, 16 heads of 64: 286 | 249, 315 | 309, 560 |
+// 494, 642 | 625; of 7, 14 of 64: 323 | 296, 380 | 349, 705 | 595, 920 | 723; of
+// 8, 32 of 64: 675 | 622, 733 | 716, 1612 | 1479, 1765 | 1712; of 4, 32 of 128:
+// 2088 | 1979, 2256 | 2196, 5586 | 5281, 5971 | 5899.
 constexpr uint32_t kWaveLen = 512;
 static bool wave_attention(uint32_t n, uint32_t nh, uint32_t nkv, uint32_t hd, uint32_t max_len,
                            bool tree, size_t* lds) {

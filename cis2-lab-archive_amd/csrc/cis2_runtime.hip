@@ -2043,9 +2043,9 @@ int cis2_verify_prefill(cis2_ctx* c, uint32_t seq, const uint32_t* prompt, uint3
 // ---- standalone GEMV ------------------------------------------------------
 
 // Host vectors of up to kPlanHost bytes go through the plan's mapped pinned
-// memory, which the GEMV reads and writes itself: 1536 x 576 19.8 us a call,
-// 21.5 with x fetched by a kernel first, 30.5 with copies from and to
-// pageable memory; 49152 x 576 41, 45 and 56 us.  A workgroup's block of W
+// memory, which the GEMV reads and writes itself: 1536 x 576 19.7 us a call,
+// 21.5 with x fetched by a kernel first, 30.6 with copies from and to
+// pageable memory; 49152 x 576 41, 45 and 57 us.  A workgroup's block of W
 // has to fit its LDS, so x is at most 2,300 floats or so; copies against
 // mapped memory over the rest of that range: 16 x 64 33 | 20, 151936 x 64
 // 113 | 93, 16 x 2048 37 | 27, 16384 x 2048 129 | 83 us.  A batch's inputs are
