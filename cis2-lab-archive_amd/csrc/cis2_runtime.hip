@@ -187,9 +187,10 @@ constexpr size_t kPlanHost = 1 << 20;
 struct cis2_gemv_plan {
   uint32_t M, K, copies;
   float *W = nullptr, *x = nullptr, *y = nullptr;
-  float *xb = nullptr, *yb = nullptr;  // [ncap][K], [ncap][M]: batched launches
-  uint32_t ncap = 0;
-  float *hx = nullptr, *hy = nullptr;  // mapped pinned host memory, hcap bytes each
+  float *xb = nullptr, *yb = nullptr;  // [xcap][K], [ycap][M]: batched launches
+  uint32_t xcap = 0, ycap = 0;
+  // mapped pinned host memory, one allocation: hcap bytes at hx, hcap at hy
+  float *hx = nullptr, *hy = nullptr;
   size_t hcap = 0, hmost = kPlanHost;  // hmost: the most that is asked for
   hipStream_t st = nullptr;
   hipEvent_t e0 = nullptr, e1 = nullptr;
@@ -2052,25 +2053,44 @@ int cis2_verify_prefill(cis2_ctx* c, uint32_t seq, const uint32_t* prompt, uint3
 // fetched first (60 of 200 x 2000: 88 against 120 us; 60 of 4096 x 64, copied
 // | mapped, 165 | 156).  Larger ones are copied, and all of them where no
 // pinned memory is to be had.
-// Pinned memory of `bytes` for each of the plan's vectors; false where it is
-// refused, and from then on for that size and above without asking again.
+// Pinned memory of `bytes` (and up to 255 more) for each of the plan's vectors;
+// false where it is refused, and from then on for that size and above without
+// asking again.
 static bool plan_host(cis2_gemv_plan* p, size_t bytes) {
   if (bytes <= p->hcap) return true;
   if (bytes > p->hmost) return false;
   if (p->hx) (void)hipHostFree(p->hx);
-  if (p->hy) (void)hipHostFree(p->hy);
   p->hx = p->hy = nullptr;
   p->hcap = 0;
-  if (hipHostMalloc(reinterpret_cast<void**>(&p->hx), bytes) != hipSuccess ||
-      hipHostMalloc(reinterpret_cast<void**>(&p->hy), bytes) != hipSuccess) {
+  const size_t cap = (bytes + 255) & ~(size_t)255;
+  if (hipHostMalloc(reinterpret_cast<void**>(&p->hx), 2 * cap) != hipSuccess) {
     (void)hipGetLastError();
-    if (p->hx) (void)hipHostFree(p->hx);
     p->hx = nullptr;
     p->hmost = bytes - 1;
     return false;
   }
-  p->hcap = bytes;
+  p->hy = p->hx + cap / sizeof(float);
+  p->hcap = cap;
   return true;
+}
+
+// A device buffer for n vectors of a batched launch (`bytes` in all).
+static hipError_t plan_grow(cis2_gemv_plan* p, float*& buf, uint32_t& cap, uint32_t n,
+                            size_t bytes) {
+  if (n <= cap) return hipSuccess;
+  hipError_t e = hipStreamSynchronize(p->st);
+  if (buf) (void)hipFree(buf);
+  buf = nullptr;
+  cap = 0;
+  if (e == hipSuccess) e = hipMalloc(&buf, bytes);
+  if (e == hipSuccess) cap = n;
+  return e;
+}
+static hipError_t plan_inputs(cis2_gemv_plan* p, uint32_t n) {
+  return plan_grow(p, p->xb, p->xcap, n, (size_t)n * p->K * sizeof(float));
+}
+static hipError_t plan_outputs(cis2_gemv_plan* p, uint32_t n) {
+  return plan_grow(p, p->yb, p->ycap, n, (size_t)n * p->M * sizeof(float) + 256);
 }
 
 int cis2_gemv_plan_create(uint32_t M, uint32_t K, uint32_t copies, const float* W,
@@ -2084,18 +2104,15 @@ int cis2_gemv_plan_create(uint32_t M, uint32_t K, uint32_t copies, const float* 
   hipError_t e = hipStreamCreateWithFlags(&p->st, hipStreamNonBlocking);
   if (e == hipSuccess) e = hipMalloc(&p->W, per * copies * sizeof(float));
   if (e == hipSuccess) e = hipMalloc(&p->x, (size_t)K * sizeof(float));
-  // defined inputs for the timing runs
-  if (e == hipSuccess) e = hipMemsetAsync(p->x, 0, (size_t)K * sizeof(float), p->st);
   if (e == hipSuccess) e = hipMalloc(&p->y, ((size_t)M + 64) * sizeof(float));
   if (e == hipSuccess) e = hipMalloc(&rowmajor, (size_t)M * K * sizeof(float));
   if (e == hipSuccess) e = hipMemcpy(rowmajor, W, (size_t)M * K * sizeof(float), hipMemcpyHostToDevice);
   for (uint32_t i = 0; e == hipSuccess && i < copies; ++i)
     e = launch_relayout(rowmajor, p->W + per * i, M, K, kPlanR, p->st);
-  if (e == hipSuccess) e = hipStreamSynchronize(p->st);
   if (e == hipSuccess) e = hipEventCreate(&p->e0);
   if (e == hipSuccess) e = hipEventCreate(&p->e1);
-  const size_t host = ((size_t)std::max(M, K)) * sizeof(float) + 256;
-  if (e == hipSuccess) (void)plan_host(p, host);
+  if (e == hipSuccess) (void)plan_host(p, (size_t)std::max(M, K) * sizeof(float) + 256);
+  if (e == hipSuccess) e = hipStreamSynchronize(p->st);
   if (rowmajor) (void)hipFree(rowmajor);
   if (e != hipSuccess) {
     cis2_gemv_plan_destroy(p);
@@ -2120,29 +2137,26 @@ static hipError_t plan_launch(cis2_gemv_plan* p, uint32_t c, const float* x, flo
 // x to the device, the lone GEMV (n = 0) or n GEMVs in one launch, y back.
 static hipError_t plan_through(cis2_gemv_plan* p, uint32_t n, const float* x, float* y) {
   const size_t nx = (size_t)(n ? n : 1) * p->K, ny = (size_t)(n ? n : 1) * p->M;
-  float *dx = n ? p->xb : p->x, *dy = n ? p->yb : p->y;
-  auto launch = [&](float* yd) {
-    return n ? launch_gemv_many(p->W, blocked_floats(p->M, p->K, kPlanR), p->copies, 0, n, dx, yd,
-                                p->M, p->K, kPlanR, p->st)
-             : plan_launch(p, 0, dx, yd);
-  };
-  const size_t most = std::max(nx, ny) * sizeof(float) + 256;
-  hipError_t e;
-  if (!plan_host(p, most)) {
+  const bool mapped = plan_host(p, std::max(nx, ny) * sizeof(float) + 256);
+  hipError_t e = n ? plan_inputs(p, n) : hipSuccess;
+  if (e == hipSuccess && n && !mapped) e = plan_outputs(p, n);
+  if (e != hipSuccess) return e;
+  float* dx = n ? p->xb : (mapped ? p->hx : p->x);
+  float* dy = mapped ? p->hy : (n ? p->yb : p->y);
+  if (!mapped) {
     e = hipMemcpyAsync(dx, x, nx * sizeof(float), hipMemcpyHostToDevice, p->st);
-    if (e == hipSuccess) e = launch(dy);
-    if (e == hipSuccess)
-      e = hipMemcpyAsync(y, dy, ny * sizeof(float), hipMemcpyDeviceToHost, p->st);
-    return e == hipSuccess ? hipStreamSynchronize(p->st) : e;
+  } else {
+    memcpy(p->hx, x, nx * sizeof(float));
+    if (n) e = launch_copy16(p->hx, dx, nx / 4, p->st);
   }
-  memcpy(p->hx, x, nx * sizeof(float));
-  if (n)
-    e = launch_copy16(p->hx, dx, nx / 4, p->st);
-  else
-    dx = p->hx, e = hipSuccess;
-  if (e == hipSuccess) e = launch(p->hy);
+  if (e == hipSuccess)
+    e = n ? launch_gemv_many(p->W, blocked_floats(p->M, p->K, kPlanR), p->copies, 0, n, dx, dy,
+                             p->M, p->K, kPlanR, p->st)
+          : plan_launch(p, 0, dx, dy);
+  if (e == hipSuccess && !mapped)
+    e = hipMemcpyAsync(y, dy, ny * sizeof(float), hipMemcpyDeviceToHost, p->st);
   if (e == hipSuccess) e = hipStreamSynchronize(p->st);
-  if (e == hipSuccess) memcpy(y, p->hy, ny * sizeof(float));
+  if (e == hipSuccess && mapped) memcpy(y, dy, ny * sizeof(float));
   return e;
 }
 
@@ -2153,7 +2167,8 @@ int cis2_gemv_plan_run(cis2_gemv_plan* p, const float* x, float* y) {
 
 int cis2_gemv_plan_time(cis2_gemv_plan* p, uint32_t iters, float* ms) {
   if (!p || !ms || iters == 0) return CIS2_E_ARG;
-  hipError_t e = hipSuccess;
+  // defined inputs: runs through mapped memory leave x alone
+  hipError_t e = hipMemsetAsync(p->x, 0, (size_t)p->K * sizeof(float), p->st);
   for (uint32_t i = 0; e == hipSuccess && i < p->copies; ++i)  // warm-up pass
     e = plan_launch(p, i, p->x, p->y);
   if (e == hipSuccess) e = hipEventRecord(p->e0, p->st);
@@ -2167,36 +2182,22 @@ int cis2_gemv_plan_time(cis2_gemv_plan* p, uint32_t iters, float* ms) {
   return CIS2_OK;
 }
 
-// Device buffers for n GEMVs' inputs and outputs.
-static hipError_t plan_reserve(cis2_gemv_plan* p, uint32_t n) {
-  if (n <= p->ncap) return hipSuccess;
-  hipError_t e = hipStreamSynchronize(p->st);
-  if (p->xb) (void)hipFree(p->xb);
-  if (p->yb) (void)hipFree(p->yb);
-  p->xb = p->yb = nullptr;
-  p->ncap = 0;
-  if (e == hipSuccess) e = hipMalloc(&p->xb, (size_t)n * p->K * sizeof(float));
-  if (e == hipSuccess) e = hipMalloc(&p->yb, (size_t)n * p->M * sizeof(float) + 256);
-  if (e == hipSuccess) {
-    p->ncap = n;
-    // defined inputs for the timing runs
-    e = hipMemsetAsync(p->xb, 0, (size_t)n * p->K * sizeof(float), p->st);
-  }
-  return e;
-}
-
 int cis2_gemv_plan_run_batch(cis2_gemv_plan* p, uint32_t n, const float* x, float* y) {
   if (!p || (n && (!x || !y)) || n > 65535) return CIS2_E_ARG;
   if (n == 0) return CIS2_OK;
-  hipError_t e = plan_reserve(p, n);
-  if (e == hipSuccess) e = plan_through(p, n, x, y);
+  const hipError_t e = plan_through(p, n, x, y);
   return e == hipSuccess ? CIS2_OK : (e == hipErrorOutOfMemory ? CIS2_E_OOM : CIS2_E_DEVICE);
 }
 
 int cis2_gemv_plan_time_batch(cis2_gemv_plan* p, uint32_t n, uint32_t iters, float* ms) {
   if (!p || !ms || iters == 0 || n == 0 || n > 65535) return CIS2_E_ARG;
   const uint64_t per = blocked_floats(p->M, p->K, kPlanR);
-  hipError_t e = plan_reserve(p, n);
+  const bool grows = n > p->xcap;
+  hipError_t e = plan_inputs(p, n);
+  if (e == hipSuccess) e = plan_outputs(p, n);
+  // defined inputs: those of a run, or zeros
+  if (e == hipSuccess && grows)
+    e = hipMemsetAsync(p->xb, 0, (size_t)n * p->K * sizeof(float), p->st);
   auto launch = [&](uint32_t it) {
     return launch_gemv_many(p->W, per, p->copies, (uint32_t)(((uint64_t)it * n) % p->copies), n,
                             p->xb, p->yb, p->M, p->K, kPlanR, p->st);
@@ -2222,7 +2223,6 @@ void cis2_gemv_plan_destroy(cis2_gemv_plan* p) {
   if (p->x) (void)hipFree(p->x);
   if (p->y) (void)hipFree(p->y);
   if (p->hx) (void)hipHostFree(p->hx);
-  if (p->hy) (void)hipHostFree(p->hy);
   if (p->e0) (void)hipEventDestroy(p->e0);
   if (p->e1) (void)hipEventDestroy(p->e1);
   if (p->st) (void)hipStreamDestroy(p->st);

@@ -14,10 +14,11 @@
 namespace {
 std::map<const void*, std::string> names;
 std::map<void*, size_t> live;
-int pinned_left = 1 << 30, undefined_inputs = 0, launches = 0;
+int pinned_left = 1 << 30, undefined_inputs = 0, launches = 0, allocations = 0;
 dim3 cfg_grid, cfg_block;
 
 hipError_t take(void** p, size_t n) {
+  ++allocations;
   *p = malloc(n);
   memset(*p, 0xFF, n);
   live[*p] = n;
@@ -51,6 +52,7 @@ extern "C" {
 void stub_allow_pinned(int n) { pinned_left = n; }
 int stub_undefined_inputs() { return undefined_inputs; }
 int stub_launches() { return launches; }
+int stub_allocations() { return allocations; }
 int stub_live() { return (int)live.size(); }
 
 void** __hipRegisterFatBinary(const void*) {

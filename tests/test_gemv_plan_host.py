@@ -1,6 +1,6 @@
 """The host side of the standalone GEMV plan over a HIP runtime of stubs
 (hip_stub.cpp), without a GPU: where its pinned memory is refused, the plan
-copies instead; its timing runs read defined memory."""
+copies instead; its timing runs read defined memory; what a run allocates."""
 import os
 import shutil
 import subprocess
@@ -72,8 +72,33 @@ p = GemvPlan(np.ones((M, K), np.float32), copies=2)
 p.time(3)
 check(M, x, p(x))
 p.time(3)
+p.time_batch(2, 3)
+check(M, X[:3], p.run_batch(X[:3]))
+p.time_batch(3, 3)
 p.time_batch(4, 3)
-assert stub.stub_launches() == 2 * (2 + 3) + 1 + 4 and stub.stub_undefined_inputs() == 0
+assert stub.stub_launches() == 2 * (2 + 3) + 1 + 4 + 1 + 4 + 4
+assert stub.stub_undefined_inputs() == 0
 p.close()
 assert stub.stub_live() == 0
 """ % rows)
+
+
+def test_allocations_of_a_plan(stub):
+    """A batched run allocates where it is larger than those before it: its
+    device inputs and, where the plan's first pinned block is too small, one
+    pinned block; every other run allocates nothing."""
+    run(stub, """
+p = GemvPlan(np.ones((M, K), np.float32))
+n0 = stub.stub_allocations()
+check(M, x, p(x))
+assert stub.stub_allocations() == n0
+check(M, X, p.run_batch(X))
+assert stub.stub_allocations() <= n0 + 2
+n1 = stub.stub_allocations()
+check(M, X[:2], p.run_batch(X[:2]))
+check(M, x, p(x))
+check(M, X, p.run_batch(X))
+assert stub.stub_allocations() == n1
+p.close()
+assert stub.stub_live() == 0
+""")
