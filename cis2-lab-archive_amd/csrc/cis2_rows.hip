@@ -2986,6 +2986,16 @@ hipError_t launch_rope_attention_rows(const float* q, const float* k, const floa
                    st);
 }
 
+// LDS of k_attention_rows with hpw heads per workgroup, and its limit.
+static size_t attention_rows_lds(uint32_t hpw, uint32_t hd, uint32_t max_len) {
+  const size_t hd4 = ((size_t)hd + 3) / 4 * 4, ls = ((size_t)max_len + 3) / 4 * 4;
+  return hpw * (hd4 + ls + (ls + 31) / 32) * sizeof(float);
+}
+constexpr size_t kAttRowsLds = 60 * 1024;
+bool attention_rows_fit(uint32_t hd, uint32_t max_len) {
+  return attention_rows_lds(1, hd, max_len) <= kAttRowsLds;
+}
+
 hipError_t launch_attention_rows(const float* q, const float* kc, const float* vc,
                                  RowsDesc rows, uint32_t max_len, uint32_t nh, uint32_t nkv,
                                  uint32_t hd, uint32_t max_pos, uint64_t seq_stride, float scale,
@@ -2994,11 +3004,9 @@ hipError_t launch_attention_rows(const float* q, const float* kc, const float* v
   if (nkv == 0 || nh % nkv || max_len == 0 || max_len > max_pos || max_pos % 4)
     return hipErrorInvalidValue;
   const uint32_t group = nh / nkv;
-  const size_t hd4 = ((size_t)hd + 3) / 4 * 4, ls = ((size_t)max_len + 3) / 4 * 4;
-  auto lds_of = [&](uint32_t hpw) { return hpw * (hd4 + ls + (ls + 31) / 32) * sizeof(float); };
   const int ncu = device_cu_count();
   const uint64_t wgs_kv = (uint64_t)rows.n * nkv;
-  const uint32_t tr = tree ? 1u : 0u, ls32 = (uint32_t)ls;
+  const uint32_t tr = tree ? 1u : 0u, ls = (max_len + 3) / 4 * 4;
   {
     KvPlan kp;
     hipError_t e = kv_plan(rows.n, nh, nkv, hd, max_len, &kp);
@@ -3016,30 +3024,30 @@ hipError_t launch_attention_rows(const float* q, const float* kc, const float* v
   uint32_t hpw = 1;
   if (wgs_kv >= 4 * (uint64_t)ncu) {
     for (uint32_t h = std::min(group, kMaxHeadsPerWg); h > 1; --h)
-      if (group % h == 0 && lds_of(h) <= 60 * 1024) {
+      if (group % h == 0 && attention_rows_lds(h, hd, max_len) <= kAttRowsLds) {
         hpw = h;
         break;
       }
   }
-  const size_t shmem = lds_of(hpw);
-  if (shmem > 60 * 1024) return hipErrorInvalidValue;
+  const size_t shmem = attention_rows_lds(hpw, hd, max_len);
+  if (shmem > kAttRowsLds) return hipErrorInvalidValue;
   const dim3 grid(rows.n, nh / hpw);
   switch (hpw) {
     case 4:
       hipLaunchKernelGGL(k_attention_rows<4>, grid, dim3(kAttT), shmem, st, q, kc, vc, rows, nh,
-                         nkv, hd, max_pos, seq_stride, scale, out, tr, ls32);
+                         nkv, hd, max_pos, seq_stride, scale, out, tr, ls);
       break;
     case 3:
       hipLaunchKernelGGL(k_attention_rows<3>, grid, dim3(kAttT), shmem, st, q, kc, vc, rows, nh,
-                         nkv, hd, max_pos, seq_stride, scale, out, tr, ls32);
+                         nkv, hd, max_pos, seq_stride, scale, out, tr, ls);
       break;
     case 2:
       hipLaunchKernelGGL(k_attention_rows<2>, grid, dim3(kAttT), shmem, st, q, kc, vc, rows, nh,
-                         nkv, hd, max_pos, seq_stride, scale, out, tr, ls32);
+                         nkv, hd, max_pos, seq_stride, scale, out, tr, ls);
       break;
     default:
       hipLaunchKernelGGL(k_attention_rows<1>, grid, dim3(kAttT), shmem, st, q, kc, vc, rows, nh,
-                         nkv, hd, max_pos, seq_stride, scale, out, tr, ls32);
+                         nkv, hd, max_pos, seq_stride, scale, out, tr, ls);
   }
   return hipGetLastError();
 }

@@ -87,6 +87,9 @@ hipError_t launch_rope_attention_rows(const float* q, const float* k, const floa
                                       uint32_t nh, uint32_t nkv, uint32_t hd, uint32_t max_pos,
                                       float* kc, float* vc, uint64_t seq_stride, float scale,
                                       float* out, bool tree, hipStream_t st);
+// Whether launch_attention_rows takes any number of rows of up to max_len
+// positions (their scores fit a workgroup's LDS).
+bool attention_rows_fit(uint32_t hd, uint32_t max_len);
 // Prefill attention in tiles: rows row0 .. row0+nr-1 (nr <= 16) are rows of
 // sequence seq at positions p0 .. p0+nr-1; each tile's rows get the same
 // bits as launch_attention_rows gives them, with each K and V element read

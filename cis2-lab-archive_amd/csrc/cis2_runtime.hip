@@ -650,7 +650,8 @@ int forward_rows(cis2_ctx* c, uint32_t n, const uint32_t* d_tok, uint32_t max_le
 // Uploads row descriptors (and the logit-row list) and runs forward_rows.
 // Rows that attend in tiles: the prefill of many rows (runs of one sequence
 // at consecutive positions, up to kAttTileRows per tile) for the shapes the
-// tiled kernel has; *ntiles = 0 otherwise.
+// tiled kernel has; *ntiles = 0 otherwise, and where the tiles' scratch is
+// refused.
 // CIS2_ATT_TILES=1 / 0 forces the tiles on / off (the bits are the same).
 int plan_tiles(cis2_ctx* c, uint32_t n, const uint32_t* seq, const uint32_t* pos,
                uint32_t max_len, uint32_t* ntiles) {
@@ -689,15 +690,19 @@ int plan_tiles(cis2_ctx* c, uint32_t n, const uint32_t* seq, const uint32_t* pos
     b.tmem.clear();
     b.tcap = 0;
     b.acap = 0;
-    void* p = nullptr;
-    if (hipMalloc(&p, (size_t)nt * sizeof(AttTile)) != hipSuccess)
-      return fail(c, CIS2_E_OOM, "attention tiles");
-    b.tmem.push_back(p);
-    b.tiles = static_cast<AttTile*>(p);
-    if (hipMalloc(&p, scr * sizeof(float)) != hipSuccess)
-      return fail(c, CIS2_E_OOM, "attention tile scratch");
-    b.tmem.push_back(p);
-    b.ascr = static_cast<float*>(p);
+    void *pt = nullptr, *ps = nullptr;
+    if (hipMalloc(&pt, (size_t)nt * sizeof(AttTile)) != hipSuccess ||
+        hipMalloc(&ps, scr * sizeof(float)) != hipSuccess) {
+      (void)hipGetLastError();
+      if (pt) (void)hipFree(pt);
+      // the per-row kernels need no memory
+      return attention_rows_fit(f.head_dim, max_len)
+                 ? CIS2_OK
+                 : fail(c, CIS2_E_OOM, "attention tile scratch");
+    }
+    b.tmem = {pt, ps};
+    b.tiles = static_cast<AttTile*>(pt);
+    b.ascr = static_cast<float*>(ps);
     b.tcap = nt;
     b.acap = scr;
   }

@@ -40,10 +40,14 @@ def stub(tmp_path_factory):
     return str(so)
 
 
-def run(stub, body):
-    r = subprocess.run([sys.executable, "-c", SETUP + body, stub], capture_output=True, text=True,
+def run_stubbed(stub, setup, body):
+    r = subprocess.run([sys.executable, "-c", setup + body, stub], capture_output=True, text=True,
                        timeout=120)
     assert r.returncode == 0, r.stderr[-2000:]
+
+
+def run(stub, body):
+    run_stubbed(stub, SETUP, body)
 
 
 @pytest.mark.parametrize("pinned", [0, 1, 2, 100])
