@@ -129,7 +129,8 @@ struct cis2_ctx {
   uint32_t* ring_tok = nullptr;
   // cis2_forward of one row through the persistent kernel (mapped pinned
   // host memory the kernel reads and writes itself): logits [vocab], then
-  // the token, the argmax and the error word
+  // the token, the argmax and the error word.  Null where it was refused:
+  // such calls take the per-op path
   float* fwd_logits = nullptr;
   uint32_t* fwd_words = nullptr;
   hipEvent_t ring_ev[kRing];
@@ -1028,13 +1029,17 @@ int cis2_ctx_create(const cis2_config* cfg, cis2_ctx** out) {
   if (hipHostMalloc(reinterpret_cast<void**>(&c->ring), (size_t)kRing * V * sizeof(float)) !=
           hipSuccess ||
       hipHostMalloc(reinterpret_cast<void**>(&c->ring_tok), kRing * 2 * sizeof(uint32_t)) !=
-          hipSuccess ||
-      hipHostMalloc(reinterpret_cast<void**>(&c->fwd_logits), ((size_t)V + 4) * sizeof(float)) !=
           hipSuccess) {
     cis2_ctx_destroy(c);
     return CIS2_E_OOM;
   }
-  c->fwd_words = reinterpret_cast<uint32_t*>(c->fwd_logits + V);
+  if (hipHostMalloc(reinterpret_cast<void**>(&c->fwd_logits), ((size_t)V + 4) * sizeof(float)) ==
+      hipSuccess) {
+    c->fwd_words = reinterpret_cast<uint32_t*>(c->fwd_logits + V);
+  } else {
+    (void)hipGetLastError();
+    c->fwd_logits = nullptr;
+  }
   for (int i = 0; i < kRing; ++i)
     if (hipEventCreateWithFlags(&c->ring_ev[i], hipEventDisableTiming) != hipSuccess ||
         hipEventCreateWithFlags(&c->ring_ready[i], hipEventDisableTiming) != hipSuccess) {
@@ -1340,7 +1345,7 @@ int cis2_forward(cis2_ctx* c, uint32_t n, const uint32_t* seq, const uint32_t* p
     if (seq[i] >= c->cfg.max_seqs) return fail(c, CIS2_E_ARG, "sequence index out of range");
     if (pos[i] >= c->cfg.max_pos) return fail(c, CIS2_E_RANGE, "position beyond max_pos");
     if (tok[i] >= c->cfg.vocab) return fail(c, CIS2_E_RANGE, "token id >= vocab");
-    if (use_fast(c)) {
+    if (use_fast(c) && c->fwd_logits) {
       // token, logits, argmax and error word go through mapped host memory:
       // one launch, one word's launch and one wait, where the copies and
       // their waits took 130 us more than the kernel's 740 (196 KB of logits)

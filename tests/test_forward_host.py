@@ -6,9 +6,10 @@ import pytest
 from test_gemv_plan_host import PKG, run_stubbed, stub  # noqa: F401
 
 SETUP = """
-import ctypes, sys
+import ctypes, os, sys
 import numpy as np
 sys.path.insert(0, %r)
+os.environ["CIS2_DECODE_LOCK"] = "0"
 stub = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
 stub.stub_device_most.argtypes = [ctypes.c_size_t]
 from cis2amd import Cis2Error, Cis2Model, artifacts
@@ -54,3 +55,19 @@ except Cis2Error as e:
 m.close()
 assert stub.stub_live() == 0
 """)
+
+
+@pytest.mark.parametrize("pinned,kernel", [(2, "k_embed"), (3, "k_decode")],
+                         ids=["refused", "granted"])
+def test_context_without_pinned_memory_for_single_rows(stub, pinned, kernel):  # noqa: F811
+    """`pinned` allocations of pinned memory succeed, two of them the decode
+    ring's: a context is made either way, and a single row goes through the
+    persistent kernel where its logits have mapped memory."""
+    run_stubbed(stub, SETUP, """
+stub.stub_allow_pinned(%d)
+m = Cis2Model(spec, w, max_pos=64)
+m.forward_token(0, 5)
+assert count("k_embed") + count("k_decode") == count(%r) == 1
+m.close()
+assert stub.stub_live() == 0
+""" % (pinned, kernel))
