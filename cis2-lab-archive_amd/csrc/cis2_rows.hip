@@ -214,6 +214,7 @@ __global__ __launch_bounds__(256) void k_bgemm(BgemmArgs a) {
               x = xp[q + j];
               if (DUAL) w2 = wp2[(size_t)(q + j) * R];
             }
+            asm("" : "+v"(x) : "v"(w), "v"(w2));  // W the left operand (see ChainSums)
             l[4 * j] = w.x * x.x;
             l[4 * j + 1] = w.y * x.y;
             l[4 * j + 2] = w.z * x.z;
@@ -840,7 +841,10 @@ constexpr __host__ __device__ uint32_t mtile_k(uint32_t x) { return TREE ? x % 4
 // The adds of NT tiles.  add(): products4's p, for k = 4q .. 4q + 3 of every
 // 32, into tile s: k ascending, or in tree order (math.rs:60-125) the pairs'
 // sums of the 32, whose total acc takes (zeros before the first step: acc is
-// +0 and stays so).
+// +0 and stays so).  In tree order the earlier sum is the left operand of
+// every add, and W of every product in k_bgemm too, as in the persistent
+// kernel: of two NaNs the left one is kept.  (The compiler would swap the last
+// add; the empty asm makes its right operand the later value.)
 template <uint32_t NT, bool TREE>
 struct ChainSums {
   float t4[4] = {}, t8[4] = {}, t16[TREE ? NT : 1][4] = {};
@@ -864,7 +868,8 @@ struct ChainSums {
           t16[s][r] = v16k;
           continue;
         }
-        const float v32k = t16[s][r] + v16k;
+        float v32k = t16[s][r] + v16k;
+        asm("" : "+v"(v32k) : "v"(acc[s][r]));  // acc stays the left operand
         acc[s][r] = acc[s][r] + v32k;
       }
       float* o = q == 7 ? acc[s] : (q == 3 ? t16[s] : (q % 2 ? t8 : t4));

@@ -363,3 +363,39 @@ def test_qk_norm_of_head_dims_that_are_no_multiple_of_four(hd, tree):
     for at, k in ((0, 1), (1, 3), (4, 1)):
         lg, _ = m.forward_rows(np.zeros(k), np.arange(at, at + k), tok[at:at + k])
         assert np.array_equal(want[at:at + k], lg.view(np.uint32)), at
+
+
+@pytest.mark.parametrize("tree", [True, False], ids=["tree", "seq"])
+@pytest.mark.parametrize("k,n", [(68, 40), (300, 17)])
+def test_several_nans_keep_their_places(k, n, tree):
+    """Where different NaNs and infinities meet in the sums, every path has
+    the same NaN logits and the same bits in all others; in tree order the row
+    GEMMs have the bits of the persistent kernel in the NaNs too (the left
+    operand's)."""
+    spec = artifacts.ModelSpec("nans%d" % k, k, 188, 2, 4, 2, 5003, 1e-5, 10000.0, False,
+                               head_dim=64)
+    w = artifacts.Weights(spec, 16)
+    rng = np.random.default_rng(16)
+    for name, _, arr in w.tensors:
+        a, some = arr.reshape(-1), arr.size // 5000
+        if "lm_head" in name:
+            sign = rng.integers(0, 2, 2 * some) << 15
+            a[rng.integers(0, a.size, some)] = 0x7F80 | sign[:some]
+            a[rng.integers(0, a.size, some)] = 0x7FA1 + rng.integers(0, 30, some) | sign[some:]
+            a[::7 * k] = 0xFFB1  # against the NaN activations of the first block
+        elif "embed" in name:
+            a[-k:][[0, 7, 8]] = [0x7FA1, 0xFFC2, 0xFF80]  # the last token's
+    tok = rng.integers(0, spec.vocab - 1, n).astype(np.uint32)
+    tok[n // 2] = spec.vocab - 1
+    m = Cis2Model(spec, w, max_pos=n, max_seqs=1, reduction_mode=1 if tree else 0)
+    rows, _ = run(m, n, n, tok, "1")
+    vec, _ = run(m, n, n, tok, "0")
+    m.reset(0)
+    one = np.stack([m.forward_token(p, int(tok[p]))[0] for p in range(n)])
+    nan = np.isnan(one)
+    assert nan[n // 2].all() and nan[0].any() and not nan[:n // 2].all(axis=1).any()
+    for got in (rows, vec):
+        assert np.array_equal(np.isnan(got.view(np.float32)), nan)
+        assert np.array_equal(got[~nan], one.view(np.uint32)[~nan])
+        if tree:
+            assert np.array_equal(got, one.view(np.uint32))
